@@ -170,9 +170,9 @@ int emma_assign_noalloc(const float *X, int64_t n, int32_t d, const float *C, in
 
 /*
  * Variants of the MFMA assignment, for the autotuner: the pipeline of its
- * first pass (a coarse fp16 pass over every frame whose undecided frames go
- * to the fine bf16 x 3 pass, or the fine pass over every frame) and the tile
- * shape (waves per workgroup, workgroups per CU, frame blocks per wave).
+ * first pass (0, the default: a coarse fp16 pass over every frame whose
+ * undecided frames go to the fine bf16 x 3 pass; 1: the fine pass over every
+ * frame).
  * emma_assign_variants(d) is the
  * number of variants at dimension d (0 if d is beyond the MFMA path);
  * emma_assign_select(d, k, v) makes variant v the one used for every later

@@ -1,9 +1,9 @@
-"""Tile-shape autotuner of the assignment kernel.
+"""Autotuner of the assignment's first pass.
 
-The MFMA assignment kernel exists in a few tile variants (waves per
-workgroup x workgroups per CU, emma_assign_variants).  Which one is fastest
-depends on the dimension (register footprint of the frame fragments, size of
-a center tile) and on the number of centers (tiles per frame block).  The
+The MFMA assignment exists in a few variants (emma_assign_variants): a coarse
+fp16 pass with the fine pass on the frames it leaves, or the fine pass over
+every frame.  Which one is faster depends on the dimension, the number of
+centers and the data (how many frames the coarse bound leaves).  The
 first call for a (dimension, center count) bucket times every variant on a
 sample of the caller's own frames (up to 2^21 frames: smaller samples fill
 the device for only a few rounds, where the variants tie and the full-size
@@ -41,7 +41,7 @@ def tuned():
 
 
 def tune_assign(Xt, Ct, mode=_native.EMMA_ASSIGN_BF16X3_RECHECK, sample=2097152, reps=2):
-    """Select the fastest assignment tile variant for these sizes (once per bucket)."""
+    """Select the fastest assignment variant for these sizes (once per bucket)."""
     if mode != _native.EMMA_ASSIGN_BF16X3_RECHECK:
         return None
     t = _native.torch()

@@ -9,17 +9,16 @@
 //
 //  * k_assign_plain: the sequential FP32 loop itself on the vector ALUs
 //    (4 frames x 4 centers per thread, LDS-staged tiles).
-//  * k_assign_mfma, then k_assign_plain on a list: distances from bf16 hi/lo MFMA products on
-//    shifted data, d~_j = |a|^2 + |b_j|^2 - 2 a.b_j with a = fl(x - mu),
-//    b_j = fl(c_j - mu).  With E_j = CE (|a| + |b_j|)^2 a rigorous bound on
-//    |d~_j - d_j| (CE from u = 2^-24, the bf16 split residual 2^-16 and the
-//    FP32 accumulation of 3 d products, see assign_error_coeff) and
-//    g = gamma_{d+2} the relative rounding of the reference loop, a frame is
-//    decided when
+//  * k_assign_tile in up to three passes, then exact loops on what they leave:
+//    distances d~_j = |a|^2 + |b_j|^2 - 2 a.b_j on shifted data a = fl(x - mu),
+//    b_j = fl(c_j - mu), from fp16 products (coarse pass, every frame) and from
+//    bf16 hi/lo products (fine pass, the frames the coarse pass leaves).  With
+//    E_j a rigorous bound on |d~_j - d_j| (see AsgCoef) and g = gamma_{d+2} the
+//    relative rounding of the reference loop, a frame is decided when
 //        (1 - g) min_{j != best} (d~_j - E_j)  >  (1 + g)(d~_best + E_best);
-//    then no other center can reach the reference loop's minimum.  All other
-//    frames are appended to a list and re-evaluated by k_assign_plain with the
-//    sequential FP32 loop over every center.
+//    then no other center can reach the reference loop's minimum.  The other
+//    frames are appended to a list and re-evaluated with the sequential FP32
+//    loop, over recorded candidates or over every center (k_assign_plain).
 #include <math.h>
 
 #include <mutex>
@@ -50,8 +49,12 @@ __global__ __launch_bounds__(256) void k_assign_plain(const float *__restrict__ 
                                                       int32_t *__restrict__ labels,
                                                       const int64_t *__restrict__ list,
                                                       const int64_t *__restrict__ list_count,
+                                                      int64_t *__restrict__ n_rechecked,
+                                                      const int64_t *__restrict__ n_listed,
                                                       const int32_t *__restrict__ done) {
     if (done && *done) return;
+    // the call's count of re-evaluated frames (0 for the loop over every frame)
+    if (n_rechecked && blockIdx.x == 0 && threadIdx.x == 0) *n_rechecked = n_listed ? *n_listed : 0;
     __shared__ __align__(16) float xs[PD][PPITCH];
     __shared__ __align__(16) float cs[PD][PPITCH];
     __shared__ float s_best[16][PF];
@@ -159,152 +162,188 @@ __global__ __launch_bounds__(256) void k_assign_plain(const float *__restrict__ 
     }
 }
 
-__global__ void k_copy_i64(int64_t *dst, const int64_t *src) { *dst = *src; }
+constexpr int N_COUNTS = 8;  // counters and maxima at the head of the workspace, cleared by every call
+
 __global__ void k_add_i64(int64_t *dst, const int64_t *src) { *dst += *src; }
 
 // ------------------------------------------------------------------
 // center preparation for the MFMA path
 // ------------------------------------------------------------------
-// Centers are packed once per call into "tile images": for every tile of 32
-// centers one contiguous block that is byte-for-byte the LDS layout the MFMA
-// kernel reads,
-//   uint16 hi[32][pitch], lo[32][pitch]   bf16 bits of b = fl(c - mu), rows
-//                                          padded from d_pad to pitch = d_pad + 8
-//   float  nb[32], q[32], r[32]           |b|^2 (FP32 sequential), nb - CE bn^2, 2 CE bn
-// so that a tile moves from L2 to LDS with asynchronous 16-byte copies.
+// Centers are packed once per call into "tile images", one contiguous block
+// per tile of 32 centers.  An image holds the MFMA operand fragments in the
+// order the lanes read them: for K-step s (16 dims) and plane p, 64 lanes x 16
+// bytes, lane l the 8 dims 16 s + 8 (l / 32) .. of center l % 32, so that a
+// wave loads a fragment with one contiguous 1 KB read from L2.
+//   bf16 image: planes hi, lo of -2 b, b = fl(c - mu), d_pad / 16 K-steps; then
+//               the constants of the 32 centers (FC_*)
+//   fp16 image: one plane of -2 2^t b; then the constants HC_*
+// (the factor -2 and the constant |b|^2 make d~ - |a|^2 = |b|^2 - 2 a.b the
+// matrix core's own result when the accumulator starts from |b|^2).
 struct CenterPack {
-    uint8_t *img;    // k_pad / 32 tile images of img_bytes each
-    uint8_t *img16;  // k_pad / 32 fp16 tile images of img16_bytes each (the coarse pass)
-    float *bn;       // [k_pad] |b| rounded up
+    uint8_t *img;    // k_pad / 32 bf16 tile images of tile_img_bytes each
+    uint8_t *img16;  // k_pad / 32 fp16 tile images of tile_img16_bytes each (the coarse pass)
     float *mu;       // [d_pad] shift
-    float *bmax;     // max_j |b_j| (zeroed before the packing, then an atomic max)
-    float *sc16;     // [4] coarse pass: 2^t, -2^(1 - 2t), the coefficient c3 of its absolute error term
+    float *mx;       // [8] maxima over the centers (MX_*), zeroed before the packing, then atomic maxima
+    float *sc16;     // [4] coarse pass: 2^t, 2^-2t, 2^-t
 };
+// constants of a bf16 image, 32 floats each: |b|^2, |b|^2 - c1b |b|^2 (the
+// lower-bound start of the candidate pass), |b|, |lo part|, |what hi + lo leave|
+constexpr int FC_NB = 0, FC_Q = 32, FC_BN = 64, FC_D1 = 96, FC_D2 = 128;
+// constants of an fp16 image: 2^2t |b|^2, |b|, |what fp16 leaves of b|
+constexpr int HC_NB = 0, HC_BN = 32, HC_D1 = 64;
+constexpr int MX_BN = 0, MX_D1 = 1, MX_D2 = 2, MX_D16 = 3;
 
-__host__ __device__ constexpr int tile_pitch(int d_pad) { return d_pad + 8; }
-__host__ __device__ constexpr int tile_img_bytes(int d_pad) { return 128 * tile_pitch(d_pad) + 3 * 32 * 4; }
-// fp16 image of the coarse pass: uint16 h[32][pitch] (fp16 bits of 2^t b),
-// then the same constants nb, q, r
-__host__ __device__ constexpr int tile_img16_bytes(int d_pad) { return 64 * tile_pitch(d_pad) + 3 * 32 * 4; }
+__host__ __device__ constexpr int tile_img_bytes(int d_pad) { return 128 * (d_pad + 8) + 3 * 32 * 4; }
+__host__ __device__ constexpr int tile_img16_bytes(int d_pad) { return 64 * (d_pad + 8) + 3 * 32 * 4; }
+static_assert(128 * 8 + 3 * 32 * 4 >= 5 * 32 * 4 && 64 * 8 + 3 * 32 * 4 >= 3 * 32 * 4, "constants fit behind the fragments");
 
-// mu = mean of the centers (FP64 in a fixed order, rounded to FP32):
-// 64 dims per workgroup, wave w sums centers w, w + 4, ...
-__global__ __launch_bounds__(256) void k_center_mean(const float *__restrict__ C, int k, int d, int d_pad,
-                                                     float *__restrict__ mu) {
-    __shared__ double s_part[4][64];
+// mu = FP64 mean (in a fixed order, rounded to FP32) of at most MU_SAMPLE
+// centers spread over the set.  Any shift gives the same labels; one near the
+// middle of the centers keeps |a| and |b|, and with them the error bound,
+// small, and the mean of 128 centers is within a tenth of their spread of the
+// mean of all.  64 dims per workgroup, wave w sums samples w, w + 16, ...: 8
+// loads per lane, in flight together (one wave walking all of k = 1000 .. 4096
+// centers took 92 .. 391 us, this 5).  The first workgroup clears the call's
+// counters and maxima.
+constexpr int MU_SAMPLE = 128, MU_WAVES = 16;
+__global__ __launch_bounds__(64 * MU_WAVES) void k_center_mean(const float *__restrict__ C, int k, int d, int d_pad,
+                                                               float *__restrict__ mu, int64_t *__restrict__ counts) {
+    __shared__ double s_part[MU_WAVES][64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (blockIdx.x == 0 && threadIdx.x < N_COUNTS) counts[threadIdx.x] = 0;
     const int i = blockIdx.x * 64 + lane;
+    const int ns = k < MU_SAMPLE ? k : MU_SAMPLE;
+    float v[MU_SAMPLE / MU_WAVES];
+#pragma unroll
+    for (int u = 0; u < MU_SAMPLE / MU_WAVES; ++u) {
+        const int q = u * MU_WAVES + wave;
+        v[u] = (i < d && q < ns) ? C[((int64_t)q * k / ns) * d + i] : 0.0f;
+    }
     double acc = 0.0;
-    if (i < d)
-        for (int j = wave; j < k; j += 4) acc += (double)C[(int64_t)j * d + i];
+#pragma unroll
+    for (int u = 0; u < MU_SAMPLE / MU_WAVES; ++u) acc += (double)v[u];
     s_part[wave][lane] = acc;
     __syncthreads();
-    if (wave == 0 && i < d_pad)
-        mu[i] = i < d ? (float)(((s_part[0][lane] + s_part[1][lane]) + (s_part[2][lane] + s_part[3][lane])) / k) : 0.0f;
+    if (wave == 0 && i < d_pad) {
+        double t = 0.0;
+#pragma unroll
+        for (int w = 0; w < MU_WAVES; ++w) t += s_part[w][lane];
+        mu[i] = i < d ? (float)(t / ns) : 0.0f;
+    }
 }
 
-// one wavefront per (padded) center
+// upper bound of sqrt(v) as a float (v a nonnegative FP64 sum)
+__device__ __forceinline__ float norm_up(double v) { return (float)(sqrt(v) * (1.0 + 1e-6)); }
+__device__ __forceinline__ void atomic_max_pos(float *p, float v) {  // v >= 0 or NaN (which then stays)
+    atomicMax(reinterpret_cast<unsigned int *>(p), __float_as_uint(v) & 0x7fffffffu);
+}
+
+// bf16 tile images; one wavefront per (padded) center, lane l owns dims 8 l .. 8 l + 7
 __global__ __launch_bounds__(256) void k_center_pack(const float *__restrict__ C, int k, int d, int d_pad,
-                                                     int k_pad, float2 CE, CenterPack cp) {
+                                                     int k_pad, float c1b, CenterPack cp) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int j = blockIdx.x * 4 + wave;
     if (j >= k_pad) return;
-    const int pitch = tile_pitch(d_pad);
     uint8_t *img = cp.img + (int64_t)(j >> 5) * tile_img_bytes(d_pad);
-    uint16_t *hi = reinterpret_cast<uint16_t *>(img) + (j & 31) * pitch;
-    uint16_t *lo = hi + 32 * pitch;
-    float *cst = reinterpret_cast<float *>(img + 128 * pitch);
-    double n2 = 0.0;
-    for (int i = lane; i < pitch; i += 64) {
-        float b = 0.0f;
-        if (j < k && i < d) b = __fsub_rn(C[(int64_t)j * d + i], cp.mu[i]);
-        uint32_t h, l;
-        split_bf16(b, h, l);
-        hi[i] = (uint16_t)h;  // the pad columns d_pad .. pitch - 1 hold zeros
-        lo[i] = (uint16_t)l;
-        n2 += (double)b * (double)b;
-    }
-    // FP32 |b|^2 in index order (one lane walks the row; the error bound only
-    // needs gamma_d, any order would do, this keeps it deterministic)
-    double n2s = wave_butterfly_sum(n2);
-    if (lane == 0) {
-        float nb, q, r, bn;
-        if (j < k) {
-            float acc = 0.0f;
-            for (int i = 0; i < d; ++i) {
-                const float b = __fsub_rn(C[(int64_t)j * d + i], cp.mu[i]);
-                acc = __fadd_rn(acc, __fmul_rn(b, b));
-            }
-            bn = (float)(sqrt(n2s) * (1.0 + 1e-6));  // rounded up
-            nb = acc;
-            q = acc - CE.x * bn * bn;
-            r = 2.0f * CE.y * bn;
-        } else {
-            // padding: a finite value beyond every real d~ (the epilogue's
-            // index bits must not turn it into a NaN); never a candidate
-            nb = 3.0e38f;
-            bn = 0.0f;
-            q = 3.0e38f;
-            r = 0.0f;
+    double n2 = 0.0, e1 = 0.0, e2 = 0.0;
+    if (lane * 8 < d_pad) {
+        float b[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int i = lane * 8 + q;
+            b[q] = (j < k && i < d) ? __fsub_rn(C[(int64_t)j * d + i], cp.mu[i]) : 0.0f;
         }
-        cp.bn[j] = bn;
-        if (j < k) atomicMax(reinterpret_cast<unsigned int *>(cp.bmax), __float_as_uint(bn));  // bn >= 0
-        cst[j & 31] = nb;
-        cst[32 + (j & 31)] = q;
-        cst[64 + (j & 31)] = r;
+        uint32_t h[8], l[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            split_bf16(-2.0f * b[q], h[q], l[q]);
+            const float lf = bf16_bits_to_f32(l[q]);
+            const float r = (-2.0f * b[q] - bf16_bits_to_f32(h[q])) - lf;
+            n2 += (double)b[q] * (double)b[q];
+            e1 += (double)lf * (double)lf;
+            e2 += (double)r * (double)r;
+        }
+        const int slot = (j & 31) + 32 * (lane & 1);
+        uint8_t *dst = img + (lane >> 1) * 2048 + slot * 16;
+        *reinterpret_cast<uint4 *>(dst) = make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7]));
+        *reinterpret_cast<uint4 *>(dst + 1024) = make_uint4(pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7]));
+    }
+    n2 = wave_butterfly_sum(n2);
+    e1 = wave_butterfly_sum(e1);
+    e2 = wave_butterfly_sum(e2);
+    if (lane == 0) {
+        float *cst = reinterpret_cast<float *>(img + 128 * d_pad) + (j & 31);
+        // padding: a finite value beyond every real d~ (the epilogue's index
+        // bits must not turn it into a NaN); never a candidate
+        const bool in = j < k;
+        const float nb = in ? (float)n2 : 3.0e38f, bn = in ? norm_up(n2) : 0.0f;
+        const float d1 = in ? norm_up(0.25 * e1) : 0.0f, d2 = in ? norm_up(0.25 * e2) : 0.0f;
+        cst[FC_NB] = nb;
+        cst[FC_Q] = in ? nb - c1b * bn * bn : 3.0e38f;
+        cst[FC_BN] = bn;
+        cst[FC_D1] = d1;
+        cst[FC_D2] = d2;
+        if (in) {
+            atomic_max_pos(cp.mx + MX_BN, bn);
+            atomic_max_pos(cp.mx + MX_D1, d1);
+            atomic_max_pos(cp.mx + MX_D2, d2);
+        }
     }
 }
 
-// Scale of the coarse pass: 2^t with t = 9 - e, bmax = m 2^e (m in [1/2, 1)),
-// clamped to |t| <= 60, so that every |2^t b_ji| < 2^10 (fp16 holds up to
-// 65504: frames with |a_i| < 64 max|b| stay finite; larger ones overflow to
-// inf and go to the fine pass).  c3 bounds the effect of fp16 underflow
-// (absolute error <= 2^-25 of a scaled component) on d~:
-// 2 * 1.01 * 2^-25 2^-t sqrt(d) (|a| + |b_j|), with a 25 % margin.
-__global__ void k_center_scale16(int d, CenterPack cp) {
-    const float bm = *cp.bmax;
-    int e = 0;
-    frexpf(bm, &e);
-    int t = bm > 0.0f && bm == bm && bm < INFINITY ? 9 - e : 0;
-    t = t > 60 ? 60 : (t < -60 ? -60 : t);
-    cp.sc16[0] = ldexpf(1.0f, t);
-    cp.sc16[1] = -ldexpf(1.0f, 1 - 2 * t);
-    cp.sc16[2] = (float)(1.25 * 2.0 * 1.01 * ldexp(1.0, -25 - t) * sqrt((double)d));
-    cp.sc16[3] = 0.0f;
-}
-
-// fp16 tile images of 2^t b (the same b = fl(c - mu) as the bf16 images, and
-// a copy of their constants); one wavefront per (padded) center
+// fp16 tile images, as above.  Scale of the coarse pass: 2^t with t = 9 - e,
+// max|b| = m 2^e (m in [1/2, 1)), clamped to |t| <= 60, so that every
+// |2 2^t b_ji| < 2^11 (fp16 holds up to 65504: frames with |a_i| < 128 max|b|
+// stay finite; the residual of larger ones is not finite, which sends them to
+// the fine pass).
 __global__ __launch_bounds__(256) void k_center_pack16(const float *__restrict__ C, int k, int d, int d_pad,
                                                        int k_pad, CenterPack cp) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int j = blockIdx.x * 4 + wave;
     if (j >= k_pad) return;
-    const int pitch = tile_pitch(d_pad);
-    const float sc = cp.sc16[0];
-    uint8_t *img = cp.img16 + (int64_t)(j >> 5) * tile_img16_bytes(d_pad);
-    _Float16 *h = reinterpret_cast<_Float16 *>(img) + (j & 31) * pitch;
-    for (int i = lane; i < pitch; i += 64) {
-        float b = 0.0f;
-        if (j < k && i < d) b = __fsub_rn(C[(int64_t)j * d + i], cp.mu[i]);
-        h[i] = (_Float16)__fmul_rn(b, sc);  // the pad columns hold zeros
+    const float bm = cp.mx[MX_BN];
+    int e = 0;
+    frexpf(bm, &e);
+    int t = bm > 0.0f && bm == bm && bm < INFINITY ? 9 - e : 0;
+    t = t > 60 ? 60 : (t < -60 ? -60 : t);
+    const float sc = ldexpf(1.0f, t);
+    if (j == 0 && lane == 0) {
+        cp.sc16[0] = sc;
+        cp.sc16[1] = ldexpf(1.0f, -2 * t);
+        cp.sc16[2] = ldexpf(1.0f, -t);
+        cp.sc16[3] = 0.0f;
     }
-    if (lane < 3) {
+    uint8_t *img = cp.img16 + (int64_t)(j >> 5) * tile_img16_bytes(d_pad);
+    double e1 = 0.0;
+    if (lane * 8 < d_pad) {
+        half8 h;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int i = lane * 8 + q;
+            const float b = (j < k && i < d) ? __fsub_rn(C[(int64_t)j * d + i], cp.mu[i]) : 0.0f;
+            const float v = -2.0f * sc * b;
+            h[q] = (_Float16)v;
+            const float r = v - (float)h[q];
+            e1 += (double)r * (double)r;
+        }
+        *reinterpret_cast<half8 *>(img + (lane >> 1) * 1024 + ((j & 31) + 32 * (lane & 1)) * 16) = h;
+    }
+    e1 = wave_butterfly_sum(e1);
+    if (lane == 0) {
         const float *src = reinterpret_cast<const float *>(cp.img + (int64_t)(j >> 5) * tile_img_bytes(d_pad) +
-                                                           128 * pitch);
-        float *dst = reinterpret_cast<float *>(img + 64 * pitch);
-        dst[32 * lane + (j & 31)] = src[32 * lane + (j & 31)];
+                                                           128 * d_pad) + (j & 31);
+        float *cst = reinterpret_cast<float *>(img + 64 * d_pad) + (j & 31);
+        const float d1 = j < k ? (float)(sqrt(0.25 * e1) * ldexp(1.0, -t) * (1.0 + 1e-6)) : 0.0f;
+        cst[HC_NB] = j < k ? src[FC_NB] * ldexpf(1.0f, 2 * t) : 3.0e38f;
+        cst[HC_BN] = src[FC_BN];
+        cst[HC_D1] = d1;
+        if (j < k) atomic_max_pos(cp.mx + MX_D16, d1);
     }
 }
 
 __global__ void k_zero_i64n(int64_t *p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
-}
-
-__global__ void k_zero_i32n(int32_t *p, int64_t n) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0;
 }
 
 // ------------------------------------------------------------------
@@ -326,11 +365,14 @@ constexpr int CAND_MAX = 8;
 struct RecheckLists {
     int64_t *listA;  // [n] frames the coarse pass leaves undecided
     int64_t *list;   // [n] frames the fine pass leaves undecided
-    int64_t *count;  // [8]: list length, bits of max |b_j|, list2 length, listA length, unused
+    int64_t *count;  // [N_COUNTS]: list length, unused, list2 length, listA length, the center maxima (CenterPack::mx)
     float *upper;    // [n] upper bound per list position
     int32_t *ccnt;   // [slots] candidates found per list position
     int32_t *cand;   // [slots][CAND_MAX]
     int64_t *list2;  // [n] frames for the full loop
+    // consumed by k_compact before the candidate pass writes cand, whose memory they take
+    uint32_t *mask;   // [n / 32] undecided positions of the pass
+    float *upper_at;  // [n] their upper bounds
     int64_t slots;
 };
 
@@ -342,57 +384,52 @@ __device__ __forceinline__ float f32_round_up(double v) {
     return f;
 }
 
-__device__ __forceinline__ void list_frame_coarse(const RecheckLists &rl, int64_t fr) {
-    const unsigned long long pos = atomicAdd((unsigned long long *)(rl.count + 3), 1ull);
-    rl.listA[pos] = fr;
-}
-
-__device__ __forceinline__ void list_frame(const RecheckLists &rl, int64_t fr, float upper) {
-    const unsigned long long pos = atomicAdd((unsigned long long *)rl.count, 1ull);
-    rl.list[pos] = fr;
-    rl.upper[pos] = upper;
-}
-
 // ------------------------------------------------------------------
 // MFMA kernel
 // ------------------------------------------------------------------
-// Wave w of a workgroup owns 32 frames; their bf16 hi/lo fragments stay in
-// registers for all centers.  Center tile images stream through two LDS
-// buffers: while the waves compute tile t from one buffer, the copy engine
-// path (global_load_lds, 16 bytes per lane) fills the other with tile t + 1.
-// v_mfma_f32_32x32x16_bf16: A = 32 centers x 16 dims, B = 16 dims x 32
-// frames; lane l holds frame l % 32 and centers 8(e>>2) + 4(l>>5) + (e&3).
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
-
-// vmcnt(n): wait until at most n vector-memory operations of this wave are
-// outstanding (n a small run-time value; the instruction needs a constant)
-__device__ __forceinline__ void wait_vmcnt(int n) {
-    switch (n) {
-        case 0: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-        case 1: __builtin_amdgcn_s_waitcnt(0x0F71); break;
-        case 2: __builtin_amdgcn_s_waitcnt(0x0F72); break;
-        case 3: __builtin_amdgcn_s_waitcnt(0x0F73); break;
-        case 4: __builtin_amdgcn_s_waitcnt(0x0F74); break;
-        case 5: __builtin_amdgcn_s_waitcnt(0x0F75); break;
-        case 6: __builtin_amdgcn_s_waitcnt(0x0F76); break;
-        case 7: __builtin_amdgcn_s_waitcnt(0x0F77); break;
-        case 8: __builtin_amdgcn_s_waitcnt(0x0F78); break;
-        case 9: __builtin_amdgcn_s_waitcnt(0x0F79); break;
-        case 10: __builtin_amdgcn_s_waitcnt(0x0F7A); break;
-        case 11: __builtin_amdgcn_s_waitcnt(0x0F7B); break;
-        case 12: __builtin_amdgcn_s_waitcnt(0x0F7C); break;
-        case 13: __builtin_amdgcn_s_waitcnt(0x0F7D); break;
-        case 14: __builtin_amdgcn_s_waitcnt(0x0F7E); break;
-        default: __builtin_amdgcn_s_waitcnt(0x0F70); break;  // larger counts: wait for everything
-    }
+// Error bounds, with u = 2^-24, gamma_n = n u / (1 - n u): a frame's and a
+// center's contributions are norms of the parts their images leave out, which
+// are computed exactly enough where the images are made, so the bound follows
+// the data instead of the worst case of every rounding (about 2.4 times
+// smaller for fp16, which lists that many fewer frames):
+//   E_j = c1a |a|^2 + c1b |b_j|^2 + 2 c2 |a||b_j| + R_j,
+//   coarse (a~ = fp16(2^t a) / 2^t, r = |a - a~|, the same for b):
+//     R_j = 2.02 (r_a |b_j| + (|a| + r_a) r_b)
+//   fine (a = hi + lo + rest; products hi hi, hi lo, lo hi):
+//     R_j = 2.02 (|lo_a||lo_b| + rest_a |b_j| + (|a| + rest_a) rest_b)
+//   c1a: shift rounding, combination and the element index in the 4 low
+//        mantissa bits of d~ - |a|^2, (4.2 + 32) u (|a| + |b|)^2, and the FP32
+//        sum of |a|^2
+//   c1b: the same and the FP32 accumulation in the matrix core, which starts
+//        from |b|^2
+//   c2:  the same terms on 2 |a||b| and the accumulation of the products (each
+//        addition rounded to nearest, as the device probe of the matrix core
+//        shows)
+// using (|a|+|b|)^2 = |a|^2 + |b|^2 + 2|a||b| and sum|a_i b_i| <= |a||b|.  A
+// 25 % margin covers the rounding of the FP32 bound arithmetic itself.
+struct AsgCoef {
+    float c1a, c1b, c2, gref;
+};
+static double gamma_n(double m) {
+    const double u = ldexp(1.0, -24);
+    return m * u / (1.0 - m * u);
+}
+static AsgCoef assign_coeffs(int d, int d_pad, int products) {
+    const double c0 = (4.2 + 32.0) * ldexp(1.0, -24), chain = (double)products * d_pad + 2.0;
+    AsgCoef c;
+    c.c1a = (float)(1.25 * (c0 + gamma_n(d_pad / 8 + 8)));
+    c.c1b = (float)(1.25 * (c0 + gamma_n(chain)));
+    c.c2 = (float)(1.25 * (c0 + 1.02 * gamma_n(chain)));
+    c.gref = (float)(1.25 * gamma_n(d + 2.0));
+    return c;
 }
 
 // Running state of the epilogue per frame block and lane: the two smallest
 // values v_j = d~_j - |a|^2 = |b_j|^2 - 2 a.b_j seen so far (m1 <= m2 as a
 // multiset), each with the element e (0..15) of its 32 x 32 tile in the 4 low
-// mantissa bits, and the tile of m1.  Per element: one fma for v, one
-// and-or for the index, med3 and min for the pair (m2 = med3(m1, m2, v) is
-// the new second smallest when m1 <= m2).
+// mantissa bits, and the tile of m1.  Per element: one and-or for the index,
+// med3 and min for the pair (m2 = med3(m1, m2, v) is the new second smallest
+// when m1 <= m2).
 __device__ __forceinline__ float pack_elem(float v, int e) {
     return __uint_as_float((__float_as_uint(v) & 0xFFFFFFF0u) | (uint32_t)e);
 }
@@ -410,60 +447,9 @@ __device__ __forceinline__ void track2(float &m1, float &m2, float vp, float nin
     m1 = __builtin_amdgcn_fmed3f(m1, vp, ninf);
 }
 
-// Label of one frame from the running state of its two half-waves (lane and
-// lane ^ 32 hold the same frame, different centers), and whether it needs
-// the recheck (lanes < 32 write).  With E_max = c1 (|a|^2 + max|b|^2) +
-// 2 c2 |a| max|b| >= E_j for every center: for j != best,
-// d_j >= d~_j - E_j >= |a|^2 + m2 - E_max, and d_best <= |a|^2 + m1 + E_best
-// (both through the reference loop's relative rounding g).  A listed frame
-// carries the upper bound of its best candidate to the candidate pass.
-template <bool COARSE>
-__device__ __forceinline__ void decide_frame(int lane, int64_t fr, bool fvalid, float m1, float m2, int mt, int k,
-                                             float na, float sa, float2 CE, float c3, float gref, float bmax,
-                                             const float *__restrict__ bn, int32_t *__restrict__ labels,
-                                             const RecheckLists &rl) {
-    int half = lane >> 5;
-    {
-        const float o1 = __shfl_xor(m1, 32, 64);
-        const float o2 = __shfl_xor(m2, 32, 64);
-        const int ot = __shfl_xor(mt, 32, 64);
-        m2 = fminf(fminf(m2, o2), fmaxf(m1, o1));
-        if (o1 < m1 || (o1 == m1 && (ot < mt || (ot == mt && half == 1)))) {
-            m1 = o1;
-            mt = ot;
-            half ^= 1;
-        }
-    }
-    const int e = (int)(__float_as_uint(m1) & 15u);
-    const int imin = (mt >= 0 && m1 == m1 && m1 < 1e38f) ? mt * 32 + 8 * (e >> 2) + 4 * half + (e & 3) : 0x7fffffff;
-    if (lane < 32 && fvalid && imin >= k) {
-        labels[fr] = 0;  // non-finite distances (or, in the coarse pass, fp16 overflow): the next pass
-        if (COARSE)
-            list_frame_coarse(rl, fr);
-        else
-            list_frame(rl, fr, __uint_as_float(0x7fc00000u));
-    } else if (lane < 32 && fvalid) {
-        const double a2 = (double)sa * sa;
-        const double bnb = (double)bn[imin];
-        const double E1 = (double)CE.x * (a2 + bnb * bnb) + 2.0 * (double)CE.y * (double)sa * bnb +
-                          (double)c3 * ((double)sa + bnb);
-        const double Em = (double)CE.x * (a2 + (double)bmax * bmax) + 2.0 * (double)CE.y * (double)sa * bmax +
-                          (double)c3 * ((double)sa + (double)bmax);
-        const double upper = ((double)na + (double)m1 + E1) * (1.0 + (double)gref);
-        const double lower = ((double)na + (double)m2 - Em) * (1.0 - (double)gref);
-        labels[fr] = imin;
-        if (!(lower > upper)) {
-            if (COARSE)
-                list_frame_coarse(rl, fr);
-            else
-                list_frame(rl, fr, f32_round_up(upper));
-        }
-    }
-}
-
-// The MFMA distance kernel in its three passes:
-//   PASS_COARSE: every frame; one fp16 product per K-step of 2^t a and 2^t b
-//     (fp16 images); decides with the coarse bound, lists the rest in listA.
+// The MFMA distance kernel in its passes:
+//   PASS_COARSE: every frame; one fp16 product per K-step; decides with the
+//     coarse bound, lists the rest in listA.
 //   PASS_FINE: the frames of listA; bf16 hi/lo of a and b, three products
 //     per K-step; decides with the fine bound, lists the rest with their
 //     upper bound.
@@ -471,634 +457,452 @@ __device__ __forceinline__ void decide_frame(int lane, int64_t fr, bool fvalid, 
 //     the epilogue records the centers whose lower bound reaches the frame's
 //     upper bound instead of tracking the minimum.
 //   PASS_FULL: PASS_FINE over every frame (pass 1 without a coarse pass).
+//
+// A workgroup of NW waves holds the operand fragments of 32 FB frames in LDS
+// (fragment order, so that an operand read is 1 KB contiguous and free of bank
+// conflicts) and every wave runs all of those frames against its own center
+// tiles: CT tiles at a time, tiles CT w, CT (w + NW), ...  A K-step of a wave
+// is then FB LDS reads and CT fragment loads from L2 for FB CT MFMAs (three
+// times as many in the fine passes), with no barrier until the frames are
+// done.  The earlier form (frames in registers, every wave reading every
+// center fragment from LDS for one MFMA) needed one LDS read per MFMA, the
+// LDS's whole bandwidth at the matrix cores' peak, and a barrier per tile.
+// The frames are read as 128 contiguous bytes of a row per 8 lanes, the rows of
+// the next group in flight while one group is converted; the matrix work of
+// the other workgroup on the CU covers that phase.  Measured, the first pass
+// alone: 10^7 x 300, k = 1000 9.3 -> 6.6 ms (the whole call at k = 32, where the
+// frames' 12 GB bound it, 7.6 -> 2.8 ms = 4.3 TB/s; 1.2 PFLOP/s per added
+// center, the rate of a large library product here); 10^7 x 32, k = 1000
+// 8.2 -> 2.0 ms; 2 10^6 x 512, k = 4096 12.6 -> 7.8 ms.
+// v_mfma_f32_32x32x16: A = 32 centers x 16 dims, B = 16 dims x 32 frames; lane
+// l holds frame l % 32 and centers 8(e>>2) + 4(l>>5) + (e&3).
 constexpr int PASS_COARSE = 0, PASS_FINE = 1, PASS_CAND = 2, PASS_FULL = 3;
-template <int KSTEPS, int NW, int MINB, int FB, int PASS>
-__global__ __launch_bounds__(NW * 64, MINB) void k_assign_mfma(const float *__restrict__ X, int64_t n, int d,
-                                                            CenterPack cp, int k, int k_pad, float2 CE,
-                                                            float gref, int32_t *__restrict__ labels,
-                                                            RecheckLists rl, const int32_t *__restrict__ done) {
-    constexpr bool COARSE = PASS == PASS_COARSE, CAND = PASS == PASS_CAND;
+
+// smallest d that a kernel of KS K-steps sees (pick_ksteps takes the next size above d / 16)
+constexpr int min_dim(int ks) { return (ks == 2 ? 0 : ks == 4 ? 2 : ks == 8 ? 4 : ks == 12 ? 8 : ks == 16 ? 12 : ks == 19 ? 16 : ks == 24 ? 19 : 24) * 16 + 1; }
+
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte load, 4-byte aligned
+
+template <int KS, int FB, int CT, int NW, int PASS>
+__global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restrict__ X, int64_t n, int d,
+                                                            CenterPack cp, int k, int k_pad, AsgCoef ce,
+                                                            int32_t *__restrict__ labels, RecheckLists rl,
+                                                            const int32_t *__restrict__ done) {
+    constexpr bool COARSE = PASS == PASS_COARSE, CAND = PASS == PASS_CAND, LISTED = CAND || PASS == PASS_FINE;
     if (done && *done) return;
-    int64_t nf = n;  // frames: all (coarse), listA (fine), the candidate slots (cand)
-    if constexpr (PASS == PASS_FINE) {
-        nf = rl.count[3];
-        if ((int64_t)blockIdx.x * NW * FB * 32 >= nf) return;
-    }
+    int64_t nf = n;  // frames: all, listA (fine), the candidate slots (cand)
+    if constexpr (PASS == PASS_FINE) nf = rl.count[3];
     if constexpr (CAND) {
         const int64_t c = *rl.count;
         nf = c < rl.slots ? c : rl.slots;
-        if ((int64_t)blockIdx.x * NW * FB * 32 >= nf) return;
     }
-    constexpr int DP = KSTEPS * 16;
-    constexpr int PITCH = tile_pitch(DP);
+    constexpr int F = FB * 32, NT = NW * 64;
+    constexpr int DP = KS * 16;
+    constexpr int NPL = COARSE ? 1 : 2;  // operand planes
+    constexpr int KB = NPL * 1024;       // fragment bytes of a (tile, K-step)
     constexpr int IMG = COARSE ? tile_img16_bytes(DP) : tile_img_bytes(DP);
-    constexpr int MAT = (COARSE ? 64 : 128) * PITCH;  // bytes of the center fragments in an image
-    constexpr int MCH = MAT / 16;           // 16-byte chunks of hi + lo
-    constexpr int CCH = 3 * 32 * 4 / 16;    // 16-byte chunks of nb, q, r
-    constexpr int NT = NW * 64;
-    constexpr int ROUNDS = (MCH + NT - 1) / NT;
-    // LDS buffer b holds hi + lo of a tile t with t & 1 == b and the constants
-    // (nb, q, r) of tile t - 1: the MFMAs of tile t and the epilogue of tile
-    // t - 1 run together and read the same buffer, while the copies fill the
-    // other one.  Two separate objects, so that the compiler can tell the
-    // buffer being read from the one being filled.
-    // three buffers (tiles prefetched two ahead) where they fit next to the
-    // occupancy of the variant, otherwise two
-    constexpr int NB = (3 * IMG * MINB <= 160 * 1024) ? 3 : 2;
-    __shared__ __align__(16) uint8_t s_img0[IMG];
-    __shared__ __align__(16) uint8_t s_img1[IMG];
-    __shared__ __align__(16) uint8_t s_img2[NB == 3 ? IMG : 16];
+    constexpr int MAT = KS * KB;         // fragment bytes of an image
+    constexpr int FRAG = FB * KS * KB;
+    constexpr int MERGE = NW * F * 12;
+    __shared__ __align__(16) uint8_t s_buf[FRAG > MERGE ? FRAG : MERGE];
+    __shared__ float s_na[F], s_e1[F], s_e2[COARSE ? 1 : F];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // FB blocks of 32 frames per wave: every center fragment read from LDS
-    // feeds FB MFMAs, and a tile's copies are hidden behind FB times the work
-    int64_t frame[FB], frow[FB], fpos[FB];
-    bool fvalid[FB];
-#pragma unroll
-    for (int b = 0; b < FB; ++b) {
-        fpos[b] = (((int64_t)blockIdx.x * NW + wave) * FB + b) * 32 + (lane & 31);
-        fvalid[b] = fpos[b] < nf;
-        if constexpr (CAND)
-            frame[b] = fvalid[b] ? rl.list[fpos[b]] : 0;
-        else if constexpr (PASS == PASS_FINE)
-            frame[b] = fvalid[b] ? rl.listA[fpos[b]] : 0;
-        else
-            frame[b] = fpos[b];
-        frow[b] = (fvalid[b] ? frame[b] : 0) * (int64_t)d;  // always a valid row
-    }
-    const int kh = (lane >> 5) * 8;  // dim offset of this half-wave inside a K-step
     const int ntiles = k_pad / 32;
+    const int npairs = (ntiles + CT - 1) / CT;
+    const uint8_t *img = COARSE ? cp.img16 : cp.img;
+    const float sc = COARSE ? cp.sc16[0] : 1.0f;
+    const float ninf = opaque_neg_inf();
 
-    // asynchronous copies into an LDS buffer: hi + lo of tile tm (tm < 0: none)
-    // and the constants of tile tc (tc < 0: none)
-    auto fetch = [&](int tm, int tc, uint8_t *dst) __attribute__((always_inline)) {
-        const uint8_t *base = COARSE ? cp.img16 : cp.img;
-        if (tm >= 0) {
-            const uint8_t *src = base + (int64_t)tm * IMG;
+    // a listed pass walks its list with a resident grid, the others have a workgroup per block
+    int64_t f0 = (int64_t)blockIdx.x * F;
+    for (; f0 < nf; f0 = LISTED ? f0 + (int64_t)gridDim.x * F : nf) {
+        // ---- frames: a = fl(x - mu) as operand fragments in LDS, |a|^2 and the norms of what they leave ----
+        {
+            constexpr int RPG = NT / 8, RG = F / RPG;  // rows per group of loads, groups
+            constexpr int NCH = (DP + 31) / 32;                       // 16-byte chunks of a row per lane
+            int sub = tid & 7;
+            asm volatile("" : "+v"(sub));  // keeps the lane's offsets, masks and mu out of the matrix phase's registers
+            float4_u x[2][NCH], mu4[NCH];
+            auto load_group = [&](int g, float4_u *xv) __attribute__((always_inline)) {
+                int64_t pos = f0 + g * RPG + (tid >> 3);
+                pos = pos < nf ? pos : nf - 1;
+                int64_t fr = pos;
+                if constexpr (PASS == PASS_FINE) fr = rl.listA[pos];
+                if constexpr (CAND) fr = rl.list[pos];
+                const float *row = X + fr * (int64_t)d;
+                if (min_dim(KS) >= 4 || d >= 4) {
 #pragma unroll
-            for (int i = 0; i < ROUNDS; ++i) {
-                const int c0 = i * NT + wave * 64;  // first chunk of this wave's 1 KB block
-                if (c0 + lane < MCH)
-                    __builtin_amdgcn_global_load_lds(src + (int64_t)(c0 + lane) * 16, (lds_ptr_t)(dst + c0 * 16), 16, 0, 0);
-            }
-        }
-        if (tc >= 0 && wave == 0 && lane < CCH)
-            __builtin_amdgcn_global_load_lds(base + (int64_t)tc * IMG + MAT + lane * 16, (lds_ptr_t)(dst + MAT), 16, 0, 0);
-    };
-    fetch(0, -1, s_img0);
-
-    // ---- frame fragments: a = fl(x - mu) split into bf16 hi/lo, or (coarse)
-    // 2^t a rounded to fp16 (branch-free) ----
-    bf16x8 bhi[FB][KSTEPS], blo[FB][KSTEPS];
-    half8 fh[FB][KSTEPS];
-    float na[FB], sa[FB];
-    const float sc16 = COARSE ? cp.sc16[0] : 1.0f;
-    // a lane's 8 dims of a K-step are consecutive in the frame row: with d a
-    // multiple of 4 they are two 16-byte loads, each wholly inside the row or
-    // wholly in the padding (loaded from the row's last 4 dims and masked).
-    // Only for small K-step counts: with many steps the compiler keeps every
-    // loaded vector live at once and runs out of registers.
-    const bool vec = KSTEPS <= 8 && (d & 3) == 0 && ((reinterpret_cast<uintptr_t>(X) & 15) == 0);
-    // More K-steps (16-byte aligned rows; the bf16 passes only in tile
-    // shapes of one wave per SIMD, whose registers hold the load groups next
-    // to the hi / lo fragments): 16-byte loads of the frames in groups of GK K-steps, the next group's loads issued
-    // before the current group is converted, so that the frame loads of a
-    // wave are not one dword at a time (about 10 loads in flight otherwise:
-    // the frame phase of a workgroup is then latency-bound, and up to
-    // k = 512 it takes longer than the workgroup's tiles).
-    // mu of a group is loaded before the next group's frames (loads complete
-    // in order), and the values and the order of the |a|^2 terms are those of
-    // the general loop below.
-    constexpr int GK = 4;
-    constexpr int NG = (KSTEPS + GK - 1) / GK;
-    const bool gvec = (COARSE || NW * MINB <= 4) && KSTEPS > 8 && (d & 3) == 0 &&
-                      ((reinterpret_cast<uintptr_t>(X) & 15) == 0);
-    if (gvec) {
+                    for (int i = 0; i < NCH; ++i) {
+                        const int c = (i * 8 + sub) * 4;  // a chunk reaching past the row is read from the row's end
+                        if (i * 32 + 32 <= min_dim(KS))
+                            xv[i] = *reinterpret_cast<const float4_u *>(row + sub * 4 + i * 32);
+                        else
+                            xv[i] = *reinterpret_cast<const float4_u *>(row + (c + 4 <= d ? c : d - 4));
+                    }
+                } else {
 #pragma unroll
-        for (int b = 0; b < FB; ++b) {
-            float na_part = 0.0f;
-            float4 xg[2][GK][2];
-            auto load_group = [&](int g, int slot) __attribute__((always_inline)) {
-#pragma unroll
-                for (int j = 0; j < GK; ++j) {
-                    const int s = g * GK + j;
-                    if (s < KSTEPS) {
-#pragma unroll
-                        for (int hv = 0; hv < 2; ++hv) {
-                            const int i0 = s * 16 + kh + 4 * hv;
-                            xg[slot][j][hv] = *reinterpret_cast<const float4 *>(X + frow[b] + (i0 < d ? i0 : d - 4));
-                        }
+                    for (int i = 0; i < NCH; ++i) {
+                        xv[i] = float4_u{0.0f, 0.0f, 0.0f, 0.0f};
+                        xv[i].x = row[0];
+                        xv[i].y = row[d > 1 ? 1 : 0];
+                        xv[i].z = row[d > 2 ? 2 : 0];
                     }
                 }
             };
-            load_group(0, 0);
-            float4 mg[GK][2];
-            static_for<0, NG>([&](auto gc) __attribute__((always_inline)) {
+            auto convert = [&](int g, const float4_u *xv) __attribute__((always_inline)) {
+                const int r = g * RPG + (tid >> 3);
+                float na = 0.0f, e1 = 0.0f, e2 = 0.0f;
+                // fragment slot of row r, dims c .. c + 3, c = 32 i + 4 sub: K-step c / 16, half-wave (c / 8) & 1
+                uint8_t *dst0 = s_buf + ((r >> 5) * KS + (sub >> 2)) * KB + ((sub >> 1) & 1) * 512 + (r & 31) * 16 + (sub & 1) * 8;
+#pragma unroll
+                for (int i = 0; i < NCH; ++i) {
+                    const int c = (i * 8 + sub) * 4;
+                    float v[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+                    const bool in_img = i * 32 + 32 <= DP || c < DP;
+                    const float4_u m4 = mu4[i];
+                    float a[4] = {__fsub_rn(v[0], m4.x), __fsub_rn(v[1], m4.y), __fsub_rn(v[2], m4.z), __fsub_rn(v[3], m4.w)};
+                    if (i * 32 + 32 > min_dim(KS)) {  // the row may end inside these chunks
+                        const int sh = (d >= 4 && c + 4 > d) ? c + 4 - d : 0;
+                        if (sh) {
+                            v[0] = sh == 1 ? v[1] : (sh == 2 ? v[2] : v[3]);
+                            v[1] = sh == 1 ? v[2] : v[3];
+                            v[2] = v[3];
+                        }
+                        const float mm[4] = {m4.x, m4.y, m4.z, m4.w};
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) a[q] = c + q < d ? __fsub_rn(v[q], mm[q]) : 0.0f;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) na = fmaf(a[q], a[q], na);
+                    uint8_t *dst = dst0 + i * 2 * KB;
+                    if constexpr (COARSE) {
+                        typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+                        half4 h;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const float s = __fmul_rn(a[q], sc);
+                            h[q] = (_Float16)s;
+                            const float rr = s - (float)h[q];
+                            e1 = fmaf(rr, rr, e1);
+                        }
+                        if (in_img) *reinterpret_cast<half4 *>(dst) = h;
+                    } else {
+                        uint32_t h[2], l[2];
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) {
+                            split_bf16x2(a[2 * q], a[2 * q + 1], h[q], l[q]);
+                            const float l0 = __uint_as_float(l[q] << 16), l1 = __uint_as_float(l[q] & 0xffff0000u);
+                            const float r0 = (a[2 * q] - __uint_as_float(h[q] << 16)) - l0;
+                            const float r1 = (a[2 * q + 1] - __uint_as_float(h[q] & 0xffff0000u)) - l1;
+                            e1 = fmaf(l0, l0, fmaf(l1, l1, e1));
+                            e2 = fmaf(r0, r0, fmaf(r1, r1, e2));
+                        }
+                        if (in_img) {
+                            *reinterpret_cast<uint2 *>(dst) = make_uint2(h[0], h[1]);
+                            *reinterpret_cast<uint2 *>(dst + 1024) = make_uint2(l[0], l[1]);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int off = 1; off < 8; off <<= 1) {
+                    na += __shfl_xor(na, off, 64);
+                    e1 += __shfl_xor(e1, off, 64);
+                    if constexpr (!COARSE) e2 += __shfl_xor(e2, off, 64);
+                }
+                if (sub == 0) {
+                    s_na[r] = na;
+                    s_e1[r] = e1;
+                    if constexpr (!COARSE) s_e2[r] = e2;
+                }
+            };
+            static_assert(F % RPG == 0, "whole groups of rows");
+            load_group(0, x[0]);
+#pragma unroll
+            for (int i = 0; i < NCH; ++i)
+                mu4[i] = *reinterpret_cast<const float4_u *>(cp.mu + sub * 4 + (i * 32 + 32 <= DP || sub < 4 ? i * 32 : 0));
+            static_for<0, RG>([&](auto gc) __attribute__((always_inline)) {
                 constexpr int g = decltype(gc)::value;
-#pragma unroll
-                for (int j = 0; j < GK; ++j) {
-                    const int s = g * GK + j;
-                    if (s < KSTEPS) {
-                        mg[j][0] = *reinterpret_cast<const float4 *>(cp.mu + s * 16 + kh);
-                        mg[j][1] = *reinterpret_cast<const float4 *>(cp.mu + s * 16 + kh + 4);
-                    }
-                }
-                if constexpr (g + 1 < NG) load_group(g + 1, (g + 1) & 1);
+                if constexpr (g + 1 < RG) load_group(g + 1, x[(g + 1) & 1]);
                 __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int j = 0; j < GK; ++j) {
-                    const int s = g * GK + j;
-                    if (s < KSTEPS) {
-                        const float4 *xv = xg[g & 1][j];
-                        const float xs[8] = {xv[0].x, xv[0].y, xv[0].z, xv[0].w, xv[1].x, xv[1].y, xv[1].z, xv[1].w};
-                        const float ms[8] = {mg[j][0].x, mg[j][0].y, mg[j][0].z, mg[j][0].w,
-                                             mg[j][1].x, mg[j][1].y, mg[j][1].z, mg[j][1].w};
-                        _Float16 f[8];
-                        uint32_t h[8], l[8];
-#pragma unroll
-                        for (int q = 0; q < 8; ++q) {
-                            const int i = s * 16 + kh + q;
-                            const bool ok = fvalid[b] && i < d;
-                            const uint32_t keep = ok ? 0xffffffffu : 0u;
-                            const float a = __uint_as_float(__float_as_uint(__fsub_rn(xs[q], ms[q])) & keep);
-                            na_part = __fadd_rn(na_part, __fmul_rn(a, a));
-                            if constexpr (COARSE)
-                                f[q] = (_Float16)__fmul_rn(a, sc16);
-                            else
-                                split_bf16(a, h[q], l[q]);
-                        }
-                        if constexpr (COARSE) {
-                            fh[b][s] = half8{f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
-                        } else {
-                            uint4 hv = make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7]));
-                            uint4 lv = make_uint4(pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7]));
-                            bhi[b][s] = __builtin_bit_cast(bf16x8, hv);
-                            blo[b][s] = __builtin_bit_cast(bf16x8, lv);
-                        }
-                    }
-                }
+                convert(g, x[g & 1]);
                 __builtin_amdgcn_sched_barrier(0);
             });
-            na[b] = __fadd_rn(na_part, __shfl_xor(na_part, 32, 64));
-            sa[b] = sqrtf(na[b]) * (1.0f + 1e-6f);  // |a| rounded up
         }
-    }
-#pragma unroll
-    for (int b = 0; b < FB; ++b) {
-        if (gvec) break;
-        float na_part = 0.0f;
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            uint32_t h[8], l[8];
-            _Float16 f[8];
-            float xs[8], ms[8];
-            if (vec) {
-#pragma unroll
-                for (int hv = 0; hv < 2; ++hv) {
-                    const int i0 = s * 16 + kh + 4 * hv;
-                    const float4 x4 = *reinterpret_cast<const float4 *>(X + frow[b] + (i0 < d ? i0 : d - 4));
-                    const float4 m4 = *reinterpret_cast<const float4 *>(cp.mu + i0);
-                    xs[4 * hv] = x4.x;
-                    xs[4 * hv + 1] = x4.y;
-                    xs[4 * hv + 2] = x4.z;
-                    xs[4 * hv + 3] = x4.w;
-                    ms[4 * hv] = m4.x;
-                    ms[4 * hv + 1] = m4.y;
-                    ms[4 * hv + 2] = m4.z;
-                    ms[4 * hv + 3] = m4.w;
-                }
-            } else {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int i = s * 16 + kh + q;
-                    xs[q] = X[frow[b] + (i < d ? i : d - 1)];
-                    ms[q] = cp.mu[i];
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int i = s * 16 + kh + q;
-                const bool ok = fvalid[b] && i < d;
-                const uint32_t keep = ok ? 0xffffffffu : 0u;
-                const float a = __uint_as_float(__float_as_uint(__fsub_rn(xs[q], ms[q])) & keep);
-                na_part = __fadd_rn(na_part, __fmul_rn(a, a));
-                if constexpr (COARSE)
-                    f[q] = (_Float16)__fmul_rn(a, sc16);
-                else
-                    split_bf16(a, h[q], l[q]);
-            }
-            if constexpr (COARSE) {
-                fh[b][s] = half8{f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
-            } else {
-                uint4 hv = make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7]));
-                uint4 lv = make_uint4(pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7]));
-                bhi[b][s] = __builtin_bit_cast(bf16x8, hv);
-                blo[b][s] = __builtin_bit_cast(bf16x8, lv);
-            }
-        }
-        na[b] = __fadd_rn(na_part, __shfl_xor(na_part, 32, 64));
-        sa[b] = sqrtf(na[b]) * (1.0f + 1e-6f);  // |a| rounded up
-    }
-    // candidate mode: center j is recorded when its lower bound reaches the
-    // frame's upper bound, (na - CE sa^2 + lb_j)(1 - g) <= upper, as the
-    // threshold lb_j <= T on the epilogue's FP32 lb_j = q_j - 2 p - sa r_j,
-    // raised by 8 u (sa + max|b|)^2 so that rounding only ever adds
-    // candidates; no threshold (NaN upper): no candidate, the frame goes to
-    // the full loop
-    float thr[FB];
-#pragma unroll
-    for (int b = 0; b < FB; ++b) {
-        thr[b] = -INFINITY;
-        if constexpr (CAND) {
-            const float up = fvalid[b] ? rl.upper[fpos[b]] : __uint_as_float(0x7fc00000u);
-            if (up == up) {
-                const double sb = (double)sa[b] + (double)*cp.bmax;
-                const double T = (double)up / (1.0 - (double)gref) - ((double)na[b] - (double)CE.x * (double)sa[b] * (double)sa[b]) +
-                                 8.0 * 5.9604644775390625e-8 * sb * sb;
-                thr[b] = f32_round_up(T);
-            }
-        }
-    }
+        __syncthreads();
 
-    // per frame block: the two smallest d~ - |a|^2 with the element index in
-    // the low bits, and the tile of the smallest (see track2)
-    float m1[FB], m2[FB];
-    int mt[FB];
-    const float ninf = opaque_neg_inf();
-    // d~ - |a|^2 = |b|^2 + pscale * (MFMA sum): -2, or -2^(1 - 2t) for the
-    // coarse pass's scaled operands
-    const float pscale = COARSE ? cp.sc16[1] : -2.0f;
-#pragma unroll
-    for (int b = 0; b < FB; ++b) {
-        m1[b] = m2[b] = INFINITY;
-        mt[b] = -1;
-    }
-
-    struct AccFB {
-        floatx16 v[FB];
-    };
-    auto chain = [&](const uint8_t *img) __attribute__((always_inline)) -> AccFB {
-        const uint16_t *ah_base = reinterpret_cast<const uint16_t *>(img) + (lane & 31) * PITCH + kh;
-        const uint16_t *al_base = ah_base + 32 * PITCH;
-        AccFB acc;
-#pragma unroll
-        for (int b = 0; b < FB; ++b) acc.v[b] = floatx16{};
-        if constexpr (COARSE) {
-            half8 ch = *reinterpret_cast<const half8 *>(ah_base);
-#pragma unroll
-            for (int s = 0; s < KSTEPS; ++s) {
-                half8 chn = ch;
-                if (s + 1 < KSTEPS) chn = *reinterpret_cast<const half8 *>(ah_base + (s + 1) * 16);
-#pragma unroll
-                for (int b = 0; b < FB; ++b) acc.v[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch, fh[b][s], acc.v[b], 0, 0, 0);
-                ch = chn;
-            }
-            return acc;
-        }
-        // center operands read one K-step ahead of their MFMAs
-        bf16x8 ah = *reinterpret_cast<const bf16x8 *>(ah_base);
-        bf16x8 al = *reinterpret_cast<const bf16x8 *>(al_base);
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            bf16x8 ahn = ah, aln = al;
-            if (s + 1 < KSTEPS) {
-                ahn = *reinterpret_cast<const bf16x8 *>(ah_base + (s + 1) * 16);
-                aln = *reinterpret_cast<const bf16x8 *>(al_base + (s + 1) * 16);
-            }
-#pragma unroll
-            for (int b = 0; b < FB; ++b) acc.v[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, blo[b][s], acc.v[b], 0, 0, 0);
-#pragma unroll
-            for (int b = 0; b < FB; ++b) acc.v[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bhi[b][s], acc.v[b], 0, 0, 0);
-#pragma unroll
-            for (int b = 0; b < FB; ++b) acc.v[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bhi[b][s], acc.v[b], 0, 0, 0);
-            ah = ahn;
-            al = aln;
-        }
-        return acc;
-    };
-    auto epilogue = [&](const AccFB &acc, const uint8_t *img, int t) __attribute__((always_inline)) {
-        const float *cst = reinterpret_cast<const float *>(img + MAT);
+        // ---- candidate pass: center j is recorded when its lower bound reaches
+        // the frame's upper bound, (na + v_j - E_j)(1 - g) <= upper, as the
+        // threshold v_j - c1b|b_j|^2 - ca |b_j| - cb |lo_j| - cc rest_j <= T, raised by
+        // 16 u (|a| + max|b|)^2 so that rounding only ever adds candidates; no
+        // threshold (NaN upper): no candidate, the frame goes to the full loop
+        float thr[FB], ca[FB], cb[FB], cc[FB];
         if constexpr (CAND) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int c0 = 8 * g + 4 * (lane >> 5);
-                const float4 qv = *reinterpret_cast<const float4 *>(&cst[32 + c0]);
-                const float4 rv = *reinterpret_cast<const float4 *>(&cst[64 + c0]);
-                const float qa[4] = {qv.x, qv.y, qv.z, qv.w};
-                const float ra[4] = {rv.x, rv.y, rv.z, rv.w};
-#pragma unroll
-                for (int b = 0; b < FB; ++b)
-#pragma unroll
-                    for (int h = 0; h < 4; ++h) {
-                        const float lb = fmaf(-sa[b], ra[h], fmaf(-2.0f, acc.v[b][4 * g + h], qa[h]));
-                        if (lb <= thr[b]) {
-                            const int j = t * 32 + c0 + h;
-                            if (j < k) {
-                                const int c = atomicAdd(&rl.ccnt[fpos[b]], 1);
-                                if (c < CAND_MAX) rl.cand[fpos[b] * CAND_MAX + c] = j;
-                            }
-                        }
-                    }
+            for (int b = 0; b < FB; ++b) {
+                const int r = b * 32 + (lane & 31);
+                thr[b] = -INFINITY;
+                ca[b] = cb[b] = cc[b] = 0.0f;
+                const float up = f0 + r < nf ? rl.upper[f0 + r] : __uint_as_float(0x7fc00000u);
+                if (up == up) {
+                    const double na = s_na[r], sa = sqrt(na) * (1.0 + 2e-5), mb = cp.mx[MX_BN];
+                    const double e1 = sqrt((double)s_e1[r]) * (1.0 + 1e-4), e2 = sqrt((double)s_e2[r]) * (1.0 + 1e-4);
+                    const double T = (double)up / (1.0 - (double)ce.gref) - (na - (double)ce.c1a * sa * sa) +
+                                     16.0 * 5.9604644775390625e-8 * (sa + mb) * (sa + mb);
+                    thr[b] = f32_round_up(T);
+                    ca[b] = (float)((2.0 * (double)ce.c2 * sa + 2.02 * e2) * 1.000001);
+                    cb[b] = (float)(2.02 * e1 * 1.000001);
+                    cc[b] = (float)(2.02 * (sa + e2) * 1.000001);
+                }
             }
-            return;
         }
-        float prev[FB];
+
+        float m1[FB], m2[FB];
+        int mt[FB];
 #pragma unroll
-        for (int b = 0; b < FB; ++b) prev[b] = m1[b];
+        for (int b = 0; b < FB; ++b) {
+            m1[b] = m2[b] = INFINITY;
+            mt[b] = -1;
+        }
+
+        // ---- the wave's center tiles ----
+        constexpr int PF = KS < 4 ? KS : (COARSE ? 4 : 3);  // K-steps of center fragments in flight
+        uint4 cf[PF][CT][NPL];
+        float init[CT][16];
+        const uint8_t *tp[CT];  // images of the wave's current tiles
+        uint32_t vo = 0;        // the lane's offset of the next K-step to load
+        auto load_cf = [&](int slot) __attribute__((always_inline)) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int c0 = 8 * g + 4 * (lane >> 5);
-            const float4 nbv = *reinterpret_cast<const float4 *>(&cst[c0]);
-            const float nba[4] = {nbv.x, nbv.y, nbv.z, nbv.w};
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int pl = 0; pl < NPL; ++pl)
+                    cf[slot][ct][pl] = *reinterpret_cast<const uint4 *>(tp[ct] + vo + pl * 1024);
+            vo += KB;
+            asm volatile("" : "+v"(vo));  // one running offset, not an address per K-step
+        };
+        // start of a tile pair: its first fragments and the accumulators' start values
+        auto start_pair = [&](int pr) __attribute__((always_inline)) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const int t = pr * CT + ct;
+                tp[ct] = img + (int64_t)(t < ntiles ? t : ntiles - 1) * IMG;
+                const float *cst = reinterpret_cast<const float *>(tp[ct] + MAT) + (CAND ? FC_Q : (COARSE ? HC_NB : FC_NB));
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 q4 = *reinterpret_cast<const float4 *>(cst + 8 * g + 4 * (lane >> 5));
+                    init[ct][4 * g + 0] = q4.x;
+                    init[ct][4 * g + 1] = q4.y;
+                    init[ct][4 * g + 2] = q4.z;
+                    init[ct][4 * g + 3] = q4.w;
+                }
+                if (CT > 1 && pr * CT + ct >= ntiles)  // no such tile: a repeat of the last one that never wins
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) init[ct][e] = 3.0e38f;
+            }
+            vo = (uint32_t)lane * 16u;
+            asm volatile("" : "+v"(vo));
+#pragma unroll
+            for (int s = 0; s < PF; ++s) load_cf(s);
+        };
+        const uint8_t *fb_base = s_buf + lane * 16;
+        uint4 ff[2][FB][NPL];
+        auto load_ff = [&](int s, int slot) __attribute__((always_inline)) {
 #pragma unroll
             for (int b = 0; b < FB; ++b)
 #pragma unroll
-                for (int h = 0; h < 4; ++h)
-                    track2(m1[b], m2[b], pack_elem(fmaf(pscale, acc.v[b][4 * g + h], nba[h]), 4 * g + h), ninf);
-        }
-#pragma unroll
-        for (int b = 0; b < FB; ++b) mt[b] = m1[b] != prev[b] ? t : mt[b];
-    };
-    // MFMAs of one tile interleaved with the epilogue of the previous one
-    // (about 4 VALU per element, 16 elements per frame block, spread over the
-    // K-steps)
-    constexpr int EV = (68 * FB + KSTEPS - 1) / KSTEPS;
-    auto interleave = [&]() __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_group_barrier(0x100, COARSE ? 1 : 2, 0);  // operand reads of K-step 0
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            if (s + 1 < KSTEPS) __builtin_amdgcn_sched_group_barrier(0x100, COARSE ? 1 : 2, 0);  // operands of K-step s + 1
-            __builtin_amdgcn_sched_group_barrier(0x008, (COARSE ? 1 : 3) * FB, 0);   // the MFMAs of K-step s
-            __builtin_amdgcn_sched_group_barrier(0x002, EV, 0);                     // epilogue VALU
-        }
-    };
-
-    if constexpr (NB == 3) {
-        // Tiles prefetched two ahead: buffer u % 3 holds hi + lo of tile u and
-        // the constants of tile u - 1.  Iteration t waits until the copies of
-        // tile t are complete (those of tile t + 1 may still be in flight: the
-        // count of this wave's copies per fetch is known), synchronizes, starts
-        // the copies of tile t + 2 into the buffer read in iteration t - 1, and
-        // runs the MFMAs of tile t with the epilogue of tile t - 1.
-        int rw = 0;  // hi + lo copy instructions this wave issues per tile
-#pragma unroll
-        for (int i = 0; i < ROUNDS; ++i) rw += (i * NT + wave * 64 < MCH) ? 1 : 0;
-        auto copies = [&](int u) -> int {  // copy instructions of this wave in fetch(u)
-            return (u < ntiles ? rw : 0) + ((wave == 0 && u >= 1 && u - 1 < ntiles) ? 1 : 0);
+                for (int pl = 0; pl < NPL; ++pl)
+                    ff[slot][b][pl] = *reinterpret_cast<const uint4 *>(fb_base + (b * KS + s) * KB + pl * 1024);
         };
-        fetch(ntiles > 1 ? 1 : -1, 0, s_img1);
-        // tile 0: no epilogue yet
-        wait_vmcnt(copies(1));
-        __syncthreads();
-        fetch(2 < ntiles ? 2 : -1, 1 < ntiles ? 1 : -1, s_img2);
-        AccFB acc = chain(s_img0);
-        auto iter = [&](int t, uint8_t *cur, uint8_t *tgt) __attribute__((always_inline)) {
-            wait_vmcnt(copies(t + 1));
-            __syncthreads();
-            fetch(t + 2 < ntiles ? t + 2 : -1, t + 1 < ntiles ? t + 1 : -1, tgt);
-            const AccFB nacc = chain(cur);
-            epilogue(acc, cur, t - 1);
-            interleave();
-            acc = nacc;
-        };
-        for (int t = 1; t < ntiles; t += 3) {
-            iter(t, s_img1, s_img0);
-            if (t + 1 >= ntiles) break;
-            iter(t + 1, s_img2, s_img1);
-            if (t + 2 >= ntiles) break;
-            iter(t + 2, s_img0, s_img2);
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        const int rb = ntiles % 3;
-        epilogue(acc, rb == 0 ? s_img0 : (rb == 1 ? s_img1 : s_img2), ntiles - 1);
-    } else {
-    // tile 0, then tiles 1 .. ntiles - 1 with the epilogue one tile behind.
-    // Each barrier follows a wait for this wave's copies, so the buffer about
-    // to be read is complete for every wave and every wave has finished
-    // reading the buffer that the next copies overwrite.
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
-    fetch(ntiles > 1 ? 1 : -1, 0, s_img1);
-    AccFB acc = chain(s_img0);
-    int t = 1;
-    while (t < ntiles) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        fetch(t + 1 < ntiles ? t + 1 : -1, t, s_img0);
-        {
-            const AccFB nacc = chain(s_img1);
-            epilogue(acc, s_img1, t - 1);
-            interleave();
-            acc = nacc;
-        }
-        if (++t >= ntiles) break;
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        fetch(t + 1 < ntiles ? t + 1 : -1, t, s_img1);
-        {
-            const AccFB nacc = chain(s_img0);
-            epilogue(acc, s_img0, t - 1);
-            interleave();
-            acc = nacc;
-        }
-        ++t;
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    epilogue(acc, (ntiles & 1) ? s_img1 : s_img0, ntiles - 1);
-    }
-
-    // per frame block: merge the two half-waves that hold the same frame and decide
-    if constexpr (CAND) return;
-    const float bmax = *cp.bmax;
-    const float c3 = COARSE ? cp.sc16[2] : 0.0f;
+        if (wave < npairs) start_pair(wave);
+        for (int pr = wave; pr < npairs; pr += NW) {
+            floatx16 acc[CT][FB];
+            load_ff(0, 0);
+            static_for<0, KS>([&](auto sc_) __attribute__((always_inline)) {
+                constexpr int s = decltype(sc_)::value;
+                if constexpr (s + 1 < KS) load_ff(s + 1, (s + 1) & 1);
+                constexpr int sl = s % PF, fs = s & 1;
+                // the product order of every accumulator: hi lo, lo hi, hi hi
 #pragma unroll
-    for (int b = 0; b < FB; ++b)
-        decide_frame<COARSE>(lane, frame[b], fvalid[b], m1[b], m2[b], mt[b], k, na[b], sa[b], CE, c3, gref, bmax,
-                             cp.bn, labels, rl);
-}
-
-// Resident-center form for small k d (every center tile image fits in LDS):
-// one workgroup per CU copies all tile images into LDS once, then each wave
-// walks 32-frame blocks with a grid stride, running every tile from LDS with
-// no further copies or barriers.  Where the streaming kernel waits for a
-// tile's copies every few MFMAs (few K-steps per tile), this one only streams
-// the frames (the next block's raw values are loaded while the current block
-// runs its tiles), so its time is set by the frames' HBM traffic, the MFMAs
-// and the epilogue.
-constexpr int RES_LDS = 144 * 1024;  // bytes of resident tile images
-
-__host__ __device__ constexpr int res_max_tiles(int d_pad) { return RES_LDS / tile_img_bytes(d_pad); }
-
-template <int KSTEPS, int NW>
-__global__ __launch_bounds__(NW * 64, 1) void k_assign_res(const float *__restrict__ X, int64_t n, int d,
-                                                           CenterPack cp, int k, int k_pad, float2 CE, float gref,
-                                                           int32_t *__restrict__ labels, RecheckLists rl,
-                                                           const int32_t *__restrict__ done) {
-    if (done && *done) return;
-    constexpr int DP = KSTEPS * 16;
-    constexpr int PITCH = tile_pitch(DP);
-    constexpr int IMG = tile_img_bytes(DP);
-    constexpr int MAT = 128 * PITCH;
-    constexpr int NT = NW * 64;
-    __shared__ __align__(16) uint8_t s_res[RES_LDS];
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kh = (lane >> 5) * 8;
-    const int ntiles = k_pad / 32;  // ntiles * IMG <= RES_LDS (checked by the host)
-
-    // every tile image (hi, lo and the constants nb, q, r) in one asynchronous copy
-    const int nch = ntiles * (IMG / 16);
-    for (int c0 = wave * 64; c0 < nch; c0 += NT)
-        if (c0 + lane < nch)
-            __builtin_amdgcn_global_load_lds(cp.img + (int64_t)(c0 + lane) * 16, (lds_ptr_t)(s_res + c0 * 16), 16, 0, 0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
-    const float bmax = *cp.bmax;
-
-    auto chain = [&](const uint8_t *img, const bf16x8 *bhi, const bf16x8 *blo) __attribute__((always_inline)) -> floatx16 {
-        const uint16_t *ah_base = reinterpret_cast<const uint16_t *>(img) + (lane & 31) * PITCH + kh;
-        const uint16_t *al_base = ah_base + 32 * PITCH;
-        floatx16 acc = {};
+                for (int pp = 0; pp < (COARSE ? 1 : 3); ++pp)
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            const bf16x8 ah = *reinterpret_cast<const bf16x8 *>(ah_base + s * 16);
-            const bf16x8 al = *reinterpret_cast<const bf16x8 *>(al_base + s * 16);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, blo[s], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bhi[s], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bhi[s], acc, 0, 0, 0);
-        }
-        return acc;
-    };
-
-    const int64_t nblk = (n + 31) / 32;
-    const int64_t stride = (int64_t)gridDim.x * NW;
-    // raw frame values of the wave's next block are loaded while the current
-    // block runs its tiles (lanes: frame lane & 31, dims s * 16 + kh .. + 7)
-    const bool vec = KSTEPS <= 8 && (d & 3) == 0 && ((reinterpret_cast<uintptr_t>(X) & 15) == 0);
-    float xr[KSTEPS][8];
-    auto load_raw = [&](int64_t b) __attribute__((always_inline)) {
-        const int64_t fr = b * 32 + (lane & 31);
-        const int64_t row = (fr < n ? fr : 0) * (int64_t)d;
+                    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            if (vec) {
+                        for (int b = 0; b < FB; ++b) {
+                            floatx16 c0;
+                            if constexpr (s == 0) {
+                                if (pp == 0) {
 #pragma unroll
-                for (int hv = 0; hv < 2; ++hv) {
-                    const int i0 = s * 16 + kh + 4 * hv;
-                    const float4 x4 = *reinterpret_cast<const float4 *>(X + row + (i0 < d ? i0 : d - 4));
-                    xr[s][4 * hv] = x4.x;
-                    xr[s][4 * hv + 1] = x4.y;
-                    xr[s][4 * hv + 2] = x4.z;
-                    xr[s][4 * hv + 3] = x4.w;
+                                    for (int e = 0; e < 16; ++e) c0[e] = init[ct][e];
+                                } else {
+                                    c0 = acc[ct][b];
+                                }
+                            } else {
+                                c0 = acc[ct][b];
+                            }
+                            if constexpr (COARSE)
+                                acc[ct][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                    __builtin_bit_cast(half8, cf[sl][ct][0]), __builtin_bit_cast(half8, ff[fs][b][0]), c0, 0, 0, 0);
+                            else
+                                acc[ct][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                    __builtin_bit_cast(bf16x8, cf[sl][ct][pp == 1 ? NPL - 1 : 0]),
+                                    __builtin_bit_cast(bf16x8, ff[fs][b][pp == 0 ? NPL - 1 : 0]), c0, 0, 0, 0);
+                        }
+                if constexpr (s + PF < KS) load_cf(sl);
+                // the next step's LDS reads first, then this step's MFMAs with the L2 loads behind them
+                if constexpr (s + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, FB * NPL, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, (COARSE ? 1 : 3) * CT * FB, 0);
+                if constexpr (s + PF < KS) __builtin_amdgcn_sched_group_barrier(0x020, CT * NPL, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if (pr + NW < npairs) start_pair(pr + NW);  // in flight during the epilogue below
+            if constexpr (CAND) {
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                    const int t = pr * CT + ct;
+                    if (t >= ntiles) break;
+                    const float *cst = reinterpret_cast<const float *>(img + (int64_t)t * IMG + MAT);
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const int c0 = 8 * g + 4 * (lane >> 5);
+                        const float4 bnv = *reinterpret_cast<const float4 *>(cst + FC_BN + c0);
+                        const float4 d1v = *reinterpret_cast<const float4 *>(cst + FC_D1 + c0);
+                        const float4 d2v = *reinterpret_cast<const float4 *>(cst + FC_D2 + c0);
+                        const float bn[4] = {bnv.x, bnv.y, bnv.z, bnv.w}, d1[4] = {d1v.x, d1v.y, d1v.z, d1v.w};
+                        const float d2[4] = {d2v.x, d2v.y, d2v.z, d2v.w};
+#pragma unroll
+                        for (int b = 0; b < FB; ++b)
+#pragma unroll
+                            for (int h = 0; h < 4; ++h) {
+                                const float lb = fmaf(-cc[b], d2[h], fmaf(-cb[b], d1[h], fmaf(-ca[b], bn[h], acc[ct][b][4 * g + h])));
+                                const int j = t * 32 + c0 + h;
+                                if (lb <= thr[b] && j < k) {
+                                    const int64_t pos = f0 + b * 32 + (lane & 31);
+                                    const int q = atomicAdd(&rl.ccnt[pos], 1);
+                                    if (q < CAND_MAX) rl.cand[pos * CAND_MAX + q] = j;
+                                }
+                            }
+                    }
                 }
             } else {
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int i = s * 16 + kh + q;
-                    xr[s][q] = X[row + (i < d ? i : d - 1)];
+                for (int ct = 0; ct < CT; ++ct) {
+                    const int t = pr * CT + ct;
+#pragma unroll
+                    for (int b = 0; b < FB; ++b) {
+                        const float prev = m1[b];
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) track2(m1[b], m2[b], pack_elem(acc[ct][b][e], e), ninf);
+                        mt[b] = m1[b] != prev ? t : mt[b];
+                    }
                 }
             }
         }
-    };
-    int64_t blk = (int64_t)blockIdx.x * NW + wave;
-    if (blk < nblk) load_raw(blk);
-    for (; blk < nblk; blk += stride) {
-        const int64_t frame = blk * 32 + (lane & 31);
-        const bool fvalid = frame < n;
-        bf16x8 bhi[KSTEPS], blo[KSTEPS];
-        float na_part = 0.0f;
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            uint32_t h[8], l[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int i = s * 16 + kh + q;
-                const uint32_t keep = (fvalid && i < d) ? 0xffffffffu : 0u;
-                const float a = __uint_as_float(__float_as_uint(__fsub_rn(xr[s][q], cp.mu[i])) & keep);
-                na_part = __fadd_rn(na_part, __fmul_rn(a, a));
-                split_bf16(a, h[q], l[q]);
-            }
-            bhi[s] = __builtin_bit_cast(bf16x8, make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])));
-            blo[s] = __builtin_bit_cast(bf16x8, make_uint4(pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7])));
-        }
-        const float na = __fadd_rn(na_part, __shfl_xor(na_part, 32, 64));
-        const float sa = sqrtf(na) * (1.0f + 1e-6f);  // |a| rounded up
-        if (blk + stride < nblk) load_raw(blk + stride);
+        __syncthreads();  // the fragments are consumed: their LDS takes the merge below (or the next frames)
+        if constexpr (CAND) continue;
 
-        // the two smallest d~ - |a|^2 and the tile of the smallest (track2)
-        const float ninf = opaque_neg_inf();
-        float m1 = INFINITY, m2 = INFINITY;
-        int mt = -1;
-        for (int t = 0; t < ntiles; ++t) {
-            const uint8_t *img = s_res + t * IMG;
-            const floatx16 acc = chain(img, bhi, blo);
-            const float *cst = reinterpret_cast<const float *>(img + MAT);
-            const float prev = m1;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int c0 = 8 * g + 4 * (lane >> 5);
-                const float4 nbv = *reinterpret_cast<const float4 *>(&cst[c0]);
-                const float nba[4] = {nbv.x, nbv.y, nbv.z, nbv.w};
-#pragma unroll
-                for (int h = 0; h < 4; ++h)
-                    track2(m1, m2, pack_elem(fmaf(-2.0f, acc[4 * g + h], nba[h]), 4 * g + h), ninf);
+        // ---- merge the half-waves (the same frames, other centers) and the waves ----
+        float *s_m1 = reinterpret_cast<float *>(s_buf), *s_m2 = s_m1 + NW * F;
+        int *s_ix = reinterpret_cast<int *>(s_m2 + NW * F);
+        auto merge = [&](float &a1, float &a2, int &ai, float o1, float o2, int oi) __attribute__((always_inline)) {
+            a2 = fminf(fminf(a2, o2), fmaxf(a1, o1));
+            if (o1 < a1 || (o1 == a1 && oi < ai)) {
+                a1 = o1;
+                ai = oi;
             }
-            mt = m1 != prev ? t : mt;
+        };
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            const int e = (int)(__float_as_uint(m1[b]) & 15u);
+            int ix = mt[b] >= 0 ? mt[b] * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3) : 0x7fffffff;
+            const float o1 = __shfl_xor(m1[b], 32, 64), o2 = __shfl_xor(m2[b], 32, 64);
+            const int oi = __shfl_xor(ix, 32, 64);
+            merge(m1[b], m2[b], ix, o1, o2, oi);
+            if (lane < 32) {
+                s_m1[wave * F + b * 32 + lane] = m1[b];
+                s_m2[wave * F + b * 32 + lane] = m2[b];
+                s_ix[wave * F + b * 32 + lane] = ix;
+            }
         }
-        decide_frame<false>(lane, frame, fvalid, m1, m2, mt, k, na, sa, CE, 0.0f, gref, bmax, cp.bn, labels, rl);
+        __syncthreads();
+        // ---- one thread per frame: its label, and whether it goes to the next
+        // pass.  d_j >= |a|^2 + m2 - E_max for j != best, with E_max from the
+        // largest norms of all centers, and d_best <= |a|^2 + m1 + E_best (both
+        // through the reference loop's relative rounding g).  Anything not
+        // finite (frames, centers, fp16 overflow) fails the comparison.
+        if (tid < F) {
+            float b1 = s_m1[tid], b2 = s_m2[tid];
+            int ix = s_ix[tid];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) merge(b1, b2, ix, s_m1[w * F + tid], s_m2[w * F + tid], s_ix[w * F + tid]);
+            const int64_t pos = f0 + tid;
+            const bool fvalid = pos < nf;
+            bool undecided = false;
+            float up = __uint_as_float(0x7fc00000u);
+            int64_t fr = pos;
+            if constexpr (PASS == PASS_FINE) fr = fvalid ? rl.listA[pos] : 0;
+            if (fvalid) {
+                undecided = true;
+                int lab = 0;
+                if (ix < k && b1 < 1e38f) {
+                    lab = ix;
+                    const float *cst = reinterpret_cast<const float *>(img + (int64_t)(ix >> 5) * IMG + MAT) + (ix & 31);
+                    const double un = COARSE ? (double)cp.sc16[1] : 1.0;  // the coarse pass's values carry 2^2t
+                    const double na = s_na[tid], sa = sqrt(na) * (1.0 + 2e-5);
+                    const double e1 = sqrt((double)s_e1[tid]) * (1.0 + 1e-4) * (COARSE ? (double)cp.sc16[2] : 1.0);
+                    const double bb = cst[COARSE ? HC_BN : FC_BN], bd = cst[COARSE ? HC_D1 : FC_D1];
+                    const double mb = cp.mx[MX_BN], md = cp.mx[COARSE ? MX_D16 : MX_D1];
+                    double Rb, Rm;
+                    if constexpr (COARSE) {
+                        Rb = e1 * bb + (sa + e1) * bd;
+                        Rm = e1 * mb + (sa + e1) * md;
+                    } else {
+                        const double e2 = sqrt((double)s_e2[tid]) * (1.0 + 1e-4);
+                        Rb = e1 * bd + e2 * bb + (sa + e2) * (double)cst[FC_D2];
+                        Rm = e1 * md + e2 * mb + (sa + e2) * (double)cp.mx[MX_D2];
+                    }
+                    const double aa = (double)ce.c1a * sa * sa;
+                    const double Eb = aa + (double)ce.c1b * bb * bb + 2.0 * (double)ce.c2 * sa * bb + 2.02 * Rb;
+                    const double Em = aa + (double)ce.c1b * mb * mb + 2.0 * (double)ce.c2 * sa * mb + 2.02 * Rm;
+                    const double upper = (na + un * (double)b1 + Eb) * (1.0 + (double)ce.gref);
+                    const double lower = (na + un * (double)b2 - Em) * (1.0 - (double)ce.gref);
+                    undecided = !(lower > upper);
+                    if (fabs(upper) < 3e38) up = f32_round_up(upper);
+                }
+                labels[fr] = lab;
+            }
+            const unsigned long long um = __ballot(undecided);
+            if constexpr (FB == 1) {
+                // few frames: appended here, one list reservation per wave
+                if (um) {
+                    const int leader = __builtin_ctzll(um);
+                    unsigned long long base = 0;
+                    if (lane == leader)
+                        base = atomicAdd((unsigned long long *)(rl.count + (COARSE ? 3 : 0)), (unsigned long long)__popcll(um));
+                    base = __shfl(base, leader, 64);
+                    if (undecided) {
+                        const int64_t q = (int64_t)base + __popcll(um & ((1ull << lane) - 1ull));
+                        if constexpr (COARSE) {
+                            rl.listA[q] = fr;
+                        } else {
+                            rl.list[q] = fr;
+                            rl.upper[q] = up;
+                            rl.ccnt[q] = 0;
+                        }
+                    }
+                }
+            } else {
+                // otherwise one bit per position, made into the list by k_compact:
+                // the waves' reservations would all go to one address, about 29 ns
+                // each (10^7 frames x 32, k = 1000: 4.6 ms of reservations around
+                // 1.6 ms of work)
+                if (undecided && !COARSE) rl.upper_at[pos] = up;
+                if (lane == 0) rl.mask[pos >> 5] = (uint32_t)um;
+                if (lane == 32) rl.mask[pos >> 5] = (uint32_t)(um >> 32);
+            }
+        }
+        __syncthreads();  // the merge buffers and norms are consumed before the next frames overwrite them
     }
-}
-
-// Coefficients (c1, c2) = CE of the per-candidate bound
-//   E_j = c1 (|a|^2 + |b_j|^2) + 2 c2 |a| |b_j|   >=   |d~_j - d_j|,
-// with u = 2^-24, gamma_n = n u / (1 - n u):
-//   shift rounding of a and b:            2.1 u (|a|+|b|)^2
-//   final combination and fmaf rounding:  2.1 u (|a|+|b|)^2
-//   element index in the low mantissa bits: 32 u (|a|+|b|)^2
-//   FP32 norms |a|^2, |b|^2:              gamma_d (|a|^2 + |b|^2)
-//   omitted bf16 split terms:             3.1 * 2^-16 * 2 sum|a_i b_i|
-//   FP32 MFMA accumulation of 3 d_pad terms (each addition rounded to
-//   nearest, as the device probe of the matrix core shows):
-//                                         1.02 gamma_{3 d_pad} * 2 sum|a_i b_i|
-// using (|a|+|b|)^2 = |a|^2 + |b|^2 + 2|a||b| and sum|a_i b_i| <= |a||b|, so
-// the product terms are charged on 2|a||b| only.  A 25 % margin covers the
-// rounding of the FP32 bound arithmetic itself.
-static float2 assign_error_coeffs(int d, int d_pad) {
-    const double u = ldexp(1.0, -24);
-    auto gam = [&](double m) { return m * u / (1.0 - m * u); };
-    // + 32 u: the epilogue keeps an element index in the 4 low mantissa bits
-    // of d~ - |a|^2 (|d~ - |a|^2| <= (|a|+|b|)^2), a relative change < 2^-19
-    const double c0 = 4.2 * u + 32.0 * u;
-    float2 ce;
-    ce.x = (float)(1.25 * (c0 + gam(d)));
-    ce.y = (float)(1.25 * (c0 + 3.1 * ldexp(1.0, -16) + 1.02 * gam(3.0 * d_pad)));
-    return ce;
-}
-
-// The coarse pass: one fp16 product of ah = fp16(2^t a) and bh = fp16(2^t b)
-// per dimension.  Normal fp16 values carry a relative rounding <= 2^-11
-// (|ah bh - 2^2t a_i b_i| <= (2^-10 + 2^-22) 2^2t |a_i b_i|), the FP32 MFMA
-// accumulation of d_pad exact products adds 1.01 gamma_{d_pad}; the norms and
-// the other terms are those of the fine bound (c1 unchanged).  Underflow to
-// fp16 subnormals is the absolute term c3 (|a| + |b_j|) of k_center_scale16.
-static float2 assign_error_coeffs_coarse(int d, int d_pad) {
-    const double u = ldexp(1.0, -24);
-    auto gam = [&](double m) { return m * u / (1.0 - m * u); };
-    const double c0 = 4.2 * u + 32.0 * u;
-    float2 ce;
-    ce.x = (float)(1.25 * (c0 + gam(d)));
-    ce.y = (float)(1.25 * (c0 + ldexp(1.0, -10) + ldexp(1.0, -22) + 1.01 * gam(d_pad)));
-    return ce;
-}
-
-static double gamma_ref(int d) {
-    const double u = ldexp(1.0, -24);
-    const double m = d + 2;
-    return 1.25 * m * u / (1.0 - m * u);
 }
 
 static int pick_ksteps(int d) {
@@ -1124,15 +928,16 @@ static AssignWs carve_assign(void *ws, int64_t n, int d, int k, int mode) {
     AssignWs w{};
     Carver cv(ws);
     const size_t nl = n > 0 ? (size_t)n : 1;
-    // list length, bits of max |b_j|, list2 length, listA length (zeroed per call)
-    w.rl.count = cv.take<int64_t>(8);
+    w.rl.count = cv.take<int64_t>(N_COUNTS);
     w.rl.list = cv.take<int64_t>(nl);
-    w.cp.bmax = w.rl.count ? reinterpret_cast<float *>(w.rl.count + 1) : nullptr;
+    w.cp.mx = w.rl.count ? reinterpret_cast<float *>(w.rl.count + 4) : nullptr;
     if (mode == EMMA_ASSIGN_BF16X3_RECHECK) {
         w.rl.slots = cand_slots(n);
         w.rl.upper = cv.take<float>(nl);
         w.rl.ccnt = cv.take<int32_t>((size_t)w.rl.slots);
         w.rl.cand = cv.take<int32_t>((size_t)w.rl.slots * CAND_MAX);
+        w.rl.upper_at = reinterpret_cast<float *>(w.rl.cand);
+        w.rl.mask = w.rl.cand ? reinterpret_cast<uint32_t *>(w.rl.cand) + nl : nullptr;
         // listA is consumed by the fine pass before the candidate recheck
         // writes list2: one buffer serves both
         w.rl.listA = cv.take<int64_t>(nl);
@@ -1142,7 +947,7 @@ static AssignWs carve_assign(void *ws, int64_t n, int d, int k, int mode) {
         const int k_pad = (int)cdiv(k, 32) * 32;
         w.cp.img = cv.take<uint8_t>((size_t)(k_pad / 32) * tile_img_bytes(d_pad));
         w.cp.img16 = cv.take<uint8_t>((size_t)(k_pad / 32) * tile_img16_bytes(d_pad));
-        w.cp.bn = cv.take<float>(k_pad);
+        (void)cv.take<float>(k_pad);
         w.cp.mu = cv.take<float>(d_pad);
         w.cp.sc16 = cv.take<float>(4);
     }
@@ -1214,36 +1019,13 @@ __global__ __launch_bounds__(256) void k_assign_cand_exact(const float *__restri
     }
 }
 
-// Tile variants of the MFMA kernel for each K-step count: every variant fits
-// the registers and the LDS tile buffers of its occupancy.  Several 32-frame
-// blocks per wave (small d, where the fragments of a block take few
-// registers) reuse each center fragment for more MFMAs and hide a tile's
-// copies behind more work.  Variant 0 is the default; for K steps <= 8 and
-// k small enough that every tile image fits in LDS it runs the
-// resident-center kernel instead.  The autotuner (emma_assign_select) may
-// pick another per (K steps, k) bucket.
-// (waves per workgroup, workgroups per CU, 32-frame blocks per wave)
-struct Variant {
-    int nw, minb, fb;
-};
-static const Variant kVarSmall[] = {{4, 2, 1}, {8, 1, 1}, {16, 1, 1}, {4, 2, 2}, {8, 1, 2}, {4, 1, 4}};  // KSTEPS <= 4
-static const Variant kVarK8[] = {{4, 2, 1}, {8, 1, 1}, {4, 1, 2}};                                      // KSTEPS = 8
-static const Variant kVarMid[] = {{4, 2, 1}, {8, 1, 1}};                                              // 12 .. 19
-static const Variant kVarLarge[] = {{4, 1, 1}};                                                       // 24, 32
-
-static int n_shapes(int ks) {
-    if (ks <= 4) return (int)(sizeof(kVarSmall) / sizeof(Variant));
-    if (ks <= 8) return (int)(sizeof(kVarK8) / sizeof(Variant));
-    if (ks <= 19) return (int)(sizeof(kVarMid) / sizeof(Variant));
-    return (int)(sizeof(kVarLarge) / sizeof(Variant));
-}
-// variants 0 .. n_shapes - 1: the coarse pass in tile shape v (variant 0 of a
-// small K-step count: the resident fine kernel where its images fit);
-// n_shapes .. 2 n_shapes - 1: the fine pass over every frame in tile shape
-// v - n_shapes.  Which pipeline is faster depends on d, k and the data (how
-// many frames the coarse bound leaves to the fine pass), so the autotuner
-// times both.
-static int n_variants(int ks) { return 2 * n_shapes(ks); }
+// First-pass pipelines, timed by the autotuner (emma_assign_select may pick one
+// per (K steps, k) bucket): variant 0, the default, is the coarse pass over
+// every frame with the fine pass on what it leaves; variant 1 the fine pass
+// over every frame.  Which is faster depends on d, k and the data: the coarse
+// pass costs a third of the fine one's products, so it loses only where its
+// bound leaves about two thirds of the frames or more.
+static int n_variants(int) { return 2; }
 
 // process-wide selection table: [K-step class][ceil(log2(k_pad / 32))]
 static std::mutex g_sel_mu;
@@ -1268,43 +1050,6 @@ static int selected_variant(int ks, int k_pad) {
     return v < n_variants(ks) ? v : 0;
 }
 
-// pass 1 over every frame (PASS_COARSE or PASS_FULL), tile shape (NW, MINB, FB)
-template <int KS, int PASS, int NW, int MINB, int FB = 1>
-static void launch_v(const float *X, int64_t n, int d, const AssignWs &w, int k, int k_pad, float2 CE, float gref,
-                     int32_t *labels, const int32_t *done, hipStream_t s) {
-    const int64_t blocks = cdiv(n, 32 * NW * FB);
-    k_assign_mfma<KS, NW, MINB, FB, PASS><<<(unsigned)blocks, NW * 64, 0, s>>>(X, n, d, w.cp, k, k_pad, CE, gref,
-                                                                             labels, w.rl, done);
-}
-
-template <int KS, int PASS>
-static void launch_shape(int v, const float *X, int64_t n, int d, const AssignWs &w, int k, int k_pad, float2 CE,
-                         float gref, int32_t *labels, const int32_t *done, hipStream_t s) {
-    if constexpr (KS <= 4) {
-        switch (v) {
-            case 1: launch_v<KS, PASS, 8, 1>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-            case 2: launch_v<KS, PASS, 16, 1>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-            case 3: launch_v<KS, PASS, 4, 2, 2>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-            case 4: launch_v<KS, PASS, 8, 1, 2>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-            case 5: launch_v<KS, PASS, 4, 1, 4>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-            default: launch_v<KS, PASS, 4, 2>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-        }
-    } else if constexpr (KS <= 8) {
-        switch (v) {
-            case 1: launch_v<KS, PASS, 8, 1>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-            case 2: launch_v<KS, PASS, 4, 1, 2>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-            default: launch_v<KS, PASS, 4, 2>(X, n, d, w, k, k_pad, CE, gref, labels, done, s); return;
-        }
-    } else if constexpr (KS <= 19) {
-        if (v == 1)
-            launch_v<KS, PASS, 8, 1>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-        else
-            launch_v<KS, PASS, 4, 2>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-    } else {
-        launch_v<KS, PASS, 4, 1>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-    }
-}
-
 static int device_cus() {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -1313,41 +1058,109 @@ static int device_cus() {
     return cus;
 }
 
-// pass 1: variant 0 of a small K-step count with every bf16 tile image
-// resident in LDS is the resident kernel with the fine bound (it lists to the
-// fine pass's output directly, listA stays empty); every other variant is the
-// coarse streaming pass
-template <int KS>
-static void launch_mfma_ks(const float *X, int64_t n, int d, const AssignWs &w, int k, int k_pad, float2 CE,
-                           float2 CEc, float gref, int32_t *labels, const int32_t *done, hipStream_t s) {
-    const int v = selected_variant(KS, k_pad);
-    if constexpr (KS <= 8) {
-        if (v == 0 && k_pad / 32 <= res_max_tiles(KS * 16)) {
-            constexpr int NW = KS <= 4 ? 8 : 4;  // 8 K-steps: 4 waves, the registers of one wave per SIMD
-            int64_t blocks = cdiv(n, 32 * NW);
-            const int64_t cap = device_cus();
-            if (blocks > cap) blocks = cap;
-            k_assign_res<KS, NW><<<(unsigned)blocks, NW * 64, 0, s>>>(X, n, d, w.cp, k, k_pad, CE, gref, labels,
-                                                                    w.rl, done);
-            return;
+// List of a pass's undecided positions from its bit mask.  A workgroup takes
+// 1024 words (32768 positions) at a time and reserves their list range with one
+// atomic.  FINE: the positions are those of listA (or frames, LISTED = false)
+// and go to `list` with their upper bounds; otherwise frames to listA.
+template <bool FINE, bool LISTED>
+__global__ __launch_bounds__(256) void k_compact(int64_t n, RecheckLists rl, const int32_t *__restrict__ done) {
+    if (done && *done) return;
+    __shared__ uint32_t s_wave[4];
+    __shared__ unsigned long long s_base;
+    const int64_t np = LISTED ? rl.count[3] : n;
+    const int64_t words = (np + 31) >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int64_t w0 = (int64_t)blockIdx.x * 1024; w0 < words; w0 += (int64_t)gridDim.x * 1024) {
+        uint32_t m[4];
+        uint32_t cnt = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t w = w0 + tid * 4 + q;
+            m[q] = w < words ? rl.mask[w] : 0u;
+            cnt += __popc(m[q]);
         }
+        uint32_t pre = cnt;  // inclusive scan over the wave
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(pre, off, 64);
+            if (lane >= off) pre += o;
+        }
+        if (lane == 63) s_wave[wave] = pre;
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned long long tot = (unsigned long long)s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+            s_base = tot ? atomicAdd((unsigned long long *)(rl.count + (FINE ? 0 : 3)), tot) : 0ull;
+        }
+        __syncthreads();
+        int64_t q0 = (int64_t)s_base + pre - cnt;
+        for (int w = 0; w < wave; ++w) q0 += s_wave[w];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            uint32_t b = m[q];
+            while (b) {
+                const int64_t pos = (w0 + tid * 4 + q) * 32 + __builtin_ctz(b);
+                b &= b - 1;
+                if constexpr (FINE) {
+                    rl.list[q0] = LISTED ? rl.listA[pos] : pos;
+                    rl.upper[q0] = rl.upper_at[pos];
+                    rl.ccnt[q0] = 0;
+                } else {
+                    rl.listA[q0] = pos;
+                }
+                ++q0;
+            }
+        }
+        __syncthreads();  // s_wave and s_base are consumed
     }
-    const int ns = n_shapes(KS);
-    if (v < ns)
-        launch_shape<KS, PASS_COARSE>(v, X, n, d, w, k, k_pad, CEc, gref, labels, done, s);
-    else
-        launch_shape<KS, PASS_FULL>(v - ns, X, n, d, w, k, k_pad, CE, gref, labels, done, s);
 }
 
-// the fine pass over listA and the candidate pass over the fine pass's list:
-// grids for the most frames the lists can hold, blocks past a list's end exit
+struct TileArgs {
+    const float *X;
+    int64_t n;
+    int d, k, k_pad;
+    int32_t *labels;
+    const int32_t *done;
+    int cus;
+    hipStream_t s;
+};
+
+template <int KS, int FB, int CT, int NW, int PASS>
+static void launch_tile(const TileArgs &a, const AssignWs &w, const AsgCoef &ce) {
+    int64_t blocks = cdiv(PASS == PASS_CAND ? w.rl.slots : a.n, 32 * FB);
+    // a listed pass does not know its list's length here: a resident grid walks it
+    const int64_t cap = (int64_t)a.cus * (NW == 4 ? 2 : 1);
+    if ((PASS == PASS_FINE || PASS == PASS_CAND) && blocks > cap) blocks = cap;
+    k_assign_tile<KS, FB, CT, NW, PASS><<<(unsigned)blocks, NW * 64, 0, a.s>>>(a.X, a.n, a.d, w.cp, a.k, a.k_pad, ce,
+                                                                               a.labels, w.rl, a.done);
+}
+
+// Tile shape of a pass: 128 (coarse) or 64 frames per workgroup, two center
+// tiles per wave step; two 4-wave workgroups per CU while the fragments of
+// both fit in LDS (d <= 304), one of 8 waves beyond.  Few frames (less than
+// one such workgroup per CU) are cut into workgroups of 32.
 template <int KS, int PASS>
-static void launch_list_ks(const float *X, int64_t n, int d, const AssignWs &w, int k, int k_pad, float2 CE,
-                           float gref, int32_t *labels, const int32_t *done, hipStream_t s) {
-    constexpr int NW = 4, MINB = KS <= 19 ? 2 : 1;
-    const int64_t blocks = cdiv(PASS == PASS_CAND ? w.rl.slots : n, 32 * NW);
-    k_assign_mfma<KS, NW, MINB, 1, PASS><<<(unsigned)blocks, NW * 64, 0, s>>>(X, n, d, w.cp, k, k_pad, CE, gref,
-                                                                            labels, w.rl, done);
+static void launch_pass(const TileArgs &a, const AssignWs &w, const AsgCoef &ce) {
+    constexpr int FB = PASS == PASS_COARSE ? 4 : 2, NW = KS <= 19 ? 4 : 8;
+    if (cdiv(a.n, 32 * FB) < a.cus) {
+        launch_tile<KS, 1, 1, 4, PASS>(a, w, ce);
+        return;
+    }
+    launch_tile<KS, FB, 2, NW, PASS>(a, w, ce);
+    if (PASS != PASS_CAND) {
+        const int64_t chunks = cdiv(a.n, 32768);
+        k_compact<PASS != PASS_COARSE, PASS == PASS_FINE><<<(unsigned)(chunks < 512 ? chunks : 512), 256, 0, a.s>>>(a.n, w.rl, a.done);
+    }
+}
+
+template <int KS>
+static void launch_mfma_ks(const TileArgs &a, const AssignWs &w, const AsgCoef &ce, const AsgCoef &ce16) {
+    if (selected_variant(KS, a.k_pad) == 0) {
+        launch_pass<KS, PASS_COARSE>(a, w, ce16);
+        launch_pass<KS, PASS_FINE>(a, w, ce);
+    } else {
+        launch_pass<KS, PASS_FULL>(a, w, ce);
+    }
+    launch_pass<KS, PASS_CAND>(a, w, ce);
 }
 
 }  // namespace asg
@@ -1360,74 +1173,32 @@ int assign_run(const float *X, int64_t n, int d, const float *C, int k, int32_t 
     using namespace asg;
     AssignWs w = carve_assign(workspace, n, d, k, mode);
     if (mode == EMMA_ASSIGN_FP32_PLAIN) {
-        k_assign_plain<<<(unsigned)cdiv(n, PF), 256, 0, s>>>(X, n, d, C, k, labels, nullptr, nullptr, done);
-        EMMA_TRY(check_launch("assign plain"));
-        if (n_rechecked) k_zero_i64n<<<1, 64, 0, s>>>(n_rechecked, 1);
+        k_assign_plain<<<(unsigned)cdiv(n, PF), 256, 0, s>>>(X, n, d, C, k, labels, nullptr, nullptr, n_rechecked,
+                                                             nullptr, done);
         return check_launch("assign plain");
     }
     const int ks = pick_ksteps(d);
     EMMA_REQUIRE(ks > 0, "emma_assign: d=%d exceeds the MFMA path limit (512)", d);
     const int d_pad = ks * 16;
     const int k_pad = (int)cdiv(k, 32) * 32;
-    const float2 CE = assign_error_coeffs(d, d_pad);
-    const float2 CEc = assign_error_coeffs_coarse(d, d_pad);
-    const float gref = (float)gamma_ref(d);
-    k_zero_i64n<<<1, 64, 0, s>>>(w.rl.count, 4);
-    k_zero_i32n<<<(unsigned)(cdiv(w.rl.slots, 256) < 1024 ? cdiv(w.rl.slots, 256) : 1024), 256, 0, s>>>(w.rl.ccnt,
-                                                                                                   w.rl.slots);
-    k_center_mean<<<(unsigned)cdiv(d_pad, 64), 256, 0, s>>>(C, k, d, d_pad, w.cp.mu);
-    k_center_pack<<<(unsigned)cdiv(k_pad, 4), 256, 0, s>>>(C, k, d, d_pad, k_pad, CE, w.cp);
-    k_center_scale16<<<1, 1, 0, s>>>(d, w.cp);
+    const AsgCoef ce = assign_coeffs(d, d_pad, 3), ce16 = assign_coeffs(d, d_pad, 1);
+    k_center_mean<<<(unsigned)cdiv(d_pad, 64), 64 * MU_WAVES, 0, s>>>(C, k, d, d_pad, w.cp.mu, w.rl.count);
+    k_center_pack<<<(unsigned)cdiv(k_pad, 4), 256, 0, s>>>(C, k, d, d_pad, k_pad, ce.c1b, w.cp);
     k_center_pack16<<<(unsigned)cdiv(k_pad, 4), 256, 0, s>>>(C, k, d, d_pad, k_pad, w.cp);
     EMMA_TRY(check_launch("assign center pack"));
+    // the first pass over every frame, then the passes over what it leaves: the
+    // fine pass, the candidates of the frames that one leaves, the reference
+    // loop over them, the full loop over every center for the rest
+    const TileArgs a = {X, n, d, k, k_pad, labels, done, device_cus(), s};
     switch (ks) {
-        case 2: launch_mfma_ks<2>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-        case 4: launch_mfma_ks<4>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-        case 8: launch_mfma_ks<8>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-        case 12: launch_mfma_ks<12>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-        case 16: launch_mfma_ks<16>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-        case 19: launch_mfma_ks<19>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-        case 24: launch_mfma_ks<24>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-        case 32: launch_mfma_ks<32>(X, n, d, w, k, k_pad, CE, CEc, gref, labels, done, s); break;
-    }
-    EMMA_TRY(check_launch("assign mfma"));
-    // the frames the coarse pass left: the fine pass (bf16 x 3), then the
-    // recheck of those it leaves: candidates by the MFMA kernel, the
-    // reference loop over them, the full loop over every center for the rest;
-    // the grids cover the device, the kernels read the list lengths themselves
-    switch (ks) {
-        case 2:
-            launch_list_ks<2, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<2, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
-        case 4:
-            launch_list_ks<4, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<4, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
-        case 8:
-            launch_list_ks<8, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<8, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
-        case 12:
-            launch_list_ks<12, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<12, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
-        case 16:
-            launch_list_ks<16, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<16, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
-        case 19:
-            launch_list_ks<19, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<19, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
-        case 24:
-            launch_list_ks<24, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<24, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
-        case 32:
-            launch_list_ks<32, PASS_FINE>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            launch_list_ks<32, PASS_CAND>(X, n, d, w, k, k_pad, CE, gref, labels, done, s);
-            break;
+        case 2: launch_mfma_ks<2>(a, w, ce, ce16); break;
+        case 4: launch_mfma_ks<4>(a, w, ce, ce16); break;
+        case 8: launch_mfma_ks<8>(a, w, ce, ce16); break;
+        case 12: launch_mfma_ks<12>(a, w, ce, ce16); break;
+        case 16: launch_mfma_ks<16>(a, w, ce, ce16); break;
+        case 19: launch_mfma_ks<19>(a, w, ce, ce16); break;
+        case 24: launch_mfma_ks<24>(a, w, ce, ce16); break;
+        case 32: launch_mfma_ks<32>(a, w, ce, ce16); break;
     }
     EMMA_TRY(check_launch("assign candidates"));
     const int64_t eb = cdiv(n * CAND_MAX, 256) < 4096 ? cdiv(n * CAND_MAX, 256) : 4096;
@@ -1437,11 +1208,10 @@ int assign_run(const float *X, int64_t n, int d, const float *C, int k, int32_t 
     else
         k_assign_cand_exact<false><<<(unsigned)eb, 256, 0, s>>>(X, d, C, labels, w.rl, done);
     EMMA_TRY(check_launch("assign candidate recheck"));
-    const int64_t rb = cdiv(n, PF) < 2048 ? cdiv(n, PF) : 2048;
-    k_assign_plain<<<(unsigned)rb, 256, 0, s>>>(X, n, d, C, k, labels, w.rl.list2, w.rl.count + 2, done);
-    EMMA_TRY(check_launch("assign recheck"));
-    if (n_rechecked) k_copy_i64<<<1, 1, 0, s>>>(n_rechecked, w.rl.count);
-    return check_launch("assign copy count");
+    const int64_t rb = cdiv(n, PF) < 1024 ? cdiv(n, PF) : 1024;
+    k_assign_plain<<<(unsigned)rb, 256, 0, s>>>(X, n, d, C, k, labels, w.rl.list2, w.rl.count + 2, n_rechecked,
+                                                w.rl.count, done);
+    return check_launch("assign recheck");
 }
 
 }  // namespace emma

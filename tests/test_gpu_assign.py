@@ -221,3 +221,27 @@ def test_coarse_pass_edge_cases(d, case):
     ref = on.assign(X, C, nthreads=4)
     for v, lab in enumerate(_every_variant(X, C)):
         np.testing.assert_array_equal(lab, ref, err_msg="variant %d" % v)
+
+
+@pytest.mark.parametrize("n", [1, 31, 33, 129, 16383, 16385, 32767, 32769])
+@pytest.mark.parametrize("d,k", [(1, 31), (3, 65), (4, 1), (5, 32), (33, 33), (63, 129), (129, 64), (191, 97), (257, 63),
+                                 (303, 130), (305, 34), (383, 66), (385, 255), (511, 65)])
+def test_tile_edges(n, d, k):
+    """Labels at the edges of the tile kernel: one frame more or less than a row block and than
+    the frame counts where the small and the large workgroup shape take over, dimensions
+    around the K-step sizes (d < 4, d % 4 != 0, one past a size), center counts around one
+    and two tiles per wave.  Every variant gives the plain loop's labels."""
+    t = _native.torch()
+    g = t.Generator(device="cuda").manual_seed(1000 * d + k + n)
+    means = 2.0 * t.randn((7, d), generator=g, device="cuda")
+    X = (means[t.randint(0, 7, (n,), generator=g, device="cuda")] + t.randn((n, d), generator=g, device="cuda")).contiguous()
+    C = (X[t.randint(0, n, (k,), generator=g, device="cuda")] + 0.3 * t.randn((k, d), generator=g, device="cuda")).contiguous()
+    ref = _native.assign(X, C, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
+    L = _native.lib()
+    try:
+        for v in range(L.emma_assign_variants(d)):
+            _native.check(L.emma_assign_select(d, k, v), "emma_assign_select")
+            lab = _native.assign(X, C, mode=_native.EMMA_ASSIGN_BF16X3_RECHECK)
+            assert t.equal(lab, ref), "variant %d: %d labels differ" % (v, int((lab != ref).sum()))
+    finally:
+        _native.check(L.emma_assign_select(d, k, -1), "emma_assign_select")
