@@ -481,8 +481,6 @@ constexpr int PASS_COARSE = 0, PASS_FINE = 1, PASS_CAND = 2, PASS_FULL = 3;
 // smallest d that a kernel of KS K-steps sees (pick_ksteps takes the next size above d / 16)
 constexpr int min_dim(int ks) { return (ks == 2 ? 0 : ks == 4 ? 2 : ks == 8 ? 4 : ks == 12 ? 8 : ks == 16 ? 12 : ks == 19 ? 16 : ks == 24 ? 19 : 24) * 16 + 1; }
 
-typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte load, 4-byte aligned
-
 template <int KS, int FB, int CT, int NW, int PASS>
 __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restrict__ X, int64_t n, int d,
                                                             CenterPack cp, int k, int k_pad, AsgCoef ce,

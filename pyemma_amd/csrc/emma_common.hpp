@@ -98,6 +98,8 @@ __device__ __forceinline__ void static_for(F &&f) {
     }
 }
 
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte load, 4-byte aligned
+
 // 64-lane butterfly sum (every lane ends with the same value).
 __device__ __forceinline__ double wave_butterfly_sum(double v) {
 #pragma unroll

@@ -63,6 +63,8 @@ struct Params {
     int rev;              // reversible
     int ctt;              // compute Y'Y in NR_SYM tasks
     int has_xy;           // non-reversible XY tasks present
+    int tri;              // column groups of k_tri (0: the other kernels)
+    int n_sub;            // k_tri: workgroups (of one span) per slice, counted in n_slices
     // workspace
     int64_t *P_total;     // [1]
     int64_t *pair_off;    // [ntraj + 1]
@@ -1084,6 +1086,498 @@ __global__ __launch_bounds__(RNT) void k_rev_bf16(Params p) {
 }
 
 // ------------------------------------------------------------------
+// reversible moments up to d = 320: column groups of 64, one matrix per wave
+// ------------------------------------------------------------------
+// UU and VV are cut into 64 x 64 blocks on and above the diagonal; every one of
+// a workgroup's 8 waves owns one block of one matrix (or, where a task has fewer
+// blocks, subtiles of a block), and a task stages only the operand
+// "units" (U or V of one column group) that its blocks need.  At d = 300 that
+// is 4 tasks with 30 of 32 waves at work and every operand split 3.6 times per
+// pair, against 6 tasks of 128 x 128 tiles with 30 of 48 and 7.7 times.
+//
+// Stages of SP pairs.  A loader lane owns 4 adjacent columns and 8 consecutive
+// pairs (16 lanes a unit's 64 columns): 16 loads of 16 bytes, and per column the
+// 8 pairs' bf16 hi and lo as one 16-byte LDS write each, directly in operand
+// fragment order (1 KB per 32 columns and 16 pairs, so that an operand read is
+// contiguous and free of bank conflicts).  The rows of a stage's pairs are a
+// table of addresses in LDS, built a stage ahead; pairs past the slice point at
+// the shift vector for x and y, so that U = V = 0.  Columns past d repeat the
+// last four of the row and are never read back (tri_pos).
+//
+// While the waves run the MFMAs of stage s from one LDS buffer, stage s + 1 is
+// split from registers into the other, in the first half K-steps (two products
+// each), and the loads of stage s + 2 follow at once; one barrier per stage.
+// Two-level accumulation: a sub-span of 64 pairs starts from zero accumulators and
+// is added in FP32 into the span sum, which goes to the workgroup's
+// FP64 slot every 4096 pairs; sub-spans, spans, slices and the order of the
+// products are those of k_rev_bf16, so that the sums round alike to the last bit.
+//
+// What bounds it at d = 300: the frames' way through L1 (x and y of 18 units,
+// 92 GB per 10^7 pairs) and the split's vector work, beside the matrix cores (40 %
+// busy at 1.9 GHz).  A timing copy without the loads takes 9.5 ms instead of 11.5.
+// The loads must be started early in a stage (right after the split: a column per
+// half K-step instead of two, the loads three halves later, takes 14.6 ms; at 2
+// groups 2.51 against 2.59 ms, hence PPH), and nothing may spill inside the loop: a
+// scratch reload waits for every frame load before it.  Measured, whole call, 10^7
+// frames, against the 128 x 128 tiles: d = 30 1.46 -> 1.01 ms, d = 64 1.54 -> 1.11,
+// d = 128 2.58 -> 2.52, d = 192 6.9 -> 4.8, d = 256 9.0 -> 8.2, d = 300 15.0 -> 12.2,
+// d = 320 (9.4 10^6 frames) 13.8 -> 12.2.
+constexpr int TRI_UB = 4096;  // LDS bytes of a unit's 16 pairs: hi, lo x 2 column blocks x 1 KB
+
+struct TriTask {
+    int nu;          // units: kind 0 U, 1 V, and column group
+    int kind[5], grp[5];
+    int nb;          // blocks: row and column unit
+    int r[8], c[8];
+};
+template <int NG>
+struct Tri;
+template <>
+struct Tri<1> {
+    static constexpr int NU = 2, NO = 16, NT = 1;
+    static constexpr TriTask T[NT] = {{2, {0, 1}, {0, 0}, 2, {0, 1}, {0, 1}}};
+};
+template <>
+struct Tri<2> {
+    static constexpr int NU = 4, NO = 8, NT = 1;
+    static constexpr TriTask T[NT] = {{4, {0, 0, 1, 1}, {0, 1, 0, 1}, 6, {0, 0, 1, 2, 2, 3}, {0, 1, 1, 2, 3, 3}}};
+};
+template <>
+struct Tri<3> {
+    static constexpr int NU = 3, NO = 8, NT = 2;
+    static constexpr TriTask T[NT] = {{3, {0, 0, 0}, {0, 1, 2}, 6, {0, 0, 0, 1, 1, 2}, {0, 1, 2, 1, 2, 2}},
+                                      {3, {1, 1, 1}, {0, 1, 2}, 6, {0, 0, 0, 1, 1, 2}, {0, 1, 2, 1, 2, 2}}};
+};
+template <>
+struct Tri<4> {
+    static constexpr int NU = 4, NO = 8, NT = 3;
+    static constexpr TriTask T[NT] = {
+        {4, {0, 0, 0, 0}, {0, 1, 2, 3}, 8, {0, 0, 0, 0, 1, 1, 1, 2}, {0, 1, 2, 3, 1, 2, 3, 2}},
+        {4, {1, 1, 1, 1}, {0, 1, 2, 3}, 8, {0, 0, 0, 0, 1, 1, 1, 2}, {0, 1, 2, 3, 1, 2, 3, 2}},
+        {4, {0, 0, 1, 1}, {2, 3, 2, 3}, 4, {0, 1, 2, 3}, {1, 1, 3, 3}}};
+};
+template <>
+struct Tri<5> {
+    static constexpr int NU = 5, NO = 6, NT = 4;
+    static constexpr TriTask T[NT] = {
+        {5, {0, 0, 0, 0, 0}, {0, 1, 2, 3, 4}, 8, {0, 0, 0, 0, 0, 1, 1, 1}, {0, 1, 2, 3, 4, 1, 2, 3}},
+        {5, {1, 1, 1, 1, 1}, {0, 1, 2, 3, 4}, 8, {0, 0, 0, 0, 0, 1, 1, 1}, {0, 1, 2, 3, 4, 1, 2, 3}},
+        {4, {0, 0, 0, 0}, {1, 2, 3, 4}, 7, {0, 1, 1, 1, 2, 2, 3}, {3, 1, 2, 3, 2, 3, 3}},
+        {4, {1, 1, 1, 1}, {1, 2, 3, 4}, 7, {0, 1, 1, 1, 2, 2, 3}, {3, 1, 2, 3, 2, 3, 3}}};
+};
+constexpr int TRI_MAX_D = 320;
+__host__ __device__ constexpr int tri_groups(int d) { return (d + 63) / 64; }
+// waves that share a block: 1, 2 (a row of 32 x 32 subtiles each) or 4 (a subtile each)
+__host__ __device__ constexpr int tri_share(int nb) { return nb > 4 ? 1 : nb > 2 ? 2 : 4; }
+
+// Place of column c among the staged columns: 4-column quads, the last of which
+// holds the row's last four columns (d >= 4; below, the one quad is the row).
+__host__ __device__ __forceinline__ int tri_pos(int c, int d) {
+    const int nq = (d + 3) / 4;
+    return (d < 4 || c < 4 * (nq - 1)) ? c : 4 * (nq - 1) + c - (d - 4);
+}
+// Operand row of staged column p (0..63) of a group: 32-column block and row in
+// it (quad q of a block and column j of the quad sit at row 8 (j ^ block) + q, so
+// that a loader's writes and the operand reads are free of bank conflicts).
+__host__ __device__ __forceinline__ int tri_row(int p) {
+    const int q = (p >> 2) & 7, cb = p >> 5;
+    return 8 * ((p & 3) ^ cb) + q;
+}
+
+template <int NG>
+__global__ __launch_bounds__(512, 2) void k_tri(Params p) {
+    using T = Tri<NG>;
+    constexpr int NU = T::NU, NO = T::NO, SP = NO * 8, NKS = SP / 16;
+    // a partial loader wave (5 groups: 30 of 32 slots) writes its idle lanes' share past the operands
+    constexpr int USED = NKS * NU * TRI_UB + (NU * NO % 4 ? TRI_UB : 0);
+    constexpr int BUF = 65536;  // buffer stride
+    static_assert(USED <= BUF, "a stage fits its buffer");
+    __shared__ __align__(16) uint8_t s_op[BUF + USED];
+    __shared__ __align__(16) uint64_t s_row[2][SP][2];  // addresses of the x and y rows of a stage's pairs
+    __shared__ double s_sum[NO][4][NG * 16];            // column sums of U (pair octet, column of a quad, quad), one lane per entry
+    __shared__ __align__(16) float s_k[NG * 64];        // the shift of every staged column
+
+    // XCD-aware numbering: the tasks of one slice side by side on one XCD, so
+    // that they share the frames through its L2
+    const int per_xcd = gridDim.x >> 3;
+    const int wg = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (wg >= T::NT * p.n_slices) return;
+    const int slice = wg / T::NT, task = wg - slice * T::NT;
+
+    // the pairs of this workgroup: a slice, or (few pairs) one span of a slice
+    const int64_t P = *p.P_total;
+    const int n_sl = p.n_slices / p.n_sub, sl = slice / p.n_sub;
+    const int64_t per = (P + n_sl - 1) / n_sl;
+    const int64_t per_r = (per + RBT - 1) / RBT * RBT;
+    int64_t p_lo = (int64_t)sl * per_r < P ? (int64_t)sl * per_r : P;
+    int64_t p_hi = p_lo + per_r < P ? p_lo + per_r : P;
+    if (p.n_sub > 1) {
+        const int c = slice - sl * p.n_sub;
+        p_lo = p_lo + (int64_t)c * RFLUSH_TL < p_hi ? p_lo + (int64_t)c * RFLUSH_TL : p_hi;
+        if (c + 1 < p.n_sub) p_hi = p_lo + RFLUSH_TL < p_hi ? p_lo + RFLUSH_TL : p_hi;
+    }
+    const int n_stages = (int)((p_hi - p_lo + SP - 1) / SP);
+    double *slot = p.slots + (int64_t)slice * p.slot_doubles + (int64_t)task * 8 * 4096;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // ---- roles (the task table, unrolled into selects) ----
+    int nu = 0, nb = 0, ra = 0, rb = 0, kind = 0, grp = 0;
+    const int s16 = wave * 4 + (lane >> 4);  // loader slot of 16 lanes: unit s16 / NO, pairs 8 (s16 % NO) ..
+    const int unit = s16 / NO, oct = s16 - unit * NO;
+    static_for<0, T::NT>([&](auto tc) __attribute__((always_inline)) {
+        constexpr int t = decltype(tc)::value;
+        if (task == t) {
+            nu = T::T[t].nu;
+            nb = T::T[t].nb;
+            const int b = wave % T::T[t].nb;
+            static_for<0, 8>([&](auto bc) __attribute__((always_inline)) {
+                constexpr int i = decltype(bc)::value;
+                if (b == i) {
+                    ra = T::T[t].r[i];
+                    rb = T::T[t].c[i];
+                }
+            });
+            static_for<0, NU>([&](auto uc) __attribute__((always_inline)) {
+                constexpr int i = decltype(uc)::value;
+                if (unit == i) {
+                    kind = T::T[t].kind[i];
+                    grp = T::T[t].grp[i];
+                }
+            });
+        }
+    });
+    const int share = tri_share(nb);
+    const int sub = wave / nb;              // which part of the block
+    const bool act = sub < share;           // this wave has matrix work
+    const bool ld_lane = unit < nu;        // this lane's unit exists
+    const bool ld_wave = wave * 4 < nu * NO;
+    const bool own = task == 0;            // the task whose U units give the column sums
+
+    // ---- loader: 4 columns from cs, pairs 8 oct .. ----
+    const int quad = lane & 15;
+    int cs = grp * 64 + quad * 4;
+    if (p.d >= 4) cs = cs + 4 <= p.d ? cs : p.d - 4; else cs = 0;
+    const uint64_t coff = (uint64_t)cs * 4;
+    // LDS place of the lane's fragments (buffer, plane and column j added)
+    const uint32_t wbase = (uint32_t)((ld_lane ? (oct >> 1) * NU + unit : NKS * NU) * TRI_UB + (quad >> 3) * 1024 +
+                                      (oct & 1) * 512 + (quad >> 3) * 128 + (quad & 7) * 16);
+
+    // ---- cursor: trajectory of the slice's next pair (scalar) ----
+    typedef const __attribute__((address_space(4))) int64_t *cptr;
+    const cptr poff_c = (cptr)p.pair_off;
+    const cptr toff_c = (cptr)p.traj_off;
+    PairCursor cur;
+    {
+        int lo = 0, hi = p.ntraj - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (p.pair_off[mid] <= p_lo) lo = mid; else hi = mid - 1;
+        }
+        cur.t = lo;
+        cur.p0 = p.pair_off[lo];
+        cur.p1 = p.pair_off[lo + 1];
+        cur.base = p.traj_off[lo] + p.skip;
+    }
+    const int64_t lag_b = (int64_t)p.lag * p.d * 4;
+    // row addresses of stage s (threads 0 .. SP - 1, one pair each)
+    auto build_rows = [&](int s) __attribute__((always_inline)) {
+        if (wave * 64 >= SP) return;
+        const int64_t q0 = p_lo + (int64_t)s * SP;
+        const int64_t q = q0 + tid;
+        const int64_t lim = q0 + SP < p_hi ? q0 + SP : p_hi;
+        uint64_t ax = (uint64_t)p.K, ay = (uint64_t)p.K;
+        while (q0 < p_hi) {
+            if (q >= cur.p0 && q < cur.p1 && q < lim) {
+                ax = (uint64_t)p.X + (uint64_t)((cur.base + (q - cur.p0) * p.stride) * p.d * 4);
+                ay = ax + lag_b;
+            }
+            if (cur.p1 >= lim) break;
+            ++cur.t;
+            cur.p0 = cur.p1;
+            cur.p1 = poff_c[cur.t + 1];
+            cur.base = toff_c[cur.t] + p.skip;
+        }
+        if (tid < SP) {
+            s_row[s & 1][tid][0] = ax;
+            s_row[s & 1][tid][1] = ay;
+        }
+    };
+
+    float4_u xr[8], yr[8];
+    auto issue = [&](int s) __attribute__((always_inline)) {
+        const uint64_t(*rt)[2] = &s_row[s & 1][oct * 8];
+        if (NG > 1 || p.d >= 4) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                xr[i] = *reinterpret_cast<const __attribute__((address_space(1))) float4_u *>(rt[i][0] + coff);
+                yr[i] = *reinterpret_cast<const __attribute__((address_space(1))) float4_u *>(rt[i][1] + coff);
+            }
+        } else {
+            for (int i = 0; i < 8; ++i) {
+                const float *x = reinterpret_cast<const float *>(rt[i][0]), *y = reinterpret_cast<const float *>(rt[i][1]);
+                const int c1 = p.d > 1 ? 1 : 0, c2 = p.d > 2 ? 2 : 0;
+                xr[i] = float4_u{x[0], x[c1], x[c2], 0.0f};
+                yr[i] = float4_u{y[0], y[c1], y[c2], 0.0f};
+            }
+        }
+    };
+    const int kpos = grp * 64 + quad * 4;
+    double *my_sum = &s_sum[oct][0][kpos >> 2];
+    // column j of the lane's quad: split into the buffer (KIND 0: U with its
+    // column sum, 1: U, 2: V; the same for all lanes of a wave)
+    auto piece = [&](auto kind_tag, uint32_t bo, int j) __attribute__((always_inline)) {
+        constexpr int KIND = decltype(kind_tag)::value;
+        const float kc = KIND == 2 ? 0.0f : s_k[kpos + j];
+        float u[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            u[i] = KIND == 2 ? __fsub_rn(xr[i][j], yr[i][j])
+                             : __fadd_rn(__fsub_rn(xr[i][j], kc), __fsub_rn(yr[i][j], kc));
+        if constexpr (KIND == 0)
+            if (ld_lane) unsafeAtomicAdd(my_sum + j * (NG * 16), (double)((u[0] + u[1]) + (u[2] + u[3])) + (double)((u[4] + u[5]) + (u[6] + u[7])));
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) split_bf16x2(u[2 * i], u[2 * i + 1], h[i], l[i]);
+        uint32_t wo = wbase ^ (uint32_t)(j * 128);  // bits 7, 8: column j of the quad, the block's bit exchanged
+        asm volatile("" : "+v"(wo));
+        uint8_t *dst = &s_op[wo + bo];
+        *reinterpret_cast<uint4 *>(dst) = make_uint4(h[0], h[1], h[2], h[3]);
+        *reinterpret_cast<uint4 *>(dst + 2048) = make_uint4(l[0], l[1], l[2], l[3]);
+    };
+
+    floatx16 acc[2][2], sacc[2][2];
+    // Operands of a K-step: row lo and hi, column lo, then hi (2 x 32 rows each).
+    // The products lo lo, hi lo, lo hi, hi hi need three operand pairs at a time,
+    // each read from LDS as soon as its registers are free; the other wave of the
+    // SIMD covers the reads' latency.
+    bf16x8 al[2], ah[2], b[2];
+    // share 2: row subtile sub; share 4: row subtile sub / 2, column subtile sub % 2
+    const uint32_t offa = (uint32_t)(ra * TRI_UB + lane * 16 + (share == 1 ? 0 : (share == 2 ? sub : sub >> 1) * 1024));
+    const uint32_t offb = (uint32_t)(rb * TRI_UB + lane * 16 + (share == 4 ? (sub & 1) * 1024 : 0));
+    double *mslot = slot + (int64_t)wave * 4096;
+    auto flush = [&](auto nr_tag, auto nc_tag, auto add_tag) __attribute__((always_inline)) {
+        constexpr int NR = decltype(nr_tag)::value, NC = decltype(nc_tag)::value;
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                char *base = reinterpret_cast<char *>(mslot + (r * NC + c) * 1024);
+                uint32_t loff = (uint32_t)lane * 8u;
+                asm volatile("" : "+v"(loff));  // recomputed per flush: keeps the addresses out of the loop
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    double *dst = reinterpret_cast<double *>(base + e * 512 + loff);
+                    // private slot, one writer lane per element: no atomicity needed;
+                    // the L2-side add keeps the old value out of registers
+                    if constexpr (decltype(add_tag)::value)
+                        unsafeAtomicAdd(dst, (double)sacc[r][c][e]);
+                    else
+                        *dst = (double)sacc[r][c][e];
+                }
+                sacc[r][c] = floatx16{};
+            }
+    };
+
+    // KIND < 0: no loader work; SH: waves that share a block
+    auto run = [&](auto act_tag, auto kind_tag, auto sh_tag) __attribute__((always_inline)) {
+        constexpr bool ACT = decltype(act_tag)::value;
+        constexpr int KIND = decltype(kind_tag)::value, SH = decltype(sh_tag)::value;
+        constexpr bool LD = KIND >= 0;
+        constexpr int NR = SH == 1 ? 2 : 1, NC = SH == 4 ? 1 : 2;  // 32 x 32 subtiles of this wave
+        typedef std::integral_constant<int, NR> NR_;
+        typedef std::integral_constant<int, NC> NC_;
+        typedef std::integral_constant<bool, false> N_;
+        typedef std::integral_constant<bool, true> Y_;
+        auto rd = [&](bf16x8 *dst, uint32_t off, int kk, int plane, auto n_tag) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < decltype(n_tag)::value; ++r)
+                dst[r] = *reinterpret_cast<const bf16x8 *>(&s_op[off + kk * (NU * TRI_UB) + plane * 2048 + r * 1024]);
+        };
+        auto prod = [&](const bf16x8 *a, auto z_tag) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    if (decltype(z_tag)::value)
+                        acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r], b[c], floatx16{}, 0, 0, 0);
+                    else
+                        acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r], b[c], acc[r][c], 0, 0, 0);
+                }
+        };
+        auto fold = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sacc[r][c][e] = __fadd_rn(sacc[r][c][e], acc[r][c][e]);
+        };
+        // A sub-span is 4 K-steps (64 pairs).  Stages of whole sub-spans start them
+        // from a zero accumulator operand; with 3 K-steps a stage (DYN) they are
+        // counted and the accumulators cleared.
+        constexpr bool DYN = NKS % 4 != 0;
+        // columns split per half K-step from the stage's start on; then the lane's
+        // registers take the loads of the stage after
+        constexpr int PPH = NG == 2 ? 1 : 2, IH = 4 / PPH;
+        // prologue: stage 0 split into buffer 0, stage 1 in registers
+        if constexpr (LD) {
+            issue(0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) piece(kind_tag, 0u, j);
+            __builtin_amdgcn_sched_barrier(0);
+            issue(1);
+        }
+        __syncthreads();  // tables 0 and 1 are consumed before 2 is written
+        build_rows(2);
+        __syncthreads();
+        if constexpr (ACT) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) acc[r][c] = sacc[r][c] = floatx16{};
+            rd(al, offa, 0, 1, NR_());
+            rd(b, offb, 0, 1, NC_());
+            rd(ah, offa, 0, 0, NR_());
+        }
+        const int n_run = n_stages > 0 ? n_stages : 1;
+        uint32_t bo = 0;  // byte offset of the stage's buffer
+        int kcount = 0;   // K-steps done (DYN)
+        for (int s = 0; s < n_run; ++s) {
+            const uint32_t nbo = bo ^ (uint32_t)BUF;
+            // half K-steps: two products and their share of the split
+            static_for<0, 2 * NKS>([&](auto hc) __attribute__((always_inline)) {
+                constexpr int h = decltype(hc)::value, k = h / 2;
+                constexpr bool last = k + 1 == NKS;
+                if constexpr (LD && h == IH) issue(s + 2);
+                if constexpr (last && h % 2 == 0) build_rows(s + 3);
+                // stage s + 1 is complete in its buffer and nothing reads this one any
+                // more; its first operands arrive beside the last products
+                if constexpr (last && h % 2 == 1) __syncthreads();
+                if constexpr (ACT && h % 2 == 0) {
+                    prod(al, std::integral_constant<bool, !DYN && k % 4 == 0>());
+                    prod(ah, N_());
+                    rd(b, offb + bo, k, 0, NC_());
+                }
+                if constexpr (ACT && h % 2 == 1) {
+                    const uint32_t o = last ? nbo : bo;
+                    constexpr int nk = last ? 0 : k + 1;
+                    prod(al, N_());
+                    rd(al, offa + o, nk, 1, NR_());
+                    prod(ah, N_());
+                    rd(b, offb + o, nk, 1, NC_());
+                    rd(ah, offa + o, nk, 0, NR_());
+                }
+                if constexpr (LD && h < IH) {
+#pragma unroll
+                    for (int j = h * PPH; j < (h + 1) * PPH; ++j) piece(kind_tag, nbo, j);
+                    if constexpr (ACT) {
+#pragma unroll
+                        for (int i = 0; i < 2 * NR * NC; ++i) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                               // 1 MFMA
+                            __builtin_amdgcn_sched_group_barrier(0x002, (8 * PPH - 1) * 4 / (NR * NC), 0);  // vector ALU
+                        }
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (ACT && h % 2 == 1) {
+                    if constexpr (DYN) {
+                        ++kcount;
+                        if ((kcount & 3) == 0) {
+                            fold();
+#pragma unroll
+                            for (int r = 0; r < NR; ++r)
+#pragma unroll
+                                for (int c = 0; c < NC; ++c) acc[r][c] = floatx16{};
+                            if (kcount % (RFLUSH_TL / 16) == 0) {
+                                if (kcount == RFLUSH_TL / 16)
+                                    flush(NR_(), NC_(), N_());
+                                else
+                                    flush(NR_(), NC_(), Y_());
+                            }
+                        }
+                    } else if constexpr (k % 4 == 3) {
+                        fold();
+                        if constexpr (last) {
+                            if ((s + 1) % (RFLUSH_TL / SP) == 0) {
+                                if (s < RFLUSH_TL / SP)
+                                    flush(NR_(), NC_(), N_());
+                                else
+                                    flush(NR_(), NC_(), Y_());
+                            }
+                        }
+                    }
+                }
+            });
+            bo = nbo;
+        }
+        if constexpr (ACT) {
+            const int kdone = n_run * NKS;
+            if (kdone % (RFLUSH_TL / 16)) {  // a started span (and, DYN, sub-span)
+                if constexpr (DYN) fold();
+                if (kdone < RFLUSH_TL / 16)
+                    flush(NR_(), NC_(), N_());
+                else
+                    flush(NR_(), NC_(), Y_());
+            }
+        }
+    };
+    if (own)
+        for (int i = tid; i < NO * NG * 64; i += 512) (&s_sum[0][0][0])[i] = 0.0;
+    for (int i = tid; i < NG * 64; i += 512) {
+        const int q0 = i & ~3, c0 = p.d >= 4 ? (q0 + 4 <= p.d ? q0 : p.d - 4) : 0, c = c0 + (i & 3);
+        s_k[i] = p.K[c < p.d ? c : p.d - 1];
+    }
+    build_rows(0);
+    build_rows(1);
+    __syncthreads();
+    typedef std::integral_constant<bool, true> Y_;
+    typedef std::integral_constant<bool, false> N_;
+    typedef std::integral_constant<int, 0> UO_;
+    typedef std::integral_constant<int, 1> U_;
+    typedef std::integral_constant<int, 2> V_;
+    typedef std::integral_constant<int, -1> I_;
+    typedef std::integral_constant<int, NG == 1 ? 4 : 1> S_;
+    // the kinds of waves that the task table has (a wave's loader lanes are of one kind)
+    const bool wu = __builtin_amdgcn_readfirstlane(kind) == 0;
+    if (act && ld_wave) {
+        if constexpr (NG == 4) {
+            typedef std::integral_constant<int, 2> S2_;
+            if (share == 2) {
+                if (wu) run(Y_(), U_(), S2_()); else run(Y_(), V_(), S2_());
+            } else if (own) {
+                run(Y_(), UO_(), S_());
+            } else {
+                run(Y_(), V_(), S_());
+            }
+        } else if (!wu) {
+            run(Y_(), V_(), S_());
+        } else if (own) {
+            run(Y_(), UO_(), S_());
+        } else if constexpr (NG == 5) {
+            run(Y_(), U_(), S_());
+        }
+    } else if (act) {
+        if constexpr (NG == 5) run(Y_(), I_(), S_());
+    } else if (ld_wave) {
+        if constexpr (NG == 2) run(N_(), V_(), S_());
+    } else {
+        if constexpr (NG == 3 || NG == 5) run(N_(), I_(), S_());
+    }
+
+    // ---- column sums of U, over the pair octets in order ----
+    if (own) {
+        double *out = p.slots + (int64_t)slice * p.slot_doubles + (int64_t)T::NT * 8 * 4096;
+        for (int c = tid; c < NG * 64; c += 512) {
+            double a = 0.0;
+            for (int o = 0; o < NO; ++o) a += s_sum[o][c & 3][c >> 2];
+            out[c] = a;
+        }
+    }
+}
+
+// ------------------------------------------------------------------
 // frame weights: sum of the weights of every trajectory's pairs, then the
 // total (both in a fixed order)
 // ------------------------------------------------------------------
@@ -1235,6 +1729,112 @@ __global__ __launch_bounds__(256) void k_reduce_mats(Params p, const double *Sx,
     }
 }
 
+// Sum over the slices (in order, four quarters) of the column sums of U: the
+// sums of x and y.  64 columns per workgroup, a quarter of the slices per wave.
+template <int NG>
+__global__ __launch_bounds__(256) void k_tri_sums(Params p, double *Sx, double *Sy, double *w_out, double *sx_out,
+                                                  double *sy_out) {
+    __shared__ double s_part[4][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int c = blockIdx.x * 64 + lane;
+    const int64_t P = *p.P_total;
+    const double w = 2.0 * (double)P;
+    if (c == 0 && wave == 0) *w_out = w;
+    const int n4 = (p.n_slices + 3) / 4, s0 = wave * n4, s1 = s0 + n4 < p.n_slices ? s0 + n4 : p.n_slices;
+    double a = 0.0;
+    if (c < p.d) {
+        const double *src = p.slots + (int64_t)Tri<NG>::NT * 8 * 4096 + tri_pos(c, p.d);
+#pragma unroll 8
+        for (int s = s0; s < s1; ++s) a += src[(int64_t)s * p.slot_doubles];
+    }
+    s_part[wave][lane] = a;
+    __syncthreads();
+    if (wave == 0 && c < p.d) {
+        const double S = (s_part[0][lane] + s_part[1][lane]) + (s_part[2][lane] + s_part[3][lane]);
+        Sx[c] = S;
+        Sy[c] = 0.0;
+        const double o = S + w * (double)p.K[c];
+        sx_out[c] = o;
+        if (sy_out) sy_out[c] = o;
+    }
+}
+
+// UU and VV from the slots, and the reversible moments with their corrections:
+// one workgroup per 64 consecutive elements of a 64 x 64 block (the same
+// elements of every slice are contiguous), a quarter of the slices per wave.
+template <int NG>
+__global__ __launch_bounds__(256) void k_tri_reduce(Params p, const double *Sx, int remove_mean, double *Mxx, double *Mxy) {
+    using T = Tri<NG>;
+    __shared__ double s_part[2][4][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int I = 0, rem = blockIdx.x >> 6;  // block (I, J) of the upper triangle of groups
+    while (rem >= NG - I) {
+        rem -= NG - I;
+        ++I;
+    }
+    const int J = I + rem;
+    const int pos = (blockIdx.x & 63) * 64 + lane;  // element of the block, in the order of the slots
+    double part[2] = {0.0, 0.0};
+    const int n4 = (p.n_slices + 3) / 4, s0 = wave * n4, s1 = s0 + n4 < p.n_slices ? s0 + n4 : p.n_slices;
+    static_for<0, T::NT>([&](auto tc) __attribute__((always_inline)) {
+        constexpr TriTask t = T::T[decltype(tc)::value];
+        constexpr int nb = t.nb, sh = tri_share(nb);
+        static_for<0, nb>([&](auto bc) __attribute__((always_inline)) {
+            constexpr int b = decltype(bc)::value, m = t.kind[t.r[b]];
+            if (t.grp[t.r[b]] == I && t.grp[t.c[b]] == J) {
+                // subtile pos >> 10 of the block: of the wave that owns it, its (pos >> 10) % (4 / sh)-th
+                const int st = pos >> 10, w = b + (st * sh / 4) * nb;
+                const double *src = p.slots + (int64_t)(decltype(tc)::value * 8 + w) * 4096 + (st % (4 / sh)) * 1024 + (pos & 1023);
+#pragma unroll 8
+                for (int s = s0; s < s1; ++s) part[m] += src[(int64_t)s * p.slot_doubles];
+            }
+        });
+    });
+    s_part[0][wave][lane] = part[0];
+    s_part[1][wave][lane] = part[1];
+    __syncthreads();
+    if (wave) return;
+    const double uu = (s_part[0][0][lane] + s_part[0][1][lane]) + (s_part[0][2][lane] + s_part[0][3][lane]);
+    const double vv = (s_part[1][0][lane] + s_part[1][1][lane]) + (s_part[1][2][lane] + s_part[1][3][lane]);
+    // matrix element of this slot position
+    const int e = (pos >> 6) & 15, r = (pos >> 11) & 1, cb = (pos >> 10) & 1;
+    const int si = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), sj = lane & 31;
+    const int d = p.d, nq = (d + 3) / 4;
+    auto column = [&](int g, int blk, int s) -> int {  // column of operand row s, -1: none of its own
+        const int pp = g * 64 + blk * 32 + (s & 7) * 4 + ((s >> 3) ^ blk), q = pp >> 2;
+        if (d < 4 || q < nq - 1) return pp < d ? pp : -1;
+        const int c = d - 4 + (pp & 3);
+        return q == nq - 1 && c >= 4 * (nq - 1) ? c : -1;
+    };
+    const int i = column(I, r, si), j = column(J, cb, sj);
+    if (i < 0 || j < 0 || i > j) return;
+    const int64_t ij = (int64_t)i * d + j, ji = (int64_t)j * d + i;
+    const int64_t P = *p.P_total;
+    double xx = 0.0, xy = 0.0;
+    if (P > 0) {
+        const double w = 2.0 * (double)P, Si = Sx[i], Sj = Sx[j], Ki = (double)p.K[i], Kj = (double)p.K[j];
+        const double corr = remove_mean ? -(Si * Sj) / w : (Si * Kj + Ki * Sj) + w * (Ki * Kj);
+        xx = 0.5 * (uu + vv) + corr;
+        xy = 0.5 * (uu - vv) + corr;
+    }
+    Mxx[ij] = xx;
+    Mxx[ji] = xx;
+    if (Mxy) {
+        Mxy[ij] = xy;
+        Mxy[ji] = xy;
+    }
+}
+
+template <int NG>
+static int launch_tri(const Params &p, double *Sx, double *Sy, int remove_mean, double *w, double *sx, double *sy,
+                      double *Mxx, double *Mxy, hipStream_t s) {
+    k_tri<NG><<<(unsigned)(cdiv((int64_t)Tri<NG>::NT * p.n_slices, 8) * 8), 512, 0, s>>>(p);
+    EMMA_TRY(check_launch("moments main"));
+    k_tri_sums<NG><<<NG, 256, 0, s>>>(p, Sx, Sy, w, sx, sy);
+    k_tri_reduce<NG><<<NG * (NG + 1) / 2 * 64, 256, 0, s>>>(p, Sx, remove_mean, Mxx, Mxy);
+    return check_launch("moments reduce");
+}
+
 template <int PREC, bool WT>
 static void launch_kind_w(const Params &p, hipStream_t s) {
     const int n_sym = p.n_sym;
@@ -1302,7 +1902,7 @@ struct Plan {
 };
 
 static void make_plan(Plan &pl, const float *X, int64_t n_rows, int d, const int64_t *traj_off, int ntraj,
-                      int lag, int stride, int skip, uint32_t flags, int precision, void *ws) {
+                      int lag, int stride, int skip, uint32_t flags, int precision, int acc2, void *ws) {
     Params &p = pl.p;
     p.X = X;
     p.n_rows = n_rows;
@@ -1312,7 +1912,8 @@ static void make_plan(Plan &pl, const float *X, int64_t n_rows, int d, const int
     p.lag = lag;
     p.stride = stride;
     p.skip = skip;
-    p.acc2 = 0;
+    p.acc2 = acc2;
+    p.n_sub = 1;
     p.tb = precision == EMMA_PREC_FP64 ? 64 : 128;
     p.frag = precision == EMMA_PREC_FP64 ? 0 : 1;
     p.slot_doubles = 2LL * p.tb * p.tb + 2LL * p.tb;
@@ -1323,7 +1924,19 @@ static void make_plan(Plan &pl, const float *X, int64_t n_rows, int d, const int
     p.has_xy = lag > 0 && !p.rev && (flags & EMMA_MOM_C0T) ? 1 : 0;
     p.n_tasks = p.n_sym + (p.has_xy ? p.nb * p.nb : 0);
     const bool weighted = (flags & EMMA_MOM_WEIGHTED) != 0;
-    if (precision == EMMA_PREC_BF16X4) {
+    // the column-group kernel where it is built and faster (see k_tri); weighted,
+    // non-reversible and wider moments and the single-level mode stay with k_rev_bf16
+    p.tri = precision == EMMA_PREC_BF16X4 && acc2 && p.rev && !weighted && d <= TRI_MAX_D ? tri_groups(d) : 0;
+    if (p.tri) {
+        // the slices of the 128 x 128 kernel (the same sums, to the last bit); with
+        // few of them, a workgroup per span
+        static const int nt[] = {1, 1, 2, 3, 4};
+        const int64_t cap = cdiv(n_rows > 0 ? n_rows : 1, 8192);
+        p.n_sub = cap < 256 ? 8192 / RFLUSH_TL : 1;
+        p.n_slices = (int)(cap < 256 ? cap : 256) * p.n_sub;
+        p.n_tasks = 1;
+        p.slot_doubles = (int64_t)nt[p.tri - 1] * 8 * 4096 + p.tri * 64;
+    } else if (precision == EMMA_PREC_BF16X4) {
         // one 8-wave workgroup per CU: 256 slices make the launch of
         // k_rev_bf16 a whole number of rounds (one per task) over the 256 CUs
         const int64_t cap = cdiv(n_rows > 0 ? n_rows : 1, 8192);
@@ -1368,11 +1981,12 @@ static int effective_precision(int precision, int *acc2) {
 extern "C" size_t emma_moments_workspace_size(int64_t n_rows, int32_t d, int32_t ntraj, uint32_t flags,
                                               int32_t precision) {
     if (d <= 0 || ntraj < 0) return 0;
-    if (precision == EMMA_PREC_BF16X4_ACC) precision = EMMA_PREC_BF16X4;  // the same plan
+    int acc2 = 0;
+    precision = mom::effective_precision(precision, &acc2);
     mom::Plan pl, pl0;
     // lag only matters through lag == 0; size for the larger task set
-    mom::make_plan(pl, nullptr, n_rows, d, nullptr, ntraj, 1, 1, 0, flags, precision, nullptr);
-    mom::make_plan(pl0, nullptr, n_rows, d, nullptr, ntraj, 0, 1, 0, flags, precision, nullptr);
+    mom::make_plan(pl, nullptr, n_rows, d, nullptr, ntraj, 1, 1, 0, flags, precision, acc2, nullptr);
+    mom::make_plan(pl0, nullptr, n_rows, d, nullptr, ntraj, 0, 1, 0, flags, precision, acc2, nullptr);
     return pl.ws_bytes > pl0.ws_bytes ? pl.ws_bytes : pl0.ws_bytes;
 }
 
@@ -1398,12 +2012,11 @@ extern "C" int emma_moments_lagged_weighted(const float *X, int64_t n_rows, int3
     int acc2 = 0;
     precision = mom::effective_precision(precision, &acc2);
     mom::Plan pl;
-    mom::make_plan(pl, X, n_rows, d, traj_offsets, ntraj, lag, stride, skip, flags, precision, nullptr);
+    mom::make_plan(pl, X, n_rows, d, traj_offsets, ntraj, lag, stride, skip, flags, precision, acc2, nullptr);
     EMMA_REQUIRE(workspace && workspace_bytes >= pl.ws_bytes,
                  "emma_moments_lagged: workspace too small (%zu < %zu)", workspace_bytes, pl.ws_bytes);
-    mom::make_plan(pl, X, n_rows, d, traj_offsets, ntraj, lag, stride, skip, flags, precision, workspace);
+    mom::make_plan(pl, X, n_rows, d, traj_offsets, ntraj, lag, stride, skip, flags, precision, acc2, workspace);
     pl.p.wts = row_weights;
-    pl.p.acc2 = acc2;
     hipStream_t s = (hipStream_t)stream;
     const mom::Params &p = pl.p;
     mom::k_prep<<<1, 1024, 0, s>>>(p);
@@ -1413,10 +2026,20 @@ extern "C" int emma_moments_lagged_weighted(const float *X, int64_t n_rows, int3
         mom::k_wtotal<<<1, 64, 0, s>>>(p);
         EMMA_TRY(check_launch("moments weight sums"));
     }
+    const int rm = (flags & EMMA_MOM_REMOVE_MEAN) ? 1 : 0;
+    if (p.tri) {
+        double *mxy = (flags & EMMA_MOM_C0T) ? Mxy : nullptr;
+        switch (p.tri) {
+            case 1: return mom::launch_tri<1>(p, pl.Sx, pl.Sy, rm, w, sx, sy, Mxx, mxy, s);
+            case 2: return mom::launch_tri<2>(p, pl.Sx, pl.Sy, rm, w, sx, sy, Mxx, mxy, s);
+            case 3: return mom::launch_tri<3>(p, pl.Sx, pl.Sy, rm, w, sx, sy, Mxx, mxy, s);
+            case 4: return mom::launch_tri<4>(p, pl.Sx, pl.Sy, rm, w, sx, sy, Mxx, mxy, s);
+            default: return mom::launch_tri<5>(p, pl.Sx, pl.Sy, rm, w, sx, sy, Mxx, mxy, s);
+        }
+    }
     EMMA_TRY(mom::launch_main(p, precision, s));
     mom::k_reduce_sums<<<(unsigned)cdiv(d, 256), 256, 0, s>>>(p, pl.Sx, pl.Sy, w, sx, sy);
     EMMA_TRY(check_launch("moments reduce sums"));
-    const int rm = (flags & EMMA_MOM_REMOVE_MEAN) ? 1 : 0;
     mom::k_reduce_mats<<<(unsigned)cdiv((int64_t)d * d, 256), 256, 0, s>>>(
         p, pl.Sx, pl.Sy, rm, Mxx, p.lag > 0 && (flags & EMMA_MOM_C0T) ? Mxy : nullptr, p.ctt ? Myy : nullptr);
     return check_launch("moments reduce");

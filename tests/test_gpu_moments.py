@@ -184,3 +184,37 @@ def test_deterministic_repeat():
     for x, y in zip(a, b):
         if x is not None:
             np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 31, 33, 63, 64, 65, 127, 129, 191, 193, 255, 257, 299, 319, 320, 321])
+@pytest.mark.parametrize("lengths,lag,stride,skip", [([9], 4, 1, 0), ([130, 5, 0, 64, 1, 700], 7, 1, 2),
+                                                     ([4097, 33, 2500], 20, 3, 1)])
+def test_reversible_column_groups(d, lengths, lag, stride, skip):
+    """Reversible bf16x4-acc moments around the column-group sizes (d < 4, d % 4 != 0, one
+    column more or less than a group of 64, the last d of the column-group kernel and the
+    first past it), with slices shorter than a stage, empty and too short trajectories,
+    strides and skips.  Bound: hi + lo leaves 2^-17 of each factor, 2^-16 of sum |u_i u_j|,
+    and the FP32 chains (at most 32 + 64 additions) 6e-6 of it; Cauchy-Schwarz bounds
+    that sum by the diagonal, and the shift by a sample mean at most doubles it."""
+    rng = np.random.default_rng(d + lag)
+    X = [(rng.standard_normal((n, d)) * 10.0 ** rng.uniform(-2, 2, d) + 3.0).astype(np.float32) for n in lengths]
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    Xt = _native.as_device_f32(np.concatenate(X, axis=0))
+    w, sx, sy, Mxx, Mxy, _ = _native.moments_lagged(Xt, off, lag, stride=stride, skip=skip, reversible=True,
+                                                    remove_mean=True, c0t=True, precision=_native.EMMA_PREC_BF16X4_ACC)
+    x = np.concatenate([t[skip:max(len(t) - lag, 0)][::stride] for t in X], axis=0).astype(np.float64)
+    y = np.concatenate([t[skip + lag:][::stride] for t in X], axis=0).astype(np.float64)
+    assert len(x) == len(y)
+    wr = 2.0 * len(x)
+    s = x.sum(axis=0) + y.sum(axis=0)
+    x, y = x - s / wr, y - s / wr
+    rxx, rxy = x.T @ x + y.T @ y, x.T @ y + y.T @ x
+    assert float(w.item()) == wr
+    scale = np.sqrt(np.outer(np.diag(rxx), np.diag(rxx)))
+    tol = 2.0 * (2.0 ** -16 + 6e-6)
+    Mxx, Mxy = Mxx.cpu().numpy(), Mxy.cpu().numpy()
+    assert np.all(np.abs(Mxx - rxx) <= tol * scale)
+    assert np.all(np.abs(Mxy - rxy) <= tol * scale)
+    assert np.array_equal(Mxx, Mxx.T) and np.array_equal(Mxy, Mxy.T)
+    np.testing.assert_allclose(sx.cpu().numpy(), s, rtol=1e-6, atol=1e-6 * np.sqrt(wr * np.diag(rxx)).max())
+    np.testing.assert_array_equal(sx.cpu().numpy(), sy.cpu().numpy())
