@@ -59,201 +59,436 @@ __device__ __forceinline__ double uniform(uint64_t seed, uint64_t counter) {
 // ------------------------------------------------------------------
 // kmeans++
 // ------------------------------------------------------------------
-// round 0: first pick
+// A round is three launches: the squared distances of the new center to the
+// earlier ones (k_kmpp_cc), the D^2 update (k_kmpp_d2), and the block sums with the
+// pick by the last workgroup to finish (k_kmpp_sum_pick).
+//
+// The D^2 update reads a frame only where the new center can be nearer than the
+// frame's current one: with D2 the stored FP32 distance of x to its nearest center
+// a, and cc the distance of a to the new center c, the triangle inequality gives
+// D(x, c) >= D(a, c) - D(x, a), so c cannot win where cc >= 4 D2, with the factor
+// raised by the relative rounding g = gamma_{d+2} of all three FP32 sums
+// (kmpp_factor): the loop's own result for c is then >= D2, and the strict '<'
+// leaves D2 alone.  Every D2, and so every pick, is the one of the full pass.  What
+// that saves depends on the data: 200,000 frames x 300 distances, k = 1000, read 240
+// MB per round without it (54 us of a 96 us round).
+
+// round 0: first pick; the counters of the later rounds
 __global__ void k_kmpp_first(const float *__restrict__ X, int64_t n, int d, uint64_t seed, float *__restrict__ C,
-                             int64_t *__restrict__ idx) {
+                             int64_t *__restrict__ idx, unsigned int *__restrict__ counters, int n_counters) {
     int64_t pick = (int64_t)(uniform(seed, 0) * (double)n);
     if (pick >= n) pick = n - 1;
     if (threadIdx.x == 0) idx[0] = pick;
     for (int i = threadIdx.x; i < d; i += blockDim.x) C[i] = X[pick * d + i];
+    for (int i = threadIdx.x; i < n_counters; i += blockDim.x) counters[i] = 0;
 }
 
-// D^2 update against center c (row of C): one thread per frame, the
-// sequential FP32 loop over the dims in order.  VEC: rows 16-byte aligned
-// (d % 4 == 0 and X aligned), read as float4 (the adds stay sequential).
-template <bool VEC>
-__global__ __launch_bounds__(256) void k_kmpp_d2(const float *__restrict__ X, int64_t n, int d,
-                                                 const float *__restrict__ c, int first, float *__restrict__ d2) {
-    extern __shared__ float s_c[];
-    for (int i = threadIdx.x; i < d; i += blockDim.x) s_c[i] = c[i];
-    __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float *x = X + i * d;
-    float v = first ? 0.0f : d2[i];
-    float di;
-    if constexpr (VEC) {
-        float acc = 0.0f;
-        auto step4 = [&](const float4 xv, const float4 cv) __attribute__((always_inline)) {
-            float t = __fsub_rn(xv.x, cv.x);
-            acc = __fadd_rn(acc, __fmul_rn(t, t));
-            t = __fsub_rn(xv.y, cv.y);
-            acc = __fadd_rn(acc, __fmul_rn(t, t));
-            t = __fsub_rn(xv.z, cv.z);
-            acc = __fadd_rn(acc, __fmul_rn(t, t));
-            t = __fsub_rn(xv.w, cv.w);
-            acc = __fadd_rn(acc, __fmul_rn(t, t));
-        };
-        // dims in order; the frame loads of 16 dims are issued before their terms
-        int q = 0;
-        for (; q + 16 <= d; q += 16) {
-            float4 xv[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) xv[u] = *reinterpret_cast<const float4 *>(x + q + 4 * u);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) step4(xv[u], *reinterpret_cast<const float4 *>(s_c + q + 4 * u));
-        }
-        for (; q < d; q += 4)
-            step4(*reinterpret_cast<const float4 *>(x + q), *reinterpret_cast<const float4 *>(s_c + q));
-        di = acc;
-    } else {
-        di = dist_seq(x, s_c, d);
+// cc[j] = |C_j - C_new|^2 for j < new (any summation order: its rounding is inside
+// kmpp_factor), one wavefront per center
+__global__ __launch_bounds__(256) void k_kmpp_cc(const float *__restrict__ C, int d, int nw, float *__restrict__ cc) {
+    const int lane = threadIdx.x & 63, j = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (j >= nw) return;
+    const float *a = C + (int64_t)j * d, *b = C + (int64_t)nw * d;
+    float s = 0.0f;
+#pragma unroll 4
+    for (int i = lane; i < d; i += 64) {
+        const float t = a[i] - b[i];
+        s = fmaf(t, t, s);
     }
-    if (first || di < v) v = di;
-    d2[i] = v;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) cc[j] = s;
+}
+static float kmpp_factor(int d) {
+    const double u = ldexp(1.0, -24), g = (d + 2) * u / (1.0 - (d + 2) * u);
+    return (float)(4.0 * (1.0 + 8.0 * g));
 }
 
-// Block sums of per-frame values (D^2 here, Lloyd's distances below): one
-// wavefront per block of BLOCK frames; lane l sums frames l, l + 64, ... of
-// the block in FP64 in that order, then a butterfly.  The loads of a lane are
-// issued before its adds.  done (may be null): skip once Lloyd has converged.
-__global__ __launch_bounds__(256) void k_block_sums(int64_t n, const float *__restrict__ d2,
-                                                    double *__restrict__ bsum, const int32_t *__restrict__ done) {
-    if (done && *done) return;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t b = (int64_t)blockIdx.x * 4 + wave;
-    const int64_t nb = (n + BLOCK - 1) / BLOCK;
-    if (b >= nb) return;
-    const int64_t lo = b * BLOCK;
-    double s = 0.0;
-    constexpr int U = 16;
-    for (int m0 = 0; m0 < BLOCK / 64; m0 += U) {
-        float v[U];
+__device__ __forceinline__ float dist_step(float acc, float x, float c) {
+    const float t = __fsub_rn(x, c);
+    return __fadd_rn(acc, __fmul_rn(t, t));
+}
+
+// The sequential FP32 distance of row x to c (LDS), the loads of 16 dims in flight
+// before their terms.  VEC: rows 16-byte aligned (d % 4 == 0 and X aligned).
+template <bool VEC>
+__device__ __forceinline__ float dist_row(const float *__restrict__ x, const float *c, int d) {
+    float acc = 0.0f;
+    int q = 0;
+    for (; q + 16 <= d; q += 16) {
+        float v[16];
+        if constexpr (VEC) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t i = lo + (m0 + u) * 64 + lane;
+            for (int u = 0; u < 4; ++u) {
+                const float4 w = *reinterpret_cast<const float4 *>(x + q + 4 * u);
+                v[4 * u] = w.x, v[4 * u + 1] = w.y, v[4 * u + 2] = w.z, v[4 * u + 3] = w.w;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = x[q + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) acc = dist_step(acc, v[u], c[q + u]);
+    }
+    for (; q < d; ++q) acc = dist_step(acc, x[q], c[q]);
+    return acc;
+}
+
+// D^2 update against the new center C[r - 1]: the frames that the triangle
+// inequality leaves are compacted over the workgroup, one thread each.  A thread that
+// reads its row itself touches a cache line of its own with every load; from 64 dims
+// on (ROWS_STAGED) a wave reads its 64 rows together instead, 64 dims at a time with 16
+// lanes to a row, and its threads add from LDS (the next 64 dims in flight meanwhile).
+// Below, half of the lanes or more would have no dims to read.  Rows of any alignment:
+// the loads are 4-byte aligned, those across a row's end element by element.
+// (200,000 distances x 300, k = 1000, per round: 54 us for all rows by their own threads, 30 with
+// the triangle inequality, 26 staged.)
+enum Rows { ROWS_ANY = 0, ROWS_VEC = 1, ROWS_STAGED = 2 };
+constexpr int SDIM = 64, SPITCH = SDIM + 4;  // pitch: 16-byte rows on distinct banks
+template <int ROWS>
+__global__ __launch_bounds__(256) void k_kmpp_d2(const float *__restrict__ X, int64_t n, int d,
+                                                 const float *__restrict__ c, int r, float factor,
+                                                 const float *__restrict__ cc, float *__restrict__ d2,
+                                                 int32_t *__restrict__ owner) {
+    extern __shared__ float s_c[];
+    __shared__ __align__(16) float s_x[ROWS == ROWS_STAGED ? 4 * 64 * SPITCH : 4];
+    __shared__ int s_list[256];
+    __shared__ float s_v[256];
+    __shared__ int s_cnt;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t i0 = (int64_t)blockIdx.x * 256, i = i0 + tid;
+    if (tid == 0) s_cnt = 0;
+    __syncthreads();
+    bool act = false;
+    float v = 0.0f;
+    if (i < n) {
+        act = true;
+        if (r > 1) {
+            v = d2[i];
+            // v tiny, overflowed or NaN: no argument from it
+            act = !(v > 1e-25f && v < 1e37f && cc[owner[i]] >= factor * v);
+        }
+    }
+    const unsigned long long m = __ballot(act);
+    if (m) {
+        const int leader = __builtin_ctzll(m);
+        int base = 0;
+        if (lane == leader) base = atomicAdd(&s_cnt, __popcll(m));
+        base = __shfl(base, leader, 64);
+        if (act) {
+            const int q = base + __popcll(m & ((1ull << lane) - 1ull));
+            s_list[q] = tid;
+            s_v[q] = v;
+        }
+    }
+    __syncthreads();
+    const int na = s_cnt;
+    if (na == 0) return;
+    float di = 0.0f;
+    if constexpr (ROWS == ROWS_STAGED) {
+        const int l0 = tid & ~63, cnt = na - l0 < 64 ? na - l0 : 64;
+        if (cnt <= 0) return;  // no barrier below
+        float *buf = s_x + (tid >> 6) * 64 * SPITCH;
+        const int sub = lane >> 4, col = (lane & 15) * 4;
+        int row[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) row[u] = u * 4 + sub < cnt ? s_list[l0 + u * 4 + sub] : -1;
+        const float *base = X + i0 * d;
+        float4 t[16];
+        auto load = [&](int q0) __attribute__((always_inline)) {
+            const int q = q0 + col;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                if (row[u] < 0 || q >= d) continue;
+                const float *x = base + (int64_t)row[u] * d + q;
+                if (q + 4 <= d) {
+                    const float4_u w = *reinterpret_cast<const float4_u *>(x);
+                    t[u] = make_float4(w[0], w[1], w[2], w[3]);
+                } else {
+                    t[u].x = x[0];
+                    if (q + 1 < d) t[u].y = x[1];
+                    if (q + 2 < d) t[u].z = x[2];
+                }
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < 16; ++u) t[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        load(0);
+        for (int q0 = 0; q0 < d; q0 += SDIM) {
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                *reinterpret_cast<float4 *>(buf + (u * 4 + sub) * SPITCH + col) = t[u];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (q0 + SDIM < d) load(q0 + SDIM);
+            const float *mine = buf + lane * SPITCH;
+            const int nq = d - q0 < SDIM ? d - q0 : SDIM;
+            int q = 0;
+            for (; q + 16 <= nq; q += 16) {
+                float4 w[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[u] = *reinterpret_cast<const float4 *>(mine + q + 4 * u);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    di = dist_step(di, w[u].x, c[q0 + q + 4 * u]);
+                    di = dist_step(di, w[u].y, c[q0 + q + 4 * u + 1]);
+                    di = dist_step(di, w[u].z, c[q0 + q + 4 * u + 2]);
+                    di = dist_step(di, w[u].w, c[q0 + q + 4 * u + 3]);
+                }
+            }
+            for (; q < nq; ++q) di = dist_step(di, mine[q], c[q0 + q]);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    } else {
+        for (int q = tid; q < d; q += 256) s_c[q] = c[q];
+        __syncthreads();
+        if (tid < na) di = dist_row<ROWS == ROWS_VEC>(X + (i0 + s_list[tid]) * d, s_c, d);
+    }
+    if (tid < na && (r == 1 || di < s_v[tid])) {
+        const int64_t f = i0 + s_list[tid];
+        d2[f] = di;
+        owner[f] = r - 1;
+    }
+}
+
+// Lane l's value added after those of lanes 0 .. l - 1, in that order: inclusive
+// running sums from `run`, as one thread walking the values would form them.  The
+// values are >= 0 or NaN, and 0 from lane cnt on, so that adding those changes nothing
+// and the lanes can be taken 16 at a time.
+__device__ __forceinline__ double running_sum(double a, int cnt, double run, int lane) {
+    double mine = run;
+    const long long bits = __double_as_longlong(a);
+    for (int l0 = 0; l0 < cnt; l0 += 16) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int lo = __builtin_amdgcn_readlane((int)(bits & 0xffffffffll), l0 + u);
+            const int hi = __builtin_amdgcn_readlane((int)(bits >> 32), l0 + u);
+            run = run + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+            mine = lane == l0 + u ? run : mine;
+        }
+    }
+    return mine;
+}
+__device__ __forceinline__ double lane_value(double a, int l) { return __shfl(a, l, 64); }
+
+// One step of the oracle's walk over cnt <= 64 values a (lane l holds value l):
+// the first whose running sum passes T, or else the last positive one (-1: none);
+// `before` becomes the running sum in front of it.
+__device__ __forceinline__ int walk_step(double a, int cnt, double T, double &before, int lane) {
+    const double run = running_sum(a, cnt, before, lane);
+    const unsigned long long over = __ballot(lane < cnt && run > T);
+    const unsigned long long pos = __ballot(lane < cnt && a > 0.0);
+    const int sel = over ? __builtin_ctzll(over) : (pos ? 63 - __builtin_clzll(pos) : -1);
+    if (sel > 0) before = lane_value(run, sel - 1);
+    return sel;
+}
+
+__device__ __forceinline__ void put_coherent(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_coherent(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// the counter's old value, after every earlier store of this thread has completed
+__device__ __forceinline__ unsigned int arrive(unsigned int *counter) {
+    __builtin_amdgcn_s_waitcnt(0);
+    return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Block sums (one workgroup per block of BLOCK frames), superblock sums by the last
+// block of each, and the pick of round r by the last superblock's workgroup: exactly
+// the oracle's oracle_kmpp_pick.  The sums travel between workgroups as coherent
+// (device-scope) stores and loads, waited for before the arrival count: a release
+// fence instead would write back the whole L2 from every workgroup.  The counters
+// only grow: round r is complete at r times the number of arrivals.
+// (Per round 41 us for block sums of one wave per block and a one-wave pick, 200,000
+// frames; 13 here.  What is left is a chain of some eight dependent round trips to
+// memory.)
+__global__ __launch_bounds__(256) void k_kmpp_sum_pick(const float *__restrict__ X, int64_t n, int d, uint64_t seed,
+                                                       int r, const float *__restrict__ d2,
+                                                       double *__restrict__ bsum, double *__restrict__ sbsum,
+                                                       unsigned int *__restrict__ counters,
+                                                       float *__restrict__ C, int64_t *__restrict__ idx) {
+    __shared__ float s_d[SEG * (SEG + 1)];  // a block's values, a segment per row (padded)
+    __shared__ int s_last, s_blk;
+    __shared__ int64_t s_pick;
+    __shared__ double s_before, s_T;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t nb = (n + BLOCK - 1) / BLOCK, nsb = (nb + SUPER - 1) / SUPER;
+    // past the last frame: 0, which the sums below add without a change (values >= 0 or NaN)
+    auto load_block = [&](int64_t blk) __attribute__((always_inline)) {
+        const int64_t lo = blk * BLOCK;
+        float v[BLOCK / 256];
+#pragma unroll
+        for (int u = 0; u < BLOCK / 256; ++u) {
+            const int64_t i = lo + u * 256 + tid;
             v[u] = i < n ? d2[i] : 0.0f;
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t i = lo + (m0 + u) * 64 + lane;
-            if (i < n) s = s + (double)v[u];
+        for (int u = 0; u < BLOCK / 256; ++u) {
+            const int o = u * 256 + tid;
+            s_d[(o / SEG) * (SEG + 1) + o % SEG] = v[u];
         }
-    }
-    s = wave_butterfly_sum(s);
-    if (lane == 0) bsum[b] = s;
-}
-
-// Pick of round r (one wavefront), exactly the oracle's oracle_kmpp_pick.
-__global__ __launch_bounds__(64) void k_kmpp_pick(const float *__restrict__ X, int64_t n, int d, uint64_t seed,
-                                                  int r, const float *__restrict__ d2,
-                                                  const double *__restrict__ bsum, double *__restrict__ sbsum,
-                                                  float *__restrict__ C, int64_t *__restrict__ idx) {
-    __shared__ double s_seg[SEG];
-    __shared__ int64_t s_pick;
-    const int lane = threadIdx.x;
-    const int64_t nb = (n + BLOCK - 1) / BLOCK;
-    const int64_t nsb = (nb + SUPER - 1) / SUPER;
-    for (int64_t sb = lane; sb < nsb; sb += 64) {
-        double a = 0.0;
-        for (int64_t b = sb * SUPER; b < nb && b < (sb + 1) * SUPER; ++b) a = a + bsum[b];
-        sbsum[sb] = a;
-    }
+    };
+    const int64_t b = blockIdx.x, sb = b / SUPER;
+    load_block(b);
     __syncthreads();
-    const double u = uniform(seed, (uint64_t)r);
-    // lane 0 walks superblocks and blocks
-    int64_t blk = -1;
-    double before = 0.0, total = 0.0;
-    if (lane == 0) {
-        for (int64_t sb = 0; sb < nsb; ++sb) total = total + sbsum[sb];
-        if (!(total > 0.0)) {
-            int64_t i = (int64_t)(u * (double)n);
-            s_pick = i < n ? i : n - 1;
-        } else {
-            s_pick = -1;
-            const double T = u * total;
-            double run = 0.0, last_before = 0.0;
-            int64_t sel = -1, last_pos = -1;
-            for (int64_t sb = 0; sb < nsb; ++sb) {
-                const double a = sbsum[sb];
-                const double prev = run;
-                run = run + a;
-                if (a > 0.0) { last_pos = sb; last_before = prev; }
-                if (run > T) { sel = sb; before = prev; break; }
-            }
-            if (sel < 0) { sel = last_pos; before = last_before; }
-            const int64_t sb = sel;
-            run = before; sel = -1; last_pos = -1;
-            for (int64_t b = sb * SUPER; b < nb && b < (sb + 1) * SUPER; ++b) {
-                const double prev = run;
-                run = run + bsum[b];
-                if (bsum[b] > 0.0) { last_pos = b; last_before = prev; }
-                if (run > T) { sel = b; before = prev; break; }
-            }
-            if (sel < 0) { sel = last_pos; before = last_before; }
-            blk = sel;
-        }
-        s_seg[0] = before;  // pass through shared memory
-        s_seg[1] = total > 0.0 ? u * total : 0.0;
-        s_seg[2] = (double)blk;
-    }
-    __syncthreads();
-    const double before_blk = s_seg[0], T = s_seg[1];
-    blk = (int64_t)s_seg[2];
-    __syncthreads();
-    if (blk >= 0) {
-        // segment sums of the chosen block in parallel (sequential inside each segment)
-        const int64_t blo = blk * BLOCK, bhi = blo + BLOCK < n ? blo + BLOCK : n;
-        const int64_t g = blo + (int64_t)lane * SEG;
-        double a = 0.0;
-        if (g < bhi)
-            for (int64_t i = g; i < bhi && i < g + SEG; ++i) a = a + (double)d2[i];
-        s_seg[lane] = a;
-        __syncthreads();
+    double a_blk = 0.0, a_sb = 0.0;  // this superblock's block sums, its sum (the pick of a single one)
+    if (tid < 64) {
+        double s = 0.0;
+#pragma unroll 16
+        for (int m = 0; m < BLOCK / 64; ++m) s = s + (double)s_d[m * (SEG + 1) + lane];
+        s = wave_butterfly_sum(s);
+        const int in_sb = (int)(nb - sb * SUPER < SUPER ? nb - sb * SUPER : SUPER);
+        unsigned int seen = 0;
         if (lane == 0) {
-            double run = before_blk, last_before = 0.0, before_seg = 0.0;
+            put_coherent(bsum + b, s);
+            seen = arrive(counters + 1 + sb);
+        }
+        seen = __shfl(seen, 0, 64);
+        int last = 0;
+        if (seen + 1 == (unsigned int)r * (unsigned int)in_sb) {
+            a_blk = lane < in_sb ? get_coherent(bsum + sb * SUPER + lane) : 0.0;
+            a_sb = lane_value(running_sum(a_blk, in_sb, 0.0, lane), in_sb - 1);
+            unsigned int top = 0;
+            if (nsb > 1 && lane == 0) {
+                put_coherent(sbsum + sb, a_sb);
+                top = arrive(counters);
+            }
+            last = nsb == 1 || __shfl(top, 0, 64) + 1 == (unsigned int)r * (unsigned int)nsb;
+        }
+        if (lane == 0) s_last = last;
+    }
+    __syncthreads();
+    if (!s_last) return;
+
+    const double u = uniform(seed, (uint64_t)r);
+    if (tid < 64) {
+        // superblocks 64 at a time: the total, then the walk
+        auto superblocks = [&](int64_t s0, int cnt) __attribute__((always_inline)) {
+            if (nsb == 1) return lane == 0 ? a_sb : 0.0;
+            return lane < cnt ? get_coherent(sbsum + s0 + lane) : 0.0;
+        };
+        double total = 0.0;
+        for (int64_t s0 = 0; s0 < nsb; s0 += 64) {
+            const int cnt = (int)(nsb - s0 < 64 ? nsb - s0 : 64);
+            const double a = superblocks(s0, cnt);
+            total = lane_value(running_sum(a, cnt, total, lane), cnt - 1);
+        }
+        int64_t blk = -1;
+        double before = 0.0;
+        const double T = u * total;
+        if (!(total > 0.0)) {
+            const int64_t i = (int64_t)(u * (double)n);
+            if (lane == 0) s_pick = i < n ? i : n - 1;
+        } else {
             int64_t sel = -1, last_pos = -1;
-            for (int q = 0; q < SEG; ++q) {
-                const int64_t gq = blo + (int64_t)q * SEG;
-                if (gq >= bhi) break;
-                const double prev = run;
-                run = run + s_seg[q];
-                if (s_seg[q] > 0.0) { last_pos = gq; last_before = prev; }
-                if (run > T) { sel = gq; before_seg = prev; break; }
+            double run = 0.0, last_before = 0.0;
+            for (int64_t s0 = 0; s0 < nsb && sel < 0; s0 += 64) {
+                const int cnt = (int)(nsb - s0 < 64 ? nsb - s0 : 64);
+                const double a = superblocks(s0, cnt);
+                const double rs = running_sum(a, cnt, run, lane);
+                const unsigned long long over = __ballot(lane < cnt && rs > T), pos = __ballot(lane < cnt && a > 0.0);
+                if (over) {
+                    const int q = __builtin_ctzll(over);
+                    sel = s0 + q;
+                    before = q > 0 ? lane_value(rs, q - 1) : run;
+                } else if (pos) {
+                    const int q = 63 - __builtin_clzll(pos);
+                    last_pos = s0 + q;
+                    last_before = q > 0 ? lane_value(rs, q - 1) : run;
+                }
+                run = lane_value(rs, cnt - 1);
             }
-            if (sel < 0) { sel = last_pos; before_seg = last_before; }
-            const int64_t gs = sel, ghi = gs + SEG < bhi ? gs + SEG : bhi;
-            run = before_seg; sel = -1; last_pos = -1;
-            for (int64_t i = gs; i < ghi; ++i) {
-                run = run + (double)d2[i];
-                if (d2[i] > 0.0f) last_pos = i;
-                if (run > T) { sel = i; break; }
+            if (sel < 0) {
+                sel = last_pos;
+                before = last_before;
             }
-            if (sel < 0) sel = last_pos;
-            s_pick = sel;
+            const int cnt = (int)(nb - sel * SUPER < SUPER ? nb - sel * SUPER : SUPER);
+            const double a = nsb == 1 ? a_blk : lane < cnt ? get_coherent(bsum + sel * SUPER + lane) : 0.0;
+            blk = sel * SUPER + walk_step(a, cnt, T, before, lane);
+        }
+        if (lane == 0) {
+            s_before = before;
+            s_T = T;
+            s_blk = (int)blk;
         }
     }
     __syncthreads();
+    const int64_t blk = s_blk;
+    if (blk >= 0) {
+        load_block(blk);
+        __syncthreads();
+        if (tid < 64) {
+            // segment sums (sequential inside a segment, one per lane), then the segment's frames
+            const int64_t blo = blk * BLOCK, left = n - blo < BLOCK ? n - blo : BLOCK;
+            const double T = s_T;
+            double before = s_before;
+            const int nseg = (int)((left + SEG - 1) / SEG);
+            double a = 0.0;
+#pragma unroll 16
+            for (int q = 0; q < SEG; ++q) a = a + (double)s_d[lane * (SEG + 1) + q];
+            const int seg = walk_step(a, nseg, T, before, lane);
+            const int nf = (int)(left - seg * SEG < SEG ? left - seg * SEG : SEG);
+            const int fr = walk_step((double)s_d[seg * (SEG + 1) + lane], nf, T, before, lane);
+            if (lane == 0) s_pick = blo + (int64_t)seg * SEG + fr;
+        }
+        __syncthreads();
+    }
     const int64_t pick = s_pick;
-    if (lane == 0) idx[r] = pick;
-    for (int i = lane; i < d; i += 64) C[(int64_t)r * d + i] = X[pick * d + i];
+    if (tid == 0) idx[r] = pick;
+    for (int i = tid; i < d; i += 256) C[(int64_t)r * d + i] = X[pick * d + i];
 }
 
 struct PpWs {
     float *d2;
+    int32_t *owner;
+    float *cc;
     double *bsum, *sbsum;
+    unsigned int *counters;  // [1 + superblocks]
     size_t bytes;
 };
 
-static PpWs carve_pp(void *ws, int64_t n) {
+static PpWs carve_pp(void *ws, int64_t n, int k) {
     PpWs w{};
     Carver cv(ws);
-    const int64_t nb = cdiv(n, BLOCK);
+    const int64_t nb = cdiv(n, BLOCK), nsb = cdiv(nb, SUPER);
     w.d2 = cv.take<float>(n);
+    w.owner = cv.take<int32_t>(n);
+    w.cc = cv.take<float>(k);
     w.bsum = cv.take<double>(nb);
-    w.sbsum = cv.take<double>(cdiv(nb, SUPER));
+    w.sbsum = cv.take<double>(nsb);
+    w.counters = cv.take<unsigned int>(1 + (size_t)nsb);
     w.bytes = cv.bytes();
     return w;
+}
+
+// Block sums of Lloyd's distances: one workgroup per block of BLOCK frames, whose
+// values are loaded in one round trip; the first wave's lane l adds frames l, l +
+// 64, ... in FP64 in that order, then a butterfly (the oracle's order; the zeros
+// past the last frame change no sum).  done: skip
+// once Lloyd has converged.
+__global__ __launch_bounds__(256) void k_block_sums(int64_t n, const float *__restrict__ d2,
+                                                    double *__restrict__ bsum, const int32_t *__restrict__ done) {
+    if (*done) return;
+    __shared__ float s_d[BLOCK];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t lo = (int64_t)blockIdx.x * BLOCK, left = n - lo;
+    float v[BLOCK / 256];
+#pragma unroll
+    for (int u = 0; u < BLOCK / 256; ++u) v[u] = u * 256 + tid < left ? d2[lo + u * 256 + tid] : 0.0f;
+#pragma unroll
+    for (int u = 0; u < BLOCK / 256; ++u) s_d[u * 256 + tid] = v[u];
+    __syncthreads();
+    if (tid >= 64) return;
+    double s = 0.0;
+#pragma unroll 16
+    for (int m = 0; m < BLOCK / 64; ++m) s = s + (double)s_d[m * 64 + lane];
+    s = wave_butterfly_sum(s);
+    if (lane == 0) bsum[blockIdx.x] = s;
 }
 
 // ------------------------------------------------------------------
@@ -520,9 +755,8 @@ using namespace emma;
 
 extern "C" size_t emma_kmeanspp_workspace_size(int64_t n, int32_t d, int32_t k) {
     (void)d;
-    (void)k;
-    if (n <= 0) return 0;
-    return km::carve_pp(nullptr, n).bytes;
+    if (n <= 0 || k <= 0) return 0;
+    return km::carve_pp(nullptr, n, k).bytes;
 }
 
 extern "C" int emma_kmeanspp(const float *X, int64_t n, int32_t d, int32_t k, uint64_t seed, float *C_out,
@@ -530,24 +764,28 @@ extern "C" int emma_kmeanspp(const float *X, int64_t n, int32_t d, int32_t k, ui
     EMMA_REQUIRE(n > 0 && d > 0 && k > 0, "emma_kmeanspp: bad sizes n=%lld d=%d k=%d", (long long)n, d, k);
     EMMA_REQUIRE(X && C_out && idx_out, "emma_kmeanspp: NULL pointer");
     EMMA_REQUIRE(d <= 16384, "emma_kmeanspp: d=%d too large", d);
-    const size_t need = km::carve_pp(nullptr, n).bytes;
+    const size_t need = km::carve_pp(nullptr, n, k).bytes;
     EMMA_REQUIRE(workspace && workspace_bytes >= need, "emma_kmeanspp: workspace too small (%zu < %zu)",
                  workspace_bytes, need);
-    km::PpWs w = km::carve_pp(workspace, n);
+    km::PpWs w = km::carve_pp(workspace, n, k);
     hipStream_t s = (hipStream_t)stream;
     const int64_t nb = cdiv(n, km::BLOCK);
-    km::k_kmpp_first<<<1, 256, 0, s>>>(X, n, d, seed, C_out, idx_out);
+    km::k_kmpp_first<<<1, 256, 0, s>>>(X, n, d, seed, C_out, idx_out, w.counters, (int)(1 + cdiv(nb, km::SUPER)));
     EMMA_TRY(check_launch("kmeans++ first"));
     const bool vec = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
     const size_t shm = sizeof(float) * (size_t)d;
+    const float factor = km::kmpp_factor(d);
     for (int r = 1; r < k; ++r) {
         const float *c = C_out + (int64_t)(r - 1) * d;
-        if (vec)
-            km::k_kmpp_d2<true><<<(unsigned)cdiv(n, 256), 256, shm, s>>>(X, n, d, c, r == 1 ? 1 : 0, w.d2);
+        if (r > 1) km::k_kmpp_cc<<<(unsigned)cdiv(r - 1, 4), 256, 0, s>>>(C_out, d, r - 1, w.cc);
+        const unsigned g = (unsigned)cdiv(n, 256);
+        if (d >= km::SDIM)
+            km::k_kmpp_d2<km::ROWS_STAGED><<<g, 256, 0, s>>>(X, n, d, c, r, factor, w.cc, w.d2, w.owner);
+        else if (vec)
+            km::k_kmpp_d2<km::ROWS_VEC><<<g, 256, shm, s>>>(X, n, d, c, r, factor, w.cc, w.d2, w.owner);
         else
-            km::k_kmpp_d2<false><<<(unsigned)cdiv(n, 256), 256, shm, s>>>(X, n, d, c, r == 1 ? 1 : 0, w.d2);
-        km::k_block_sums<<<(unsigned)cdiv(nb, 4), 256, 0, s>>>(n, w.d2, w.bsum, nullptr);
-        km::k_kmpp_pick<<<1, 64, 0, s>>>(X, n, d, seed, r, w.d2, w.bsum, w.sbsum, C_out, idx_out);
+            km::k_kmpp_d2<km::ROWS_ANY><<<g, 256, shm, s>>>(X, n, d, c, r, factor, w.cc, w.d2, w.owner);
+        km::k_kmpp_sum_pick<<<(unsigned)nb, 256, 0, s>>>(X, n, d, seed, r, w.d2, w.bsum, w.sbsum, w.counters, C_out, idx_out);
     }
     return check_launch("kmeans++ rounds");
 }
@@ -595,7 +833,7 @@ extern "C" int emma_lloyd(const float *X, int64_t n, int32_t d, float *C, int32_
         else
             km::k_lloyd_dist<false, false><<<(unsigned)cdiv(n, 256), 256, 0, s>>>(X, n, d, C, k, labels, w.dist,
                                                                                  w.blk_cnt, w.done);
-        km::k_block_sums<<<(unsigned)cdiv(nb, 4), 256, 0, s>>>(n, w.dist, w.bcost, w.done);
+        km::k_block_sums<<<(unsigned)nb, 256, 0, s>>>(n, w.dist, w.bcost, w.done);
         km::k_lloyd_cost_final<<<1, 1, 0, s>>>(nb, w.bcost, tol, it, w.prev_cost, inertias, n_iter, converged,
                                                w.done);
         EMMA_TRY(check_launch("lloyd iteration"));

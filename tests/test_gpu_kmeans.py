@@ -37,6 +37,29 @@ def test_kmeanspp_identical_picks(n, d, k, seed):
     np.testing.assert_array_equal(C, C_ref)
 
 
+@pytest.mark.parametrize("n,d,k,scale,shift", [
+    (5000, 7, 40, 1.0, 0), (8193, 64, 33, 1.0, 0), (8193, 64, 33, 1.0, 1), (5000, 131, 40, 1.0, 0),
+    (3000, 126, 20, 1.0, 1), (3000, 63, 20, 1.0, 0), (3000, 60, 20, 1.0, 1), (4096, 4, 130, 1.0, 0), (1, 3, 3, 1.0, 0),
+    (270000, 3, 12, 1.0, 0), (300, 16384, 5, 1.0, 0), (4097, 20, 30, 1e-14, 0), (4097, 20, 30, 1e-20, 0),
+    (4097, 20, 30, 1e19, 0), (4097, 20, 30, 1e25, 0)])
+def test_kmeanspp_skipped_frames(n, d, k, scale, shift):
+    """Separated groups, so that the triangle inequality leaves out most frames of a
+    round: picks identical at block and superblock edges, in rows that are not 16-byte
+    aligned, and where distances underflow or overflow (no frame may be left out)."""
+    t = _native.torch()
+    rng = np.random.default_rng(n + d)
+    X = (rng.standard_normal((n, d)) + 40.0 * rng.standard_normal((9, d))[rng.integers(0, 9, n)])
+    X = (X * scale).astype(np.float32)
+    with np.errstate(over="ignore"):
+        C_ref, idx_ref = on.kmeanspp(X, k, 3, nthreads=4)
+    buf = t.empty(n * d + shift, dtype=t.float32, device="cuda")
+    Xt = buf[shift:].view(n, d)
+    Xt.copy_(t.from_numpy(X))
+    C, idx = _native.kmeanspp(Xt, k, 3)
+    np.testing.assert_array_equal(idx.cpu().numpy(), idx_ref)
+    np.testing.assert_array_equal(C.cpu().numpy(), C_ref)
+
+
 def test_kmeanspp_duplicate_points_total_zero():
     X = np.repeat(np.arange(3, dtype=np.float32)[:, None], 50, axis=0)
     C_ref, idx_ref = on.kmeanspp(X, 5, 11)
