@@ -535,39 +535,47 @@ __global__ void k_lloyd_init(int32_t *done, double *prev_cost, int32_t *n_iter, 
     *converged = 0;
 }
 
-// One thread per frame.  HIST: the frame's count in its block's per-label
-// counts (before the center update).  Otherwise: the exact distance to the
-// center of its label (the sequential FP32 loop; VEC as in k_kmpp_d2, with C
-// 16-byte aligned too), run after the update so that the cost is that of the
-// new clusters against their means.  The block sums of the distances (the
-// oracle's cost order) follow in k_block_sums.
-template <bool VEC, bool HIST>
+// Counts of the labels of one block of frames, one workgroup per block, in LDS: one
+// LDS atomic per run of equal labels in a wave (consecutive frames of a trajectory
+// mostly share their label, and 64 lanes adding 1 to one counter serialize).  (Device
+// atomics and clearing the counts beforehand: 21 us at 250,000 frames, k = 200; now
+// 4.)
+__global__ __launch_bounds__(1024) void k_lloyd_hist(int64_t n, int k, const int32_t *__restrict__ labels,
+                                                     int32_t *__restrict__ blk_cnt,
+                                                     const int32_t *__restrict__ done) {
+    if (*done) return;
+    extern __shared__ int32_t s_run[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t b = blockIdx.x, lo = b * BLOCK;
+    int lab[BLOCK / 1024];
+#pragma unroll
+    for (int u = 0; u < BLOCK / 1024; ++u) lab[u] = lo + u * 1024 + tid < n ? labels[lo + u * 1024 + tid] : -1;
+    for (int j = tid; j < k; j += 1024) s_run[j] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < BLOCK / 1024; ++u) {
+        const int prev = __shfl_up(lab[u], 1, 64);
+        const bool start = lane == 0 || prev != lab[u];
+        const unsigned long long starts = __ballot(start);
+        const unsigned long long later = starts & ~((2ull << lane) - 1ull);  // starts after this lane
+        if (start && lab[u] >= 0) atomicAdd(&s_run[lab[u]], (later ? __builtin_ctzll(later) : 64) - lane);
+    }
+    __syncthreads();
+    for (int j = tid; j < k; j += 1024) blk_cnt[b * k + j] = s_run[j];
+}
+
+// The exact distance to the center of its label (the sequential FP32 loop; VEC: rows
+// of X and C 16-byte aligned), one thread per frame, run after the update so that the
+// cost is that of the new clusters against their means.  The block sums of the
+// distances (the oracle's cost order) follow in k_block_sums.
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_lloyd_dist(const float *__restrict__ X, int64_t n, int d,
-                                                    const float *__restrict__ C, int k,
-                                                    const int32_t *__restrict__ labels, float *__restrict__ dist,
-                                                    int32_t *__restrict__ blk_cnt, const int32_t *__restrict__ done) {
+                                                    const float *__restrict__ C, const int32_t *__restrict__ labels,
+                                                    float *__restrict__ dist, const int32_t *__restrict__ done) {
     if (*done) return;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int lab = labels[i];
-    if constexpr (HIST) {
-        // histogram of labels per block (zeroed by k_fill_i32 beforehand), one
-        // atomic per run of equal labels in the wave: consecutive frames of a
-        // trajectory mostly share their label, and 64 lanes adding 1 to one
-        // counter serialize.  A wave's frames lie in one block (BLOCK % 64 == 0);
-        // the active lanes are 0 .. m - 1 (only a final partial wave has m < 64).
-        const int lane = threadIdx.x & 63;
-        const unsigned long long active = __ballot(1);
-        const int prev = __shfl_up(lab, 1, 64);
-        const bool start = lane == 0 || prev != lab;
-        const unsigned long long starts = __ballot(start);
-        if (start) {
-            const unsigned long long later = starts & ~((2ull << lane) - 1ull);  // starts after this lane
-            const int end = later ? __builtin_ctzll(later) : __popcll(active);
-            atomicAdd(&blk_cnt[(i / BLOCK) * (int64_t)k + lab], end - lane);
-        }
-        return;
-    }
     const float *x = X + i * d;
     const float *c = C + (int64_t)lab * d;
     float di;
@@ -611,64 +619,117 @@ __global__ __launch_bounds__(1024) void k_lloyd_scan(int k, int64_t nb, int64_t 
                                                      int64_t *__restrict__ off, int64_t *__restrict__ coff,
                                                      int32_t *__restrict__ blk_cnt, const int32_t *__restrict__ done) {
     if (*done) return;
-    for (int j = threadIdx.x; j < k; j += blockDim.x) {
-        int32_t run = 0;
-#pragma unroll 8
-        for (int64_t b = 0; b < nb; ++b) {
-            const int32_t v = blk_cnt[b * k + j];
-            blk_cnt[b * k + j] = run;
-            run += v;
+    __shared__ int64_t s_a[16], s_c[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int64_t a0 = 0, c0 = 0;  // members and chunks of the labels before this pass of 1024
+    for (int j0 = 0; j0 < k; j0 += 1024) {
+        const int j = j0 + tid;
+        int64_t m = 0;
+        if (j < k) {
+            int32_t run = 0, v[16];
+            for (int64_t b = 0; b < nb; b += 16) {
+                const int cnt16 = nb - b < 16 ? (int)(nb - b) : 16;
+#pragma unroll
+                for (int u = 0; u < 16; ++u) v[u] = u < cnt16 ? blk_cnt[(b + u) * k + j] : 0;
+#pragma unroll
+                for (int u = 0; u < 16; ++u) {
+                    if (u < cnt16) blk_cnt[(b + u) * k + j] = run;
+                    run += v[u];
+                }
+            }
+            cnt[j] = m = run;
         }
-        cnt[j] = run;
+        const int64_t ch = (m + CHUNK - 1) / CHUNK;
+        int64_t a = m, c = ch;  // inclusive sums over the wave
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int64_t ta = __shfl_up(a, o, 64), tc = __shfl_up(c, o, 64);
+            if (lane >= o) {
+                a += ta;
+                c += tc;
+            }
+        }
+        __syncthreads();
+        if (lane == 63) {
+            s_a[wave] = a;
+            s_c[wave] = c;
+        }
+        __syncthreads();
+        int64_t ta = a0, tc = c0;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) {
+                a += s_a[w];
+                c += s_c[w];
+            }
+            ta += s_a[w];
+            tc += s_c[w];
+        }
+        if (j < k) {
+            off[j] = a0 + a - m;
+            coff[j] = c0 + c - ch;
+        }
+        a0 = ta;
+        c0 = tc;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int64_t a = 0, c = 0;
-        for (int j = 0; j < k; ++j) {
-            off[j] = a;
-            coff[j] = c;
-            a += cnt[j];
-            c += (cnt[j] + CHUNK - 1) / CHUNK;
-        }
-        off[k] = a;
-        coff[k] = c;
+    if (tid == 0) {
+        off[k] = a0;
+        coff[k] = c0;
     }
 }
 
-__global__ __launch_bounds__(256) void k_fill_i32(int32_t *p, int64_t n, const int32_t *done) {
+// Stable scatter: position of frame i = off[label] + (members of label in earlier
+// blocks) + (members in this block before i).  One workgroup per block: every wave
+// ranks its four groups of 64 frames among the lanes of their label (a ballot per bit
+// of the labels), then the waves take turns in frame order, the first lane of each
+// label moving that label's running count on.  (One wave per block that compares each
+// frame with the 63 others, a group after the other: 148 us at 250,000 frames; now
+// 10.)
+__global__ __launch_bounds__(1024) void k_lloyd_scatter(int64_t n, int k, const int32_t *__restrict__ labels,
+                                                        const int64_t *__restrict__ off,
+                                                        const int32_t *__restrict__ blk_cnt,
+                                                        int64_t *__restrict__ order, const int32_t *__restrict__ done) {
     if (*done) return;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0;
-}
-
-// Stable scatter: position of frame i = off[label] + (members of label in
-// earlier blocks) + (members in this block before i).  One wavefront per
-// block walks its frames in groups of 64 in order.
-__global__ __launch_bounds__(64) void k_lloyd_scatter(int64_t n, int k, const int32_t *__restrict__ labels,
-                                                      const int64_t *__restrict__ off,
-                                                      const int32_t *__restrict__ blk_cnt,
-                                                      int64_t *__restrict__ order, const int32_t *__restrict__ done) {
-    if (*done) return;
-    extern __shared__ int32_t s_run[];  // k running counters of this block
-    const int lane = threadIdx.x;
-    const int64_t b = blockIdx.x;
-    for (int j = lane; j < k; j += 64) s_run[j] = 0;
-    __syncthreads();
-    const int64_t lo = b * BLOCK;
-    const int32_t *bp = blk_cnt + b * (int64_t)k;
-    for (int m = 0; m < BLOCK / 64; ++m) {
-        const int64_t i = lo + m * 64 + lane;
-        const int lab = i < n ? labels[i] : -1;
-        int rank = 0;
-        for (int src = 0; src < 64; ++src) {
-            const int ol = __shfl(lab, src, 64);
-            rank += (src < lane && ol == lab) ? 1 : 0;
+    constexpr int G = BLOCK / 1024;
+    extern __shared__ int32_t s_run[];  // k running counters
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t b = blockIdx.x, lo = b * BLOCK + wave * (64 * G) + lane;
+    int lab[G], rank[G], cnt[G], lead[G];
+    int64_t start[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) lab[u] = lo + u * 64 < n ? labels[lo + u * 64] : -1;
+    for (int j = tid; j < k; j += 1024) s_run[j] = blk_cnt[b * k + j];
+    const int bits = k > 1 ? 32 - __builtin_clz((unsigned int)(k - 1)) : 0;
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+        start[u] = lab[u] >= 0 ? off[lab[u]] : 0;
+        unsigned long long same = __ballot(lab[u] >= 0);
+        for (int q = 0; q < bits; ++q) {
+            const bool bit = (lab[u] >> q) & 1;
+            const unsigned long long m = __ballot(bit);
+            same &= bit ? m : ~m;
         }
-        if (lab >= 0) order[off[lab] + bp[lab] + s_run[lab] + rank] = i;
-        __syncthreads();
-        if (lab >= 0) atomicAdd(&s_run[lab], 1);
+        rank[u] = __popcll(same & ((1ull << lane) - 1ull));
+        cnt[u] = __popcll(same);
+        lead[u] = same ? __builtin_ctzll(same) : 0;
+    }
+    __syncthreads();
+    for (int w = 0; w < 16; ++w) {
+        if (w == wave) {
+#pragma unroll
+            for (int u = 0; u < G; ++u) {
+                int base = 0;
+                if (lab[u] >= 0 && rank[u] == 0) {
+                    base = s_run[lab[u]];
+                    s_run[lab[u]] = base + cnt[u];
+                }
+                rank[u] += __shfl(base, lead[u], 64);
+            }
+        }
         __syncthreads();
     }
+#pragma unroll
+    for (int u = 0; u < G; ++u)
+        if (lab[u] >= 0) order[start[u] + rank[u]] = lo + u * 64;
 }
 
 // Chunk sums: one wavefront per chunk, lanes over dimensions, members in order.
@@ -815,12 +876,10 @@ extern "C" int emma_lloyd(const float *X, int64_t n, int32_t d, float *C, int32_
                      (reinterpret_cast<uintptr_t>(C) & 15) == 0;
     for (int it = 0; it < max_iter; ++it) {
         EMMA_TRY(assign_run(X, n, d, C, k, labels, assign_mode, nullptr, w.assign_ws, w.done, s));
-        km::k_fill_i32<<<1024, 256, 0, s>>>(w.blk_cnt, nb * (int64_t)k, w.done);
-        km::k_lloyd_dist<false, true><<<(unsigned)cdiv(n, 256), 256, 0, s>>>(X, n, d, C, k, labels, w.dist,
-                                                                            w.blk_cnt, w.done);
+        const size_t run_shm = sizeof(int32_t) * (size_t)k;
+        km::k_lloyd_hist<<<(unsigned)nb, 1024, run_shm, s>>>(n, k, labels, w.blk_cnt, w.done);
         km::k_lloyd_scan<<<1, 1024, 0, s>>>(k, nb, w.cnt, w.off, w.coff, w.blk_cnt, w.done);
-        km::k_lloyd_scatter<<<(unsigned)nb, 64, sizeof(int32_t) * k, s>>>(n, k, labels, w.off, w.blk_cnt, w.order,
-                                                                          w.done);
+        km::k_lloyd_scatter<<<(unsigned)nb, 1024, run_shm, s>>>(n, k, labels, w.off, w.blk_cnt, w.order, w.done);
         const int64_t max_chunks = n / km::CHUNK + k + 1;
         km::k_lloyd_chunks<<<(unsigned)cdiv(max_chunks, 4), 256, 0, s>>>(X, d, k, w.off, w.coff, w.order,
                                                                          w.chunk_sums, w.done);
@@ -828,11 +887,9 @@ extern "C" int emma_lloyd(const float *X, int64_t n, int32_t d, float *C, int32_
         // clusters against them and record it (which may raise the convergence flag)
         km::k_lloyd_update<<<(unsigned)cdiv(k, 4), 256, 0, s>>>(d, k, w.cnt, w.coff, w.chunk_sums, C, w.done);
         if (vec)
-            km::k_lloyd_dist<true, false><<<(unsigned)cdiv(n, 256), 256, 0, s>>>(X, n, d, C, k, labels, w.dist,
-                                                                                w.blk_cnt, w.done);
+            km::k_lloyd_dist<true><<<(unsigned)cdiv(n, 256), 256, 0, s>>>(X, n, d, C, labels, w.dist, w.done);
         else
-            km::k_lloyd_dist<false, false><<<(unsigned)cdiv(n, 256), 256, 0, s>>>(X, n, d, C, k, labels, w.dist,
-                                                                                 w.blk_cnt, w.done);
+            km::k_lloyd_dist<false><<<(unsigned)cdiv(n, 256), 256, 0, s>>>(X, n, d, C, labels, w.dist, w.done);
         km::k_block_sums<<<(unsigned)nb, 256, 0, s>>>(n, w.dist, w.bcost, w.done);
         km::k_lloyd_cost_final<<<1, 1, 0, s>>>(nb, w.bcost, tol, it, w.prev_cost, inertias, n_iter, converged,
                                                w.done);

@@ -93,3 +93,18 @@ def test_lloyd_converges_and_stops(golden_hmm):
     C, lab, inert, conv = _lloyd(X, C0, 10, 1e-5, _native.EMMA_ASSIGN_BF16X3_RECHECK)
     assert sorted(C[:, 0].tolist()) == [30.0, 60.0, 90.0, 120.0]
     assert conv and len(inert) < 10
+
+
+@pytest.mark.parametrize("n,d,k", [(1, 3, 1), (4097, 3, 1), (63, 2, 5), (4096, 4, 64), (8200, 3, 1024), (9000, 2, 1025),
+                                   (70000, 2, 2100)])
+def test_lloyd_member_order_edges(n, d, k):
+    """Label counts, offsets and the stable member order at the edges of a group of 64
+    frames, a block of 4096, 16 blocks and 1024 labels: bit-identical means and costs."""
+    rng = np.random.default_rng(n + k)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    C0 = X[rng.permutation(n)[:k]].copy()
+    C_ref, lab_ref, in_ref, _ = on.lloyd(X, C0, 3, 0.0, nthreads=4)
+    C, lab, inert, _ = _lloyd(X, C0, 3, 0.0, _native.EMMA_ASSIGN_BF16X3_RECHECK)
+    np.testing.assert_array_equal(lab, lab_ref)
+    np.testing.assert_array_equal(inert, in_ref)
+    np.testing.assert_array_equal(C, C_ref)
