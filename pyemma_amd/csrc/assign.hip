@@ -634,17 +634,19 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
         // the frame's upper bound, (na + v_j - E_j)(1 - g) <= upper, as the
         // threshold v_j - c1b|b_j|^2 - ca |b_j| - cb |lo_j| - cc rest_j <= T, raised by
         // 16 u (|a| + max|b|)^2 so that rounding only ever adds candidates; no
-        // threshold (NaN upper): no candidate, the frame goes to the full loop
+        // threshold (NaN upper, norms near overflow, and the rows past the list, whose
+        // ccnt is not set): NaN, which no value reaches (not even the -inf of an
+        // overflowed product), so no candidate, and the frame goes to the full loop
         float thr[FB], ca[FB], cb[FB], cc[FB];
         if constexpr (CAND) {
 #pragma unroll
             for (int b = 0; b < FB; ++b) {
                 const int r = b * 32 + (lane & 31);
-                thr[b] = -INFINITY;
+                thr[b] = __uint_as_float(0x7fc00000u);
                 ca[b] = cb[b] = cc[b] = 0.0f;
                 const float up = f0 + r < nf ? rl.upper[f0 + r] : __uint_as_float(0x7fc00000u);
-                if (up == up) {
-                    const double na = s_na[r], sa = sqrt(na) * (1.0 + 2e-5), mb = cp.mx[MX_BN];
+                const double na = s_na[r], sa = sqrt(na) * (1.0 + 2e-5), mb = cp.mx[MX_BN];
+                if (up == up && (sa + mb) * (sa + mb) < 1e38) {
                     const double e1 = sqrt((double)s_e1[r]) * (1.0 + 1e-4), e2 = sqrt((double)s_e2[r]) * (1.0 + 1e-4);
                     const double T = (double)up / (1.0 - (double)ce.gref) - (na - (double)ce.c1a * sa * sa) +
                                      16.0 * 5.9604644775390625e-8 * (sa + mb) * (sa + mb);

@@ -245,3 +245,26 @@ def test_tile_edges(n, d, k):
             assert t.equal(lab, ref), "variant %d: %d labels differ" % (v, int((lab != ref).sum()))
     finally:
         _native.check(L.emma_assign_select(d, k, -1), "emma_assign_select")
+
+
+@pytest.mark.parametrize("n,d,k", [(5, 1, 2), (300, 1, 2), (300, 31, 40), (3000, 300, 33), (40000, 32, 40)])
+@pytest.mark.parametrize("big", [3e38, 1e25, 1e19])
+def test_overflowing_frames_in_short_lists(n, d, k, big):
+    """Frames and a center whose squares or products overflow, in a workspace that holds
+    negative leftovers: rows past the end of a list record no candidates, and the labels
+    are those of the loop."""
+    t = _native.torch()
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    X[n // 2] = big
+    X[n - 1, d - 1] = -big
+    C = rng.standard_normal((k, d)).astype(np.float32)
+    for center in (None, big):
+        if center is not None:
+            C[k - 1] = np.float32(0.9) * np.float32(center)
+        Xt, Ct = _native.as_device_f32(X), _native.as_device_f32(C)
+        size = _native.lib().emma_assign_workspace_size(n, d, k, _native.EMMA_ASSIGN_BF16X3_RECHECK)
+        _native.workspace(size, "assign").fill_(0xC5)
+        lab = _native.assign(Xt, Ct, mode=_native.EMMA_ASSIGN_BF16X3_RECHECK)
+        ref = _native.assign(Xt, Ct, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
+        assert bool(t.equal(lab, ref))
