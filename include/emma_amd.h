@@ -147,6 +147,17 @@ int emma_assign(const float *X, int64_t n, int32_t d, const float *C, int32_t k,
                 void *stream);
 
 /*
+ * emma_assign that also reports, in n_looped (device int64, may be NULL), how many
+ * frames took the FP32 loop over all centers: every frame of
+ * EMMA_ASSIGN_FP32_PLAIN; otherwise the frames that no error bound decides, among them
+ * every frame with a NaN or an infinity.  Zero therefore says that X is finite, and the
+ * caller need not read it once more to check that.
+ */
+int emma_assign_counted(const float *X, int64_t n, int32_t d, const float *C, int32_t k, int32_t *labels,
+                        int32_t mode, int64_t *n_rechecked, int64_t *n_looped, void *workspace,
+                        size_t workspace_bytes, void *stream);
+
+/*
  * emma_assign without a workspace argument and without any allocation: no
  * counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that

@@ -63,6 +63,8 @@ def lib():
     L.emma_assign_workspace_size.argtypes = [i64, i32, i32, i32]
     L.emma_assign.restype = ctypes.c_int
     L.emma_assign.argtypes = [vp, i64, i32, vp, i32, vp, i32, vp, vp, sz, vp]
+    L.emma_assign_counted.restype = ctypes.c_int
+    L.emma_assign_counted.argtypes = [vp, i64, i32, vp, i32, vp, i32, vp, vp, vp, sz, vp]
     L.emma_assign_variants.restype = i32
     L.emma_assign_variants.argtypes = [i32]
     L.emma_assign_select.restype = ctypes.c_int
@@ -208,7 +210,7 @@ def moments_lagged(Xt, traj_offsets, lag, stride=1, skip=0, reversible=True, rem
     return w, sx, sy, Mxx, Mxy, Myy
 
 
-def assign(Xt, Ct, mode=EMMA_ASSIGN_BF16X3_RECHECK, labels=None, n_rechecked=None):
+def assign(Xt, Ct, mode=EMMA_ASSIGN_BF16X3_RECHECK, labels=None, n_rechecked=None, n_looped=None):
     t = torch()
     n, d = Xt.shape
     k = Ct.shape[0]
@@ -218,8 +220,8 @@ def assign(Xt, Ct, mode=EMMA_ASSIGN_BF16X3_RECHECK, labels=None, n_rechecked=Non
         labels = t.empty(n, dtype=t.int32, device=Xt.device)
     L = lib()
     ws = workspace(L.emma_assign_workspace_size(n, d, k, mode), "assign")
-    check(L.emma_assign(ptr(Xt), n, d, ptr(Ct), k, ptr(labels), int(mode), ptr(n_rechecked), ptr(ws), ws.numel(),
-                        stream_ptr()), "emma_assign")
+    check(L.emma_assign_counted(ptr(Xt), n, d, ptr(Ct), k, ptr(labels), int(mode), ptr(n_rechecked), ptr(n_looped),
+                                ptr(ws), ws.numel(), stream_ptr()), "emma_assign")
     return labels
 
 

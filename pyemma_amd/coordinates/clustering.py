@@ -92,16 +92,26 @@ class AbstractClustering(object):
     def output_type(self):
         return np.int32()
 
-    def _assign_device(self, dt):
-        """labels of all rows of dt (device int32)."""
+    def _assign_device(self, dt, check_finite=False):
+        """labels of all rows of dt (device int32).  check_finite: dt has not been
+        checked yet.  The bf16x3 assignment sends every non-finite frame to the loop
+        over all centers, so the rows are read once more only where a frame took it."""
         t = _native.torch()
+        mode = ASSIGN_MODES[self.assign_mode]
+        if check_finite and (mode != _native.EMMA_ASSIGN_BF16X3_RECHECK or dt.d > 512
+                             or np.shape(self.clustercenters)[1:] != (dt.d,)):
+            dt.check_finite()
+            check_finite = False
         C = _native.as_device_f32(self.clustercenters)
         if C.shape[1] != dt.d:
             raise ValueError("cluster centers have wrong dimension. Have dim=%i, but input has %i"
                              % (C.shape[1], dt.d))
-        nre = t.zeros(1, dtype=t.int64, device=dt.X.device)
-        labels = _native.assign(dt.X, C, mode=ASSIGN_MODES[self.assign_mode], n_rechecked=nre)
-        self.n_rechecked = int(nre.item())
+        counts = t.zeros(2, dtype=t.int64, device=dt.X.device)
+        labels = _native.assign(dt.X, C, mode=mode, n_rechecked=counts[:1], n_looped=counts[1:])
+        n_rechecked, n_looped = counts.tolist()
+        if check_finite and n_looped:
+            dt.check_finite()
+        self.n_rechecked = n_rechecked
         return labels
 
     def _assign_source(self, src):
@@ -134,16 +144,16 @@ class AbstractClustering(object):
             labs = self._assign_source(X)
             off = np.concatenate([[0], np.cumsum([len(l) for l in labs])]).astype(np.int64)
             return DeviceDtrajs(t.cat(labs).contiguous(), off)
-        dt = to_device(X)
-        return DeviceDtrajs(self._assign_device(dt), dt.offsets)
+        dt = to_device(X, check_finite=False)
+        return DeviceDtrajs(self._assign_device(dt, check_finite=True), dt.offsets)
 
     def transform(self, X):
         """(T, 1) int32 label columns (interface.py:157-167)."""
         if isinstance(X, FeatureSource):
             return [l.cpu().numpy()[:, None] for l in self._assign_source(X)]
         single = not isinstance(X, (list, tuple, DeviceTrajectories))
-        dt = to_device(X)
-        out = [l[:, None] for l in dt.split(self._assign_device(dt))]
+        dt = to_device(X, check_finite=False)
+        out = [l[:, None] for l in dt.split(self._assign_device(dt, check_finite=True))]
         return out[0] if single and dt.ntraj == 1 else out
 
     def get_output(self, stride=1, skip=0, chunk=None):

@@ -163,8 +163,17 @@ class LaggedCovariance(object):
     def _device_moments(self, dt, skip=None):
         return self._moments_finish(self._moments_launch(dt, skip=skip))
 
-    def _moments_finish(self, dev):
-        """Host FP64 moments of a launched call, with the constant-mean shift."""
+    def _sums_cover(self, dt):
+        """Whether the column sums of a moments call take in every row of dt: rows
+        [0, T - lag) and [lag, T) of each trajectory, without weights."""
+        return (self.weights is None and self.stride == 1 and self.skip == 0 and dt.ntraj > 0
+                and (self.lag == 0 or self.c0t) and min(dt.lengths) > self.lag and min(dt.lengths) >= 2 * self.lag)
+
+    def _moments_finish(self, dev, unchecked=None):
+        """Host FP64 moments of a launched call, with the constant-mean shift.
+        unchecked: trajectories not yet checked for non-finite values, all of whose rows
+        are in the sums.  A NaN or an infinity stays in its column's sum, so the rows
+        are read once more only if a sum is not finite."""
         lag = self.lag
         w, sx, sy, Mxx, Mxy, Myy = dev
         h = lambda t: None if t is None else t.cpu().numpy()
@@ -172,6 +181,8 @@ class LaggedCovariance(object):
         sx, sy, Mxx, Mxy, Myy = h(sx), h(sy), h(Mxx), h(Mxy), h(Myy)
         if lag == 0 or (self.c00 and not self.c0t and not self.ctt):
             sy = sx
+        if unchecked is not None and not (np.isfinite(sx).all() and np.isfinite(sy).all()):
+            unchecked.check_finite()
         c = self.remove_constant_mean
         if c is not None:
             # moments of (x - c): exact algebra on the unshifted FP64 sums
@@ -233,7 +244,12 @@ class LaggedCovariance(object):
 
         if isinstance(data, FeatureSource):
             return self._estimate_source(data, partial_fit=partial_fit)
-        dt = to_device(data)
+        dt = to_device(data, check_finite=False)
+        moments = None
+        if self._sums_cover(dt):
+            moments = self._moments_finish(self._moments_launch(dt), unchecked=dt)
+        else:
+            dt.check_finite()
         usable = [n for n in dt.lengths if n > self.lag + self.skip]
         if not usable:
             longest = int(max(dt.lengths) if dt.ntraj else 0)
@@ -245,7 +261,7 @@ class LaggedCovariance(object):
                              % (longest, self.lag + self.skip))
         if self._rc is None or not partial_fit:
             self._init_storage(len(usable))
-        self._store(*self._device_moments(dt))
+        self._store(*(moments if moments is not None else self._device_moments(dt)))
         self._estimated = True
         return self
 

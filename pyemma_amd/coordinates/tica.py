@@ -117,8 +117,11 @@ class TICA(object):
             elif hasattr(self, k):
                 setattr(self, k, v)
         # a FeatureSource is streamed chunk by chunk (its features never all exist at once)
-        dt = X if isinstance(X, FeatureSource) else to_device(X)
+        # the covariance estimate checks its input
+        dt = X if isinstance(X, FeatureSource) else to_device(X, check_finite=False)
         if not self.dim <= dt.d:
+            if not isinstance(X, FeatureSource):
+                dt.check_finite()
             raise RuntimeError("requested more output dimensions (%i) than dimension of input data (%i)"
                                % (self.dim, dt.d))
         covar = self._new_covar()
@@ -245,20 +248,32 @@ class TICA(object):
         Vd = t.as_tensor(np.ascontiguousarray(V, dtype=np.float64), device=dt.X.device)
         return _native.project(dt.X, mean, Vd, m)
 
+    def _project_checked(self, dt):
+        """Projection of trajectories not yet checked for non-finite values.  A NaN or an
+        infinity in a row makes every output of that row NaN or infinite (FP64 products
+        and sums over all columns, one rounding), so the outputs are checked, and the
+        rows read once more only if one of them is not finite."""
+        if dt.d != np.size(self.mean) or self.dimension() < 1:
+            dt.check_finite()
+            return self._project_device(dt)
+        Y = self._project_device(dt)
+        if int(_native.count_nonfinite(Y).item()):
+            dt.check_finite()
+        return Y
+
     def transform(self, X):
         """Project X (ndarray or list) onto the leading components (_tica_base.py:117-133)."""
         if isinstance(X, FeatureSource):
             return [y.cpu().numpy() for y in X.per_trajectory(self._project_device)]
         single = isinstance(X, np.ndarray) or (not isinstance(X, (list, tuple, DeviceTrajectories)))
-        dt = to_device(X)
-        Y = self._project_device(dt)
+        dt = to_device(X, check_finite=False)
+        Y = self._project_checked(dt)
         out = dt.split(Y)
         return out[0] if single and dt.ntraj == 1 else out
 
     def transform_device(self, X):
         """Projection kept on the device: (DeviceTrajectories in) -> torch tensor (N, m)."""
-        dt = to_device(X)
-        return self._project_device(dt)
+        return self._project_checked(to_device(X, check_finite=False))
 
     def get_output(self, dimensions=slice(0, None), stride=1, skip=0, chunk=None):
         """Projected estimation data, one array per trajectory."""

@@ -277,7 +277,9 @@ class VAMP(object):
                 self.chunksize = value
             elif hasattr(self, name):
                 setattr(self, name, value)
-        dt = to_device(X)
+        dt = to_device(X, check_finite=False)  # the covariance estimate checks its input
+        if isinstance(self.dim, int) and self.dim > dt.d:
+            dt.check_finite()
         self._check_dim(dt)
         covar = self._estimator()
         covar.estimate(dt)

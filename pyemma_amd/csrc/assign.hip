@@ -51,8 +51,11 @@ __global__ __launch_bounds__(256) void k_assign_plain(const float *__restrict__ 
                                                       const int64_t *__restrict__ list_count,
                                                       int64_t *__restrict__ n_rechecked,
                                                       const int64_t *__restrict__ n_listed,
+                                                      int64_t *__restrict__ n_looped,
                                                       const int32_t *__restrict__ done) {
     if (done && *done) return;
+    // the call's count of frames that this loop takes
+    if (n_looped && blockIdx.x == 0 && threadIdx.x == 0) *n_looped = list ? *list_count : n;
     // the call's count of re-evaluated frames (0 for the loop over every frame)
     if (n_rechecked && blockIdx.x == 0 && threadIdx.x == 0) *n_rechecked = n_listed ? *n_listed : 0;
     __shared__ __align__(16) float xs[PD][PPITCH];
@@ -1169,12 +1172,12 @@ static void launch_mfma_ks(const TileArgs &a, const AssignWs &w, const AsgCoef &
 size_t assign_workspace_bytes(int64_t n, int d, int k, int mode) { return asg::carve_assign(nullptr, n, d, k, mode).bytes; }
 
 int assign_run(const float *X, int64_t n, int d, const float *C, int k, int32_t *labels, int mode,
-               int64_t *n_rechecked, void *workspace, const int32_t *done, hipStream_t s) {
+               int64_t *n_rechecked, int64_t *n_looped, void *workspace, const int32_t *done, hipStream_t s) {
     using namespace asg;
     AssignWs w = carve_assign(workspace, n, d, k, mode);
     if (mode == EMMA_ASSIGN_FP32_PLAIN) {
         k_assign_plain<<<(unsigned)cdiv(n, PF), 256, 0, s>>>(X, n, d, C, k, labels, nullptr, nullptr, n_rechecked,
-                                                             nullptr, done);
+                                                             nullptr, n_looped, done);
         return check_launch("assign plain");
     }
     const int ks = pick_ksteps(d);
@@ -1210,7 +1213,7 @@ int assign_run(const float *X, int64_t n, int d, const float *C, int k, int32_t 
     EMMA_TRY(check_launch("assign candidate recheck"));
     const int64_t rb = cdiv(n, PF) < 1024 ? cdiv(n, PF) : 1024;
     k_assign_plain<<<(unsigned)rb, 256, 0, s>>>(X, n, d, C, k, labels, w.rl.list2, w.rl.count + 2, n_rechecked,
-                                                w.rl.count, done);
+                                                w.rl.count, n_looped, done);
     return check_launch("assign recheck");
 }
 
@@ -1226,6 +1229,12 @@ extern "C" size_t emma_assign_workspace_size(int64_t n, int32_t d, int32_t k, in
 extern "C" int emma_assign(const float *X, int64_t n, int32_t d, const float *C, int32_t k, int32_t *labels,
                            int32_t mode, int64_t *n_rechecked, void *workspace, size_t workspace_bytes,
                            void *stream) {
+    return emma_assign_counted(X, n, d, C, k, labels, mode, n_rechecked, nullptr, workspace, workspace_bytes, stream);
+}
+
+extern "C" int emma_assign_counted(const float *X, int64_t n, int32_t d, const float *C, int32_t k, int32_t *labels,
+                                   int32_t mode, int64_t *n_rechecked, int64_t *n_looped, void *workspace,
+                                   size_t workspace_bytes, void *stream) {
     EMMA_REQUIRE(n >= 0 && d > 0 && k > 0, "emma_assign: bad sizes n=%lld d=%d k=%d", (long long)n, d, k);
     EMMA_REQUIRE(mode == EMMA_ASSIGN_FP32_PLAIN || mode == EMMA_ASSIGN_BF16X3_RECHECK,
                  "emma_assign: unknown mode %d", mode);
@@ -1234,7 +1243,7 @@ extern "C" int emma_assign(const float *X, int64_t n, int32_t d, const float *C,
     const size_t need = assign_workspace_bytes(n, d, k, mode);
     EMMA_REQUIRE(workspace && workspace_bytes >= need, "emma_assign: workspace too small (%zu < %zu)",
                  workspace_bytes, need);
-    return assign_run(X, n, d, C, k, labels, mode, n_rechecked, workspace, nullptr, (hipStream_t)stream);
+    return assign_run(X, n, d, C, k, labels, mode, n_rechecked, n_looped, workspace, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int32_t emma_assign_variants(int32_t d) {
@@ -1313,7 +1322,7 @@ extern "C" int emma_assign_noalloc(const float *X, int64_t n, int32_t d, const f
     EMMA_REQUIRE(X && C && labels, "emma_assign_noalloc: NULL pointer");
     hipStream_t s = (hipStream_t)stream;
     if (mode == EMMA_ASSIGN_FP32_PLAIN)  // the plain loop needs no workspace
-        return assign_run(X, n, d, C, k, labels, mode, n_rechecked, nullptr, nullptr, s);
+        return assign_run(X, n, d, C, k, labels, mode, n_rechecked, nullptr, nullptr, nullptr, s);
     // the center images and constants take a fixed part of the scratch; the
     // recheck arrays (56 bytes per frame) the rest, so the frames run
     // in chunks
@@ -1337,7 +1346,7 @@ extern "C" int emma_assign_noalloc(const float *X, int64_t n, int32_t d, const f
     const AssignWs w = carve_assign(ws, chunk, d, k, mode);
     for (int64_t f0 = 0; f0 < n; f0 += chunk) {
         const int64_t m = n - f0 < chunk ? n - f0 : chunk;
-        EMMA_TRY(assign_run(X + f0 * (int64_t)d, m, d, C, k, labels + f0, mode, nullptr, ws, nullptr, s));
+        EMMA_TRY(assign_run(X + f0 * (int64_t)d, m, d, C, k, labels + f0, mode, nullptr, nullptr, ws, nullptr, s));
         if (n_rechecked) k_add_i64<<<1, 1, 0, s>>>(n_rechecked, w.rl.count);
     }
     return check_launch("emma_assign_noalloc");
