@@ -119,3 +119,24 @@ def test_out_of_range_raises():
     with pytest.raises(ValueError):
         pd.DiscreteTrajectoryStats([np.array([0, -3], dtype=np.int32)])
     assert pd.number_of_states([np.array([3, 1], dtype=np.int32), np.array([7], dtype=np.int32)]) == 8
+
+
+@pytest.mark.parametrize("n", [131071, 131072, 131073, 400001])
+@pytest.mark.parametrize("k", [1, 1000, 8192, 8193])
+def test_histogram_in_lds(n, k):
+    """Histogram and out-of-range count around the sizes where the histogram moves to LDS,
+    with unassigned frames, states out of range, and one long run."""
+    from pyemma_amd import _native
+
+    t = _native.torch()
+    rng = np.random.default_rng(n + k)
+    S = rng.integers(0, k, n).astype(np.int32)
+    S[1000:70000] = k - 1
+    S[rng.integers(0, n, 500)] = -1
+    S[rng.integers(0, n, 40)] = k
+    S[5], S[n - 1] = -2, -1
+    St = t.from_numpy(S).cuda()
+    _, H, bad = _native.count_transitions(St, np.array([0, n]), 3, True, k)
+    ok = (S >= 0) & (S < k)
+    np.testing.assert_array_equal(H.cpu().numpy(), np.bincount(S[ok], minlength=k))
+    assert int(bad.item()) == int(((S < -1) | (S >= k)).sum())

@@ -88,3 +88,17 @@ def test_projection(d, m):
     Y = X.copy()
     Y[5] = 3e38
     assert tica.transform(Y).shape == (2000, m)
+
+
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 8, 63, 1029, 40007])
+def test_count_at_every_alignment(n, shift):
+    t = _native.torch()
+    buf = t.full((n + shift + 8,), float("nan"), device="cuda")
+    x = buf[shift:shift + n]
+    x.zero_()
+    assert int(_native.count_nonfinite(x).item()) == 0
+    where = sorted({0, n // 2, max(n - 4, 0), n - 1})
+    for i, w in enumerate(where):
+        x[w] = BAD[i % 3]
+        assert int(_native.count_nonfinite(x).item()) == i + 1
