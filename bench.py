@@ -73,10 +73,12 @@ def mom_executed_flops(d, P):
     return nb * (nb + 1) // 2 * 64 * 64 * 2 * 4 * 2 * float(P)
 
 
-def asg_first_pass_products(variant):
+def asg_first_pass_products(d, variant):
     """MFMA products per dimension of the assignment's first pass: 1 for the
-    coarse fp16 pass (variant 0, the default), 3 for the bf16 split (variant 1)."""
-    return 1 if not variant else 3
+    coarse fp16 pass (the lower half of the variants), 3 for the bf16 split."""
+    from pyemma_amd import _native
+
+    return 3 if variant and variant >= _native.lib().emma_assign_variants(d) // 2 else 1
 
 
 def asg_executed_flops(d, k, n, products=3):
@@ -266,7 +268,7 @@ def main():
         cpu, par = cpu_baseline(args, X, offsets, C, labels, mats)
         parity.update(par)
     kern["moments"]["executed_tflop"] = mom_executed_flops(d, P) / 1e12
-    kern["assign"]["executed_tflop"] = asg_executed_flops(d, args.k, N, asg_first_pass_products(best)) / 1e12
+    kern["assign"]["executed_tflop"] = asg_executed_flops(d, args.k, N, asg_first_pass_products(d, best)) / 1e12
     ex = kern[dom]["executed_tflop"] * 1e12 / (kern[dom]["ms"] * 1e-3) / 1e12
     roofline.update({"executed_tflops": ex, "executed_frac": ex / PEAK_BF16_TFLOPS})
 
@@ -582,7 +584,7 @@ def large_k_leg(args, n=10_000_000, d=512, k=4096, n_seed=200_000, iters=5, n_pl
     ms_ll = _timed(run_lloyd, reps=1)
     n_iter = int(res["out"][2].item())
     f_asg = 2.0 * d * k * n
-    ex_asg = asg_executed_flops(d, k, n, asg_first_pass_products(variant))
+    ex_asg = asg_executed_flops(d, k, n, asg_first_pass_products(d, variant))
     ach = f_asg / (ms_asg * 1e-3) / 1e12
     pp_bytes = (4 * d + 8) * n_seed * (k - 1)
     out = {"workload": "%d x %d f32 Gaussian mixture, k=%d" % (n, d, k),
@@ -683,7 +685,7 @@ def batched_leg(args, ntraj=4096, d=128, lag=5, k=512, n_seed=1_000_000, n_plain
                       "hbm_frac": asg_bytes / (ms_asg * 1e-3) / 1e9 / PEAK_HBM_GBS,
                       "rechecked_frames": int(nre.item()),
                       "executed_frac": asg_executed_flops(d, k, N, asg_first_pass_products(
-                          autotune.tuned().get(autotune._bucket(d, k), (None,))[0])) / (ms_asg * 1e-3) / 1e12
+                          d, autotune.tuned().get(autotune._bucket(d, k), (None,))[0])) / (ms_asg * 1e-3) / 1e12
                                        / PEAK_BF16_TFLOPS}}
     # parity
     lab_plain = torch.empty(n_plain, dtype=torch.int32, device=dev)

@@ -4,7 +4,7 @@ The MFMA assignment exists in a few variants (emma_assign_variants): a coarse
 fp16 pass with the fine pass on the frames it leaves, or the fine pass over
 every frame.  Which one is faster depends on the dimension, the number of
 centers and the data (how many frames the coarse bound leaves).  The
-first call for a (dimension, center count) bucket times every variant on a
+first call for a (dimension, center count) bucket times both on a
 sample of the caller's own frames (up to 2^21 frames: smaller samples fill
 the device for only a few rounds, where the variants tie and the full-size
 winner is not visible) with HIP events on the current stream,
@@ -19,7 +19,7 @@ from . import _native
 __all__ = ["tune_assign", "tuned"]
 
 _lock = threading.Lock()
-_tuned = {}  # (ks, k bucket) -> (variant, [ms per variant])
+_tuned = {}  # (ks, k bucket) -> (variant, [ms of the coarse, of the fine pipeline])
 
 
 def _bucket(d, k):
@@ -58,7 +58,8 @@ def tune_assign(Xt, Ct, mode=_native.EMMA_ASSIGN_BF16X3_RECHECK, sample=2097152,
         Xs = Xt[: min(n, sample)]
         lab = t.empty(Xs.shape[0], dtype=t.int32, device=Xt.device)
         times = []
-        for v in range(nv):
+        variants = (0, nv // 2)  # the first number of each pipeline
+        for v in variants:
             _native.check(L.emma_assign_select(d, k, v), "emma_assign_select")
             _native.assign(Xs, Ct, mode=mode, labels=lab)  # warm-up
             e0, e1 = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
@@ -68,7 +69,7 @@ def tune_assign(Xt, Ct, mode=_native.EMMA_ASSIGN_BF16X3_RECHECK, sample=2097152,
             e1.record()
             e1.synchronize()
             times.append(e0.elapsed_time(e1) / reps)
-        best = min(range(nv), key=lambda i: times[i])
+        best = variants[times.index(min(times))]
         _native.check(L.emma_assign_select(d, k, best), "emma_assign_select")
         _tuned[key] = (best, times)
         return best

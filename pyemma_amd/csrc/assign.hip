@@ -1023,12 +1023,14 @@ __global__ __launch_bounds__(256) void k_assign_cand_exact(const float *__restri
 }
 
 // First-pass pipelines, timed by the autotuner (emma_assign_select may pick one
-// per (K steps, k) bucket): variant 0, the default, is the coarse pass over
-// every frame with the fine pass on what it leaves; variant 1 the fine pass
-// over every frame.  Which is faster depends on d, k and the data: the coarse
-// pass costs a third of the fine one's products, so it loses only where its
-// bound leaves about two thirds of the frames or more.
-static int n_variants(int) { return 2; }
+// per (K steps, k) bucket): the lower half of the variant numbers (0 is the
+// default) is the coarse pass over every frame with the fine pass on what it
+// leaves; the upper half the fine pass over every frame.  Which is faster depends
+// on d, k and the data: the coarse pass costs a third of the fine one's products,
+// so it loses only where its bound leaves about two thirds of the frames or more.
+// Each pipeline has one tile shape; the count of numbers per dimension is part of
+// the C ABI, so that selections kept by a caller stay valid.
+static int n_variants(int ks) { return ks <= 4 ? 12 : ks <= 8 ? 6 : ks <= 19 ? 4 : 2; }
 
 // process-wide selection table: [K-step class][ceil(log2(k_pad / 32))]
 static std::mutex g_sel_mu;
@@ -1157,7 +1159,7 @@ static void launch_pass(const TileArgs &a, const AssignWs &w, const AsgCoef &ce)
 
 template <int KS>
 static void launch_mfma_ks(const TileArgs &a, const AssignWs &w, const AsgCoef &ce, const AsgCoef &ce16) {
-    if (selected_variant(KS, a.k_pad) == 0) {
+    if (selected_variant(KS, a.k_pad) < n_variants(KS) / 2) {
         launch_pass<KS, PASS_COARSE>(a, w, ce16);
         launch_pass<KS, PASS_FINE>(a, w, ce);
     } else {
