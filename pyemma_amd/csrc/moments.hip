@@ -1579,7 +1579,9 @@ __global__ __launch_bounds__(512, 2) void k_tri(Params p) {
 
 // ------------------------------------------------------------------
 // frame weights: sum of the weights of every trajectory's pairs, then the
-// total (both in a fixed order)
+// total (both in a fixed order).  One workgroup per trajectory: the longest one's chain of
+// loads is the time, so 16 of a thread's weights are loaded before their in-order adds
+// (2 10^6 frames in 60 ragged trajectories: 270 us with one at a time, 49 now).
 // ------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_wsum(Params p) {
     __shared__ double s_part[256];
@@ -1588,7 +1590,18 @@ __global__ __launch_bounds__(256) void k_wsum(Params p) {
     const int64_t base = p.traj_off[t] + p.skip;
     double a = 0.0;
     const int64_t q0 = p.pair_off[t];
-    for (int64_t i = tid; i < np; i += 256) {
+    int64_t i = tid;
+    for (; i + 15 * 256 < np; i += 16 * 256) {
+        double wv[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) wv[u] = p.wts[base + (i + u * 256) * p.stride];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            a += wv[u];
+            p.wpair[q0 + i + u * 256] = (float)wv[u];
+        }
+    }
+    for (; i < np; i += 256) {
         const double wv = p.wts[base + i * p.stride];
         a += wv;
         p.wpair[q0 + i] = (float)wv;
