@@ -484,14 +484,13 @@ def kmeans_leg(args, X, sub, cpu=True, seed=12345, n_lloyd=1_000_000, iters=5, n
 
     ms_ll = _timed(run_lloyd, reps=1)
     n_iter = int(res["out"][2].item())
-    pp_bytes = (4 * d + 8) * n * (k - 1)
+    pp_bytes = (4 * d + 8) * n * (k - 1)  # if every round read every frame; it reads fewer
     f_ll = 2.0 * d * k * Xl.shape[0] * n_iter
-    out = {"kmeanspp": {"frames": n, "dim": d, "k": k, "ms": ms_pp, "bytes": pp_bytes,
-                        "gbs": pp_bytes / (ms_pp * 1e-3) / 1e9, "hbm_frac": pp_bytes / (ms_pp * 1e-3) / 8e12},
+    out = {"kmeanspp": {"frames": n, "dim": d, "k": k, "ms": ms_pp, "full_pass_bytes": pp_bytes},
            "lloyd": {"frames": int(Xl.shape[0]), "dim": d, "k": k, "iterations": n_iter, "ms": ms_ll,
                      "ms_per_iteration": ms_ll / max(n_iter, 1), "assign_tflops": f_ll / (ms_ll * 1e-3) / 1e12}}
-    log("kmeans++ k=%d on %d frames %.1f ms (%.0f GB/s); lloyd %d iterations on %d frames %.1f ms"
-        % (k, n, ms_pp, out["kmeanspp"]["gbs"], n_iter, Xl.shape[0], ms_ll))
+    log("kmeans++ k=%d on %d frames %.1f ms; lloyd %d iterations on %d frames %.1f ms"
+        % (k, n, ms_pp, n_iter, Xl.shape[0], ms_ll))
     if cpu:
         from oracle import native as on
 
@@ -586,10 +585,9 @@ def large_k_leg(args, n=10_000_000, d=512, k=4096, n_seed=200_000, iters=5, n_pl
     f_asg = 2.0 * d * k * n
     ex_asg = asg_executed_flops(d, k, n, asg_first_pass_products(d, variant))
     ach = f_asg / (ms_asg * 1e-3) / 1e12
-    pp_bytes = (4 * d + 8) * n_seed * (k - 1)
+    pp_bytes = (4 * d + 8) * n_seed * (k - 1)  # if every round read every frame; it reads fewer
     out = {"workload": "%d x %d f32 Gaussian mixture, k=%d" % (n, d, k),
-           "kmeanspp": {"frames": n_seed, "k": k, "ms": ms_pp, "bytes": pp_bytes,
-                        "gbs": pp_bytes / (ms_pp * 1e-3) / 1e9},
+           "kmeanspp": {"frames": n_seed, "k": k, "ms": ms_pp, "full_pass_bytes": pp_bytes},
            "assign": {"ms": ms_asg, "algorithmic_tflop": f_asg / 1e12, "tflops": ach,
                       "executed_tflop": ex_asg / 1e12, "rechecked_frames": n_re, "tile_variant": variant,
                       "roofline": {"bound": "mfma", "achieved": ach, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
