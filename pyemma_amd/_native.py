@@ -130,18 +130,37 @@ def ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
-_ws_cache = {}
+class Workspaces(object):
+    """Device scratch buffers, one per tag, kept for reuse and replaced by a larger one
+    on demand (the smaller one is then free for other tensors)."""
+
+    def __init__(self):
+        self.buffers = {}
+
+    def get(self, nbytes, tag):
+        t = torch()
+        nbytes = max(int(nbytes), 256)
+        buf = self.buffers.get(tag)
+        if buf is None or buf.numel() < nbytes:
+            buf = t.empty(nbytes, dtype=t.uint8, device=device())
+            self.buffers[tag] = buf
+        return buf
 
 
-def workspace(nbytes, tag="default"):
-    """Reusable device scratch buffer (grown on demand, per tag)."""
+_ws_cache = Workspaces()
+
+
+def workspace(nbytes, tag="default", own=None):
+    """Device scratch buffer: of `own` if the caller keeps its Workspaces, else the shared
+    one of this tag.  A call that is being captured into a graph without its own gets a
+    buffer from the graph's memory pool: the graph goes on using the address after a later
+    call has replaced the shared buffer, and that pool lives as long as the graph."""
+    if own is not None:
+        return own.get(nbytes, tag)
     t = torch()
-    nbytes = max(int(nbytes), 256)
-    buf = _ws_cache.get(tag)
-    if buf is None or buf.numel() < nbytes:
-        buf = t.empty(nbytes, dtype=t.uint8, device=device())
-        _ws_cache[tag] = buf
-    return buf
+    if t.cuda.is_current_stream_capturing():
+        return t.empty(max(int(nbytes), 256), dtype=t.uint8, device=device())
+    return _ws_cache.get(nbytes, tag)
 
 
 def as_device_f32(X):
@@ -168,10 +187,11 @@ def count_nonfinite(Xt):
 
 
 def moments_lagged(Xt, traj_offsets, lag, stride=1, skip=0, reversible=True, remove_mean=True, c0t=True,
-                   ctt=False, precision=EMMA_PREC_BF16X4, weights=None):
+                   ctt=False, precision=EMMA_PREC_BF16X4, weights=None, workspaces=None):
     """Unnormalized FP64 moments (w, sx, sy, Mxx, Mxy, Myy) as device tensors.
 
     weights: optional FP64 device tensor with one frame weight per row of Xt.
+    workspaces: the caller's own scratch buffers (None: the shared ones).
     """
     t = torch()
     n_rows, d = Xt.shape
@@ -195,7 +215,7 @@ def moments_lagged(Xt, traj_offsets, lag, stride=1, skip=0, reversible=True, rem
         weights = weights.contiguous()
     L = lib()
     ws_bytes = L.emma_moments_workspace_size(n_rows, d, ntraj, flags, precision)
-    ws = workspace(ws_bytes, "moments")
+    ws = workspace(ws_bytes, "moments", workspaces)
     f64 = dict(dtype=t.float64, device=Xt.device)
     w = t.empty(1, **f64)
     sx = t.empty(d, **f64)
@@ -210,7 +230,8 @@ def moments_lagged(Xt, traj_offsets, lag, stride=1, skip=0, reversible=True, rem
     return w, sx, sy, Mxx, Mxy, Myy
 
 
-def assign(Xt, Ct, mode=EMMA_ASSIGN_BF16X3_RECHECK, labels=None, n_rechecked=None, n_looped=None):
+def assign(Xt, Ct, mode=EMMA_ASSIGN_BF16X3_RECHECK, labels=None, n_rechecked=None, n_looped=None,
+           workspaces=None):
     t = torch()
     n, d = Xt.shape
     k = Ct.shape[0]
@@ -219,7 +240,7 @@ def assign(Xt, Ct, mode=EMMA_ASSIGN_BF16X3_RECHECK, labels=None, n_rechecked=Non
     if labels is None:
         labels = t.empty(n, dtype=t.int32, device=Xt.device)
     L = lib()
-    ws = workspace(L.emma_assign_workspace_size(n, d, k, mode), "assign")
+    ws = workspace(L.emma_assign_workspace_size(n, d, k, mode), "assign", workspaces)
     check(L.emma_assign_counted(ptr(Xt), n, d, ptr(Ct), k, ptr(labels), int(mode), ptr(n_rechecked), ptr(n_looped),
                                 ptr(ws), ws.numel(), stream_ptr()), "emma_assign")
     return labels

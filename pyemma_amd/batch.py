@@ -15,7 +15,9 @@ autotuner pick the tile shapes for these sizes), then captures it into a HIP
 graph; replay() re-issues the whole sequence with one call.  The graph reads
 the input buffers in place, so new frames of the same shape can be copied
 into `X` between replays.  Nothing inside the sequence allocates memory, uses
-a memset node or synchronizes the host.
+a memset node or synchronizes the host.  The scratch buffers belong to the
+plan: the graph holds their addresses, so they stay in place however much the
+calls made between replays need.
 """
 import numpy as np
 
@@ -55,11 +57,14 @@ class BatchedDiscretizer(object):
         self.n_rechecked = t.zeros(1, dtype=t.int64, device=dev)
         self.graph = None
         self.out = None
+        self._workspaces = _native.Workspaces()
 
     def _sequence(self):
         self.out = _native.moments_lagged(self.X, self.offsets, self.lag, reversible=self.reversible,
-                                          remove_mean=True, c0t=True, precision=self.precision)
-        _native.assign(self.X, self.C, mode=self.assign_mode, labels=self.labels, n_rechecked=self.n_rechecked)
+                                          remove_mean=True, c0t=True, precision=self.precision,
+                                          workspaces=self._workspaces)
+        _native.assign(self.X, self.C, mode=self.assign_mode, labels=self.labels, n_rechecked=self.n_rechecked,
+                       workspaces=self._workspaces)
 
     def run_eager(self):
         """One uncaptured pass (tunes tile shapes on first use); returns host results."""
@@ -76,6 +81,9 @@ class BatchedDiscretizer(object):
         with t.cuda.graph(g):
             self._sequence()
         self.graph = g
+        # everything whose address the graph holds
+        self._captured = (self.X, self.offsets, self.C, self.labels, self.n_rechecked,
+                          tuple(self._workspaces.buffers.values()))
         return self
 
     def replay(self):

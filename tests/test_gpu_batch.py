@@ -62,3 +62,31 @@ def test_batched_graph_replay_matches_eager_and_oracle():
     assert r[0] == e[0]
     for x, y in zip(r[1:], e[1:]):
         assert np.array_equal(x, y)
+
+
+def test_replay_after_larger_calls():
+    """Larger assignment and moments calls after the capture replace the shared scratch
+    buffers: the replays still give the eager results and write into no other tensor."""
+    t = _native.torch()
+    X, off = langevin_trajectories(12, 40, lmin=200, lmax=900, seed=8)
+    C = X[::37].cpu().numpy()[:60].copy()
+    b = BatchedDiscretizer(X, off, 5, C)
+    ref = b.run_eager()
+    b.capture()
+    g = t.Generator(device="cuda").manual_seed(1)
+    big = t.randn((300_000, 40), generator=g, device="cuda")
+    _native.assign(big, big[:500].contiguous())
+    _native.moments_lagged(big, np.array([0, len(big)]), 5, precision=_native.EMMA_PREC_BF16X4_ACC)
+    t.cuda.synchronize()
+    # tensors of many sizes, over whatever the calls above gave back
+    others = [t.full((1 << p,), 17, dtype=t.uint8, device="cuda") for p in range(12, 26) for _ in range(4)]
+    for i in range(3):
+        b.labels.fill_(-5)
+        b.replay()
+        t.cuda.synchronize()
+        r = b.results()
+        assert r[0] == ref[0]
+        for x, y in zip(r[1:], ref[1:]):
+            assert np.array_equal(x, y), "replay %d" % i
+        assert all(bool((o == 17).all()) for o in others), "replay %d wrote into another tensor" % i
+        _native.assign(big[:1000], big[:500].contiguous())
