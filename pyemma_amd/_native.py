@@ -5,8 +5,10 @@ visible, every entry point raises instead of falling back to anything else.
 Device buffers are torch tensors (plumbing only); pointers and the current
 HIP stream are handed to the C ABI.
 """
+import collections
 import ctypes
 import os
+import threading
 
 import numpy as np
 
@@ -147,20 +149,45 @@ class Workspaces(object):
         return buf
 
 
-_ws_cache = Workspaces()
+class _SharedWorkspaces(threading.local):
+    """The buffers that calls without their own share: one set per host thread and stream.
+    Calls on two streams may run at the same time, and the launches of calls from two
+    threads may interleave on one stream; a buffer is allocated on the stream that uses
+    it, so a dropped one is reused in that stream's order.  The least recently used sets
+    beyond MAX_STREAMS are dropped, all of a thread's when it ends."""
+
+    MAX_STREAMS = 16
+
+    def __init__(self):
+        self.sets = collections.OrderedDict()
+
+    def current(self):
+        t = torch()
+        key = (t.cuda.current_device(), t.cuda.current_stream().cuda_stream)
+        ws = self.sets.pop(key, None)
+        if ws is None:
+            ws = Workspaces()
+        self.sets[key] = ws
+        while len(self.sets) > self.MAX_STREAMS:
+            self.sets.popitem(last=False)
+        return ws
+
+
+_shared = _SharedWorkspaces()
 
 
 def workspace(nbytes, tag="default", own=None):
-    """Device scratch buffer: of `own` if the caller keeps its Workspaces, else the shared
-    one of this tag.  A call that is being captured into a graph without its own gets a
-    buffer from the graph's memory pool: the graph goes on using the address after a later
-    call has replaced the shared buffer, and that pool lives as long as the graph."""
+    """Device scratch buffer: of `own` if the caller keeps its Workspaces, else the one of
+    this tag that the calls of this thread on the current stream share.  A call that is
+    being captured into a graph without its own gets a buffer from the graph's memory pool:
+    the graph goes on using the address after a later call has replaced the shared buffer,
+    and that pool lives as long as the graph."""
     if own is not None:
         return own.get(nbytes, tag)
     t = torch()
     if t.cuda.is_current_stream_capturing():
         return t.empty(max(int(nbytes), 256), dtype=t.uint8, device=device())
-    return _ws_cache.get(nbytes, tag)
+    return _shared.current().get(nbytes, tag)
 
 
 def as_device_f32(X):
