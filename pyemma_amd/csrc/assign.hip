@@ -832,7 +832,11 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
         // pass.  d_j >= |a|^2 + m2 - E_max for j != best, with E_max from the
         // largest norms of all centers, and d_best <= |a|^2 + m1 + E_best (both
         // through the reference loop's relative rounding g).  Anything not
-        // finite (frames, centers, fp16 overflow) fails the comparison.
+        // finite (frames, centers, fp16 overflow) fails the comparison, except a
+        // center whose |b|^2 overflows: its v is +inf, or no number once it holds an
+        // element index, and from the latter m1 is -inf and m2 may be lost.  So a
+        // frame is decided only where no v, partial sums included, can overflow:
+        // all are below (|a| + max|b|)^2.
         if (tid < F) {
             float b1 = s_m1[tid], b2 = s_m2[tid];
             int ix = s_ix[tid];
@@ -847,7 +851,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
             if (fvalid) {
                 undecided = true;
                 int lab = 0;
-                if (ix < k && b1 < 1e38f) {
+                if (ix < k && fabsf(b1) < 1e38f) {
                     lab = ix;
                     const float *cst = reinterpret_cast<const float *>(img + (int64_t)(ix >> 5) * IMG + MAT) + (ix & 31);
                     const double un = COARSE ? (double)cp.sc16[1] : 1.0;  // the coarse pass's values carry 2^2t
@@ -869,7 +873,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
                     const double Em = aa + (double)ce.c1b * mb * mb + 2.0 * (double)ce.c2 * sa * mb + 2.02 * Rm;
                     const double upper = (na + un * (double)b1 + Eb) * (1.0 + (double)ce.gref);
                     const double lower = (na + un * (double)b2 - Em) * (1.0 - (double)ce.gref);
-                    undecided = !(lower > upper);
+                    undecided = !(lower > upper && (sa + mb) * (sa + mb) < 1e38);
                     if (fabs(upper) < 3e38) up = f32_round_up(upper);
                 }
                 labels[fr] = lab;

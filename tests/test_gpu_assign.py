@@ -268,3 +268,24 @@ def test_overflowing_frames_in_short_lists(n, d, k, big):
         lab = _native.assign(Xt, Ct, mode=_native.EMMA_ASSIGN_BF16X3_RECHECK)
         ref = _native.assign(Xt, Ct, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
         assert bool(t.equal(lab, ref))
+
+
+@pytest.mark.parametrize("n", [40, 20_000, 40_000])
+@pytest.mark.parametrize("d", [2, 70])
+@pytest.mark.parametrize("k", [28, 32, 60, 64, 96])
+@pytest.mark.parametrize("big", [1.5e19, 5e19, 2e25])
+def test_finite_outlier_center(n, d, k, big):
+    """A finite center so far out that its squared norm overflows, as the last one that a
+    lane takes and as any other: its distance becomes +inf or no number in the matrix
+    pass, and no frame may be decided from that."""
+    rng = np.random.default_rng(n + k)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    C0 = rng.standard_normal((k, d)).astype(np.float32)
+    X[n // 3] = np.float32(0.9 * big)
+    Xt = _native.as_device_f32(X)
+    for j in (k - 1, k - 5, 27, 0):
+        C = C0.copy()
+        C[j] = np.float32(big)
+        ref = _run(X, C, _native.EMMA_ASSIGN_FP32_PLAIN)[0]
+        for v, lab in enumerate(_every_variant(X, C)):
+            np.testing.assert_array_equal(lab, ref, err_msg="center %d, variant %d" % (j, v))
