@@ -410,8 +410,16 @@ __device__ __forceinline__ float f32_round_up(double v) {
 //        shows)
 // using (|a|+|b|)^2 = |a|^2 + |b|^2 + 2|a||b| and sum|a_i b_i| <= |a||b|.  A
 // 25 % margin covers the rounding of the FP32 bound arithmetic itself.
+// Below the normal numbers the roundings are absolute.  Each square, product and
+// sum of the pass, the element index in a value's low bits and each term and sum
+// of the reference loop is then off by at most 2^-126 (in the coarse pass of the
+// scaled values), fewer than 8 d_pad of them together: E_j also has
+//   e0 = 16 d_pad 2^-126 (1 + 2^-2t).
+// The sums of squares behind |a|, r_a, lo_a and rest_a are FP32 too and off by at
+// most 2 d_pad 2^-150 < SQ_FLOOR, which is added before each root.
+constexpr double SQ_FLOOR = 0x1p-139;
 struct AsgCoef {
-    float c1a, c1b, c2, gref;
+    float c1a, c1b, c2, gref, e0;
 };
 static double gamma_n(double m) {
     const double u = ldexp(1.0, -24);
@@ -424,6 +432,7 @@ static AsgCoef assign_coeffs(int d, int d_pad, int products) {
     c.c1b = (float)(1.25 * (c0 + gamma_n(chain)));
     c.c2 = (float)(1.25 * (c0 + 1.02 * gamma_n(chain)));
     c.gref = (float)(1.25 * gamma_n(d + 2.0));
+    c.e0 = (float)(16.0 * d_pad * ldexp(1.0, -126));
     return c;
 }
 
@@ -648,11 +657,12 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
                 thr[b] = __uint_as_float(0x7fc00000u);
                 ca[b] = cb[b] = cc[b] = 0.0f;
                 const float up = f0 + r < nf ? rl.upper[f0 + r] : __uint_as_float(0x7fc00000u);
-                const double na = s_na[r], sa = sqrt(na) * (1.0 + 2e-5), mb = cp.mx[MX_BN];
+                const double na = s_na[r], sa = sqrt(na + SQ_FLOOR) * (1.0 + 2e-5), mb = cp.mx[MX_BN];
                 if (up == up && (sa + mb) * (sa + mb) < 1e38) {
-                    const double e1 = sqrt((double)s_e1[r]) * (1.0 + 1e-4), e2 = sqrt((double)s_e2[r]) * (1.0 + 1e-4);
+                    const double e1 = sqrt((double)s_e1[r] + SQ_FLOOR) * (1.0 + 1e-4);
+                    const double e2 = sqrt((double)s_e2[r] + SQ_FLOOR) * (1.0 + 1e-4);
                     const double T = (double)up / (1.0 - (double)ce.gref) - (na - (double)ce.c1a * sa * sa) +
-                                     16.0 * 5.9604644775390625e-8 * (sa + mb) * (sa + mb);
+                                     2.0 * (double)ce.e0 + 16.0 * 5.9604644775390625e-8 * (sa + mb) * (sa + mb);
                     thr[b] = f32_round_up(T);
                     ca[b] = (float)((2.0 * (double)ce.c2 * sa + 2.02 * e2) * 1.000001);
                     cb[b] = (float)(2.02 * e1 * 1.000001);
@@ -855,8 +865,8 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
                     lab = ix;
                     const float *cst = reinterpret_cast<const float *>(img + (int64_t)(ix >> 5) * IMG + MAT) + (ix & 31);
                     const double un = COARSE ? (double)cp.sc16[1] : 1.0;  // the coarse pass's values carry 2^2t
-                    const double na = s_na[tid], sa = sqrt(na) * (1.0 + 2e-5);
-                    const double e1 = sqrt((double)s_e1[tid]) * (1.0 + 1e-4) * (COARSE ? (double)cp.sc16[2] : 1.0);
+                    const double na = s_na[tid], sa = sqrt(na + SQ_FLOOR) * (1.0 + 2e-5);
+                    const double e1 = sqrt((double)s_e1[tid] + SQ_FLOOR) * (1.0 + 1e-4) * (COARSE ? (double)cp.sc16[2] : 1.0);
                     const double bb = cst[COARSE ? HC_BN : FC_BN], bd = cst[COARSE ? HC_D1 : FC_D1];
                     const double mb = cp.mx[MX_BN], md = cp.mx[COARSE ? MX_D16 : MX_D1];
                     double Rb, Rm;
@@ -864,11 +874,11 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
                         Rb = e1 * bb + (sa + e1) * bd;
                         Rm = e1 * mb + (sa + e1) * md;
                     } else {
-                        const double e2 = sqrt((double)s_e2[tid]) * (1.0 + 1e-4);
+                        const double e2 = sqrt((double)s_e2[tid] + SQ_FLOOR) * (1.0 + 1e-4);
                         Rb = e1 * bd + e2 * bb + (sa + e2) * (double)cst[FC_D2];
                         Rm = e1 * md + e2 * mb + (sa + e2) * (double)cp.mx[MX_D2];
                     }
-                    const double aa = (double)ce.c1a * sa * sa;
+                    const double aa = (double)ce.c1a * sa * sa + (double)ce.e0 * (1.0 + un);
                     const double Eb = aa + (double)ce.c1b * bb * bb + 2.0 * (double)ce.c2 * sa * bb + 2.02 * Rb;
                     const double Em = aa + (double)ce.c1b * mb * mb + 2.0 * (double)ce.c2 * sa * mb + 2.02 * Rm;
                     const double upper = (na + un * (double)b1 + Eb) * (1.0 + (double)ce.gref);

@@ -289,3 +289,28 @@ def test_finite_outlier_center(n, d, k, big):
         ref = _run(X, C, _native.EMMA_ASSIGN_FP32_PLAIN)[0]
         for v, lab in enumerate(_every_variant(X, C)):
             np.testing.assert_array_equal(lab, ref, err_msg="center %d, variant %d" % (j, v))
+
+
+def _near_ties(d, k, seed):
+    """Frames near the midplane of two of k centers, on a lattice of a few values, so that
+    at small scales many distances are equal or a unit apart."""
+    rng = np.random.default_rng(seed)
+    C = rng.integers(-3, 4, (k, d)).astype(np.float64)
+    a, b = rng.integers(0, k, 3000), rng.integers(0, k, 3000)
+    X = 0.5 * (C[a] + C[b]) + 0.02 * rng.standard_normal((3000, d))
+    return X, C + 1e-3 * rng.standard_normal((k, d))
+
+
+@pytest.mark.parametrize("d", [1, 2, 8, 64, 300])
+@pytest.mark.parametrize("k", [4, 33])
+@pytest.mark.parametrize("exponent", [-16, -17, -18, -19, -20, -21, -22, -23])
+def test_squares_that_underflow(d, k, exponent):
+    """Data whose squared distances or squared residuals are below the smallest normal
+    FP32 number: the loop's own distances are then a few units of 2^-149 apart, and the
+    matrix passes may decide only what that leaves no doubt about."""
+    X, C = _near_ties(d, k, d + k)
+    s = 10.0 ** exponent
+    X, C = (X * s).astype(np.float32), (C * s).astype(np.float32)
+    ref = on.assign(X, C, nthreads=4)
+    for v, lab in enumerate(_every_variant(X, C)):
+        np.testing.assert_array_equal(lab, ref, err_msg="variant %d" % v)
