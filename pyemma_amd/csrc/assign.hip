@@ -1254,7 +1254,14 @@ extern "C" int emma_assign_counted(const float *X, int64_t n, int32_t d, const f
     EMMA_REQUIRE(n >= 0 && d > 0 && k > 0, "emma_assign: bad sizes n=%lld d=%d k=%d", (long long)n, d, k);
     EMMA_REQUIRE(mode == EMMA_ASSIGN_FP32_PLAIN || mode == EMMA_ASSIGN_BF16X3_RECHECK,
                  "emma_assign: unknown mode %d", mode);
-    if (n == 0) return EMMA_OK;
+    if (n == 0) {
+        for (int64_t *p : {n_rechecked, n_looped})
+            if (p) {
+                asg::k_zero_i64n<<<1, 64, 0, (hipStream_t)stream>>>(p, 1);
+                EMMA_TRY(check_launch("emma_assign"));
+            }
+        return EMMA_OK;
+    }
     EMMA_REQUIRE(X && C && labels, "emma_assign: NULL pointer");
     const size_t need = assign_workspace_bytes(n, d, k, mode);
     EMMA_REQUIRE(workspace && workspace_bytes >= need, "emma_assign: workspace too small (%zu < %zu)",
@@ -1334,9 +1341,13 @@ extern "C" int emma_assign_noalloc(const float *X, int64_t n, int32_t d, const f
     EMMA_REQUIRE(n >= 0 && d > 0 && k > 0, "emma_assign_noalloc: bad sizes n=%lld d=%d k=%d", (long long)n, d, k);
     EMMA_REQUIRE(mode == EMMA_ASSIGN_FP32_PLAIN || mode == EMMA_ASSIGN_BF16X3_RECHECK,
                  "emma_assign_noalloc: unknown mode %d", mode);
-    if (n == 0) return EMMA_OK;
-    EMMA_REQUIRE(X && C && labels, "emma_assign_noalloc: NULL pointer");
     hipStream_t s = (hipStream_t)stream;
+    if (n == 0) {
+        if (!n_rechecked) return EMMA_OK;
+        k_zero_i64n<<<1, 64, 0, s>>>(n_rechecked, 1);
+        return check_launch("emma_assign_noalloc");
+    }
+    EMMA_REQUIRE(X && C && labels, "emma_assign_noalloc: NULL pointer");
     if (mode == EMMA_ASSIGN_FP32_PLAIN)  // the plain loop needs no workspace
         return assign_run(X, n, d, C, k, labels, mode, n_rechecked, nullptr, nullptr, nullptr, s);
     // the center images and constants take a fixed part of the scratch; the

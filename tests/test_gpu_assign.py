@@ -314,3 +314,17 @@ def test_squares_that_underflow(d, k, exponent):
     ref = on.assign(X, C, nthreads=4)
     for v, lab in enumerate(_every_variant(X, C)):
         np.testing.assert_array_equal(lab, ref, err_msg="variant %d" % v)
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_counts_of_an_empty_call(mode):
+    """No frames: the counts say so, whatever they held before."""
+    t = _native.torch()
+    X = t.empty((0, 7), dtype=t.float32, device="cuda")
+    C = t.zeros((3, 7), device="cuda")
+    counts = t.full((3,), 99, dtype=t.int64, device="cuda")
+    _native.assign(X, C, mode=mode, n_rechecked=counts[:1], n_looped=counts[1:2])
+    rc = _native.lib().emma_assign_noalloc(_native.ptr(X), 0, 7, _native.ptr(C), 3, None, mode,
+                                           _native.ptr(counts[2:]), _native.stream_ptr())
+    assert rc == 0
+    assert counts.tolist() == [0, 0, 0]
