@@ -165,8 +165,10 @@ class LaggedCovariance(object):
 
     def _sums_cover(self, dt):
         """Whether the column sums of a moments call take in every row of dt: rows
-        [0, T - lag) and [lag, T) of each trajectory, without weights."""
+        [0, T - lag) and [lag, T) of each trajectory, without weights, and no row
+        in front of the first trajectory or behind the last."""
         return (self.weights is None and self.stride == 1 and self.skip == 0 and dt.ntraj > 0
+                and dt.offsets[0] == 0 and dt.n_frames == len(dt.X)
                 and (self.lag == 0 or self.c0t) and min(dt.lengths) > self.lag and min(dt.lengths) >= 2 * self.lag)
 
     def _moments_finish(self, dev, unchecked=None):

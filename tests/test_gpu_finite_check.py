@@ -102,3 +102,24 @@ def test_count_at_every_alignment(n, shift):
     for i, w in enumerate(where):
         x[w] = BAD[i % 3]
         assert int(_native.count_nonfinite(x).item()) == i + 1
+
+
+@pytest.mark.parametrize("row", [0, 299])
+@pytest.mark.parametrize("bad", BAD)
+def test_rows_of_no_trajectory(row, bad):
+    """A device matrix with rows in front of the first trajectory or behind the last is
+    refused for what they hold too."""
+    from pyemma_amd.coordinates._data import DeviceTrajectories
+    from pyemma_amd.coordinates.vamp import VAMP
+
+    t = _native.torch()
+    X = t.randn((300, 4), generator=t.Generator(device="cuda").manual_seed(2), device="cuda")
+    dt = DeviceTrajectories(X, np.array([10, 150, 280]))
+    calls = [LaggedCovariance(c00=True, c0t=True, lag=3).estimate, TICA(lag=3, dim=2).estimate,
+             VAMP(lag=3, dim=2).estimate]
+    for call in calls:
+        call(dt)
+    X[row, 1] = bad
+    for call in calls:
+        with pytest.raises(InvalidDataInStreamException):
+            call(dt)
