@@ -60,16 +60,18 @@ class BatchedDiscretizer(object):
         self._workspaces = _native.Workspaces()
 
     def _sequence(self):
-        self.out = _native.moments_lagged(self.X, self.offsets, self.lag, reversible=self.reversible,
-                                          remove_mean=True, c0t=True, precision=self.precision,
-                                          workspaces=self._workspaces)
+        """The moments as device tensors; the labels go to self.labels."""
+        out = _native.moments_lagged(self.X, self.offsets, self.lag, reversible=self.reversible,
+                                     remove_mean=True, c0t=True, precision=self.precision,
+                                     workspaces=self._workspaces)
         _native.assign(self.X, self.C, mode=self.assign_mode, labels=self.labels, n_rechecked=self.n_rechecked,
                        workspaces=self._workspaces)
+        return out
 
     def run_eager(self):
         """One uncaptured pass (tunes tile shapes on first use); returns host results."""
         autotune.tune_assign(self.X, self.C, self.assign_mode)
-        self._sequence()
+        self.out = self._sequence()
         return self.results()
 
     def capture(self):
@@ -79,8 +81,12 @@ class BatchedDiscretizer(object):
         t.cuda.synchronize()
         g = t.cuda.CUDAGraph()
         with t.cuda.graph(g):
-            self._sequence()
+            out = self._sequence()
         self.graph = g
+        for a, b in zip(out, self.out):  # the capture has not run them: the warm-up's values
+            if a is not None:
+                a.copy_(b)
+        self.out = self._graph_out = out
         # everything whose address the graph holds
         self._captured = (self.X, self.offsets, self.C, self.labels, self.n_rechecked,
                           tuple(self._workspaces.buffers.values()))
@@ -90,6 +96,7 @@ class BatchedDiscretizer(object):
         if self.graph is None:
             raise RuntimeError("capture() first")
         self.graph.replay()
+        self.out = self._graph_out
 
     def results(self):
         """(w, mean, C00, C0t, labels) on the host (synchronizes)."""

@@ -90,3 +90,30 @@ def test_replay_after_larger_calls():
             assert np.array_equal(x, y), "replay %d" % i
         assert all(bool((o == 17).all()) for o in others), "replay %d wrote into another tensor" % i
         _native.assign(big[:1000], big[:500].contiguous())
+
+
+def test_results_are_those_of_the_last_pass():
+    """results() after capture() are the warm-up's, after a replay the replay's, also where
+    an eager pass ran in between."""
+    t = _native.torch()
+    X, off = langevin_trajectories(5, 9, lmin=300, lmax=700, seed=3)
+    X2 = (X * 1.5 + 0.25).contiguous()
+    C = X[::50].cpu().numpy().copy()
+    b = BatchedDiscretizer(X.clone(), off, 4, C)
+
+    def same(r, ref):
+        return all(np.array_equal(x, y) for x, y in zip(r, ref))
+
+    ref = BatchedDiscretizer(X, off, 4, C).run_eager()
+    ref2 = BatchedDiscretizer(X2, off, 4, C).run_eager()
+    b.capture()
+    assert same(b.results(), ref)
+    held = b.out  # every replay writes these
+    for _ in range(2):
+        b.X.copy_(X2)
+        assert same(b.run_eager(), ref2)
+        b.X.copy_(X)
+        b.replay()
+        t.cuda.synchronize()
+        assert same(b.results(), ref)
+        assert b.out is held
