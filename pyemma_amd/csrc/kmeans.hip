@@ -292,10 +292,16 @@ __device__ __forceinline__ void put_coherent(double *p, double v) {
 __device__ __forceinline__ double get_coherent(const double *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// the counter's old value, after every earlier store of this thread has completed
+// The counter's old value, after every earlier store of this thread has completed and
+// before any later load: the wait orders the hardware, the signal fences (no instructions)
+// keep the compiler from moving the relaxed accesses across it.
 __device__ __forceinline__ unsigned int arrive(unsigned int *counter) {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
-    return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const unsigned int seen = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    return seen;
 }
 
 // Block sums (one workgroup per block of BLOCK frames), superblock sums by the last
