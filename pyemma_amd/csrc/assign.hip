@@ -1078,23 +1078,29 @@ static int device_cus() {
 }
 
 // List of a pass's undecided positions from its bit mask.  A workgroup takes
-// 1024 words (32768 positions) at a time and reserves their list range with one
-// atomic.  FINE: the positions are those of listA (or frames, LISTED = false)
-// and go to `list` with their upper bounds; otherwise frames to listA.
-template <bool FINE, bool LISTED>
+// 256 Q words (8192 Q positions) at a time, reserves their list range with one
+// atomic, writes the positions of the set bits to LDS and copies the entries from
+// there, a thread each: a thread that walked the bits of its words itself would
+// wait for the loads of every entry in turn (one workgroup for 32,000 frames took
+// 18 us).  FINE: the positions are those of listA (or frames, LISTED = false) and
+// go to `list` with their upper bounds; otherwise frames to listA.
+template <bool FINE, bool LISTED, int Q>
 __global__ __launch_bounds__(256) void k_compact(int64_t n, RecheckLists rl, const int32_t *__restrict__ done) {
     if (done && *done) return;
+    constexpr int WORDS = 256 * Q;
+    static_assert(WORDS * 32 <= 65536, "a position in a chunk fits 16 bits");
+    __shared__ uint16_t s_pos[WORDS * 32];
     __shared__ uint32_t s_wave[4];
     __shared__ unsigned long long s_base;
     const int64_t np = LISTED ? rl.count[3] : n;
     const int64_t words = (np + 31) >> 5;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int64_t w0 = (int64_t)blockIdx.x * 1024; w0 < words; w0 += (int64_t)gridDim.x * 1024) {
-        uint32_t m[4];
+    for (int64_t w0 = (int64_t)blockIdx.x * WORDS; w0 < words; w0 += (int64_t)gridDim.x * WORDS) {
+        uint32_t m[Q];
         uint32_t cnt = 0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int64_t w = w0 + tid * 4 + q;
+        for (int q = 0; q < Q; ++q) {
+            const int64_t w = w0 + tid * Q + q;
             m[q] = w < words ? rl.mask[w] : 0u;
             cnt += __popc(m[q]);
         }
@@ -1106,30 +1112,27 @@ __global__ __launch_bounds__(256) void k_compact(int64_t n, RecheckLists rl, con
         }
         if (lane == 63) s_wave[wave] = pre;
         __syncthreads();
-        if (tid == 0) {
-            const unsigned long long tot = (unsigned long long)s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
-            s_base = tot ? atomicAdd((unsigned long long *)(rl.count + (FINE ? 0 : 3)), tot) : 0ull;
-        }
-        __syncthreads();
-        int64_t q0 = (int64_t)s_base + pre - cnt;
-        for (int w = 0; w < wave; ++w) q0 += s_wave[w];
+        const uint32_t tot = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        if (tid == 0)
+            s_base = tot ? atomicAdd((unsigned long long *)(rl.count + (FINE ? 0 : 3)), (unsigned long long)tot) : 0ull;
+        uint32_t at = pre - cnt;
+        for (int w = 0; w < wave; ++w) at += s_wave[w];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            uint32_t b = m[q];
-            while (b) {
-                const int64_t pos = (w0 + tid * 4 + q) * 32 + __builtin_ctz(b);
-                b &= b - 1;
-                if constexpr (FINE) {
-                    rl.list[q0] = LISTED ? rl.listA[pos] : pos;
-                    rl.upper[q0] = rl.upper_at[pos];
-                    rl.ccnt[q0] = 0;
-                } else {
-                    rl.listA[q0] = pos;
-                }
-                ++q0;
+        for (int q = 0; q < Q; ++q)
+            for (uint32_t b = m[q]; b; b &= b - 1) s_pos[at++] = (uint16_t)((tid * Q + q) * 32 + __builtin_ctz(b));
+        __syncthreads();
+        const int64_t q0 = (int64_t)s_base;
+        for (uint32_t e = tid; e < tot; e += 256) {
+            const int64_t pos = w0 * 32 + s_pos[e];
+            if constexpr (FINE) {
+                rl.list[q0 + e] = LISTED ? rl.listA[pos] : pos;
+                rl.upper[q0 + e] = rl.upper_at[pos];
+                rl.ccnt[q0 + e] = 0;
+            } else {
+                rl.listA[q0 + e] = pos;
             }
         }
-        __syncthreads();  // s_wave and s_base are consumed
+        __syncthreads();  // the shared values are consumed
     }
 }
 
@@ -1153,6 +1156,21 @@ static void launch_tile(const TileArgs &a, const AssignWs &w, const AsgCoef &ce)
                                                                                a.labels, w.rl, a.done);
 }
 
+// Small chunks while there are few of them, so that more workgroups share the work (d = 32,
+// k = 500, whole call: 33,000 frames 83 us in chunks of 32768, 81 of 8192; 10^7 frames, k = 200:
+// 557 and 573 us, a reservation per chunk on one address)
+template <int PASS>
+static void launch_compact(const TileArgs &a, const AssignWs &w) {
+    constexpr bool FINE = PASS != PASS_COARSE, LISTED = PASS == PASS_FINE;
+    const int q = a.n < ((int64_t)1 << 20) ? 1 : 4;
+    const int64_t chunks = cdiv(a.n, 8192 * q);
+    const unsigned g = (unsigned)(chunks < 512 ? chunks : 512);
+    if (q == 1)
+        k_compact<FINE, LISTED, 1><<<g, 256, 0, a.s>>>(a.n, w.rl, a.done);
+    else
+        k_compact<FINE, LISTED, 4><<<g, 256, 0, a.s>>>(a.n, w.rl, a.done);
+}
+
 // Tile shape of a pass: 128 (coarse) or 64 frames per workgroup, two center
 // tiles per wave step; two 4-wave workgroups per CU while the fragments of
 // both fit in LDS (d <= 304), one of 8 waves beyond.  Few frames (less than
@@ -1165,10 +1183,7 @@ static void launch_pass(const TileArgs &a, const AssignWs &w, const AsgCoef &ce)
         return;
     }
     launch_tile<KS, FB, 2, NW, PASS>(a, w, ce);
-    if (PASS != PASS_CAND) {
-        const int64_t chunks = cdiv(a.n, 32768);
-        k_compact<PASS != PASS_COARSE, PASS == PASS_FINE><<<(unsigned)(chunks < 512 ? chunks : 512), 256, 0, a.s>>>(a.n, w.rl, a.done);
-    }
+    if (PASS != PASS_CAND) launch_compact<PASS>(a, w);
 }
 
 template <int KS>

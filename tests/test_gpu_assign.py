@@ -328,3 +328,26 @@ def test_counts_of_an_empty_call(mode):
                                            _native.ptr(counts[2:]), _native.stream_ptr())
     assert rc == 0
     assert counts.tolist() == [0, 0, 0]
+
+
+@pytest.mark.parametrize("n", [32768, 32769, 40961, 65537, (1 << 20) - 1, (1 << 20) + 33])
+@pytest.mark.parametrize("ties", ["all", "some", "none"])
+def test_list_of_undecided_frames(n, ties):
+    """Lists of every length, in chunks of both sizes: all frames undecided (each center
+    twice), a quarter of them, almost none."""
+    t = _native.torch()
+    g = t.Generator(device="cuda").manual_seed(n)
+    base = 3.0 * t.randn((40, 5), generator=g, device="cuda")
+    C = {"all": t.cat([base, base]), "some": t.cat([base, base[:10]]), "none": base}[ties].contiguous()
+    X = (base[t.randint(0, 40, (n,), generator=g, device="cuda")] + 0.05 * t.randn((n, 5), generator=g, device="cuda"))
+    ref = _native.assign(X, C, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
+    L = _native.lib()
+    counts = t.zeros(1, dtype=t.int64, device="cuda")
+    try:
+        for v in (0, L.emma_assign_variants(5) // 2):
+            _native.check(L.emma_assign_select(5, len(C), v), "emma_assign_select")
+            lab = _native.assign(X, C, n_rechecked=counts)
+            assert t.equal(lab, ref)
+            assert {"all": n, "some": n // 8}.get(ties, 0) <= int(counts.item()) <= n
+    finally:
+        _native.check(L.emma_assign_select(5, len(C), -1), "emma_assign_select")
