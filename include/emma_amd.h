@@ -182,12 +182,12 @@ int emma_assign_noalloc(const float *X, int64_t n, int32_t d, const float *C, in
 /*
  * Variants of the MFMA assignment, for the autotuner: the pipeline of its
  * first pass.  emma_assign_variants(d) is the number n of variants at dimension
- * d (0 if d is beyond the MFMA path): v < n / 2 (0 is the default) is a coarse
- * fp16 pass over every frame whose undecided frames go to the fine bf16 x 3
- * pass, v >= n / 2 the fine pass over every frame.
+ * d (0 if d is beyond the MFMA path): v < n / 2 is a coarse fp16 pass over every
+ * frame whose undecided frames go to the fine bf16 x 3 pass, v >= n / 2 the fine
+ * pass over every frame.  Without a selection the sizes of a call decide.
  * emma_assign_select(d, k, v) makes variant v the one used for every later
  * call whose dimension and center count fall in the same bucket as (d, k)
- * (process-wide, thread-safe; v = -1 restores the default).  Variants only
+ * (process-wide, thread-safe; v = -1 takes the selection back).  Variants only
  * change speed: labels are identical for every variant.
  * No reference counterpart: the reference has no tunable kernels.
  */

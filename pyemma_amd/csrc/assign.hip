@@ -1037,11 +1037,12 @@ __global__ __launch_bounds__(256) void k_assign_cand_exact(const float *__restri
 }
 
 // First-pass pipelines, timed by the autotuner (emma_assign_select may pick one
-// per (K steps, k) bucket): the lower half of the variant numbers (0 is the
-// default) is the coarse pass over every frame with the fine pass on what it
-// leaves; the upper half the fine pass over every frame.  Which is faster depends
-// on d, k and the data: the coarse pass costs a third of the fine one's products,
-// so it loses only where its bound leaves about two thirds of the frames or more.
+// per (K steps, k) bucket): the lower half of the variant numbers is the coarse
+// pass over every frame with the fine pass on what it leaves; the upper half the
+// fine pass over every frame.  Which is faster depends on d, k and the data: the
+// coarse pass costs a third of the fine one's products, so on many frames it
+// loses only where its bound leaves about two thirds of them or more.  Without a
+// selection few_frames() decides.
 // Each pipeline has one tile shape; the count of numbers per dimension is part of
 // the C ABI, so that selections kept by a caller stay valid.
 static int n_variants(int ks) { return ks <= 4 ? 12 : ks <= 8 ? 6 : ks <= 19 ? 4 : 2; }
@@ -1062,11 +1063,23 @@ static int k_bucket(int k_pad) {
     while ((32 << b) < k_pad && b < 15) ++b;
     return b;
 }
+// -1: none
 static int selected_variant(int ks, int k_pad) {
     std::lock_guard<std::mutex> lk(g_sel_mu);
-    if (!g_sel_init) return 0;
+    if (!g_sel_init) return -1;
     const int v = g_sel[ks_index(ks)][k_bucket(k_pad)];
-    return v < n_variants(ks) ? v : 0;
+    return v < n_variants(ks) ? v : -1;
+}
+// Calls bound by their launches and by the latency of a workgroup rather than by
+// products: the fine pass over every frame needs three launches less (the coarse
+// images, pass and list).  Whole calls, us, coarse and fine first pass:
+//   frames   d, k     coarse  fine      frames   d, k      coarse  fine
+//   33,000   10, 64       54    44      200,000  32, 1000     152   149
+//   66,000   32, 1000    129   116      200,000  100, 500     133   151
+//   200,000  10, 10       59    49      400,000  100, 10      107   119
+// Above 19 K-steps the fine pass has one workgroup per CU (200,000 x 350, k = 10: 227, 248).
+static bool few_frames(int64_t n, int ks, int k_pad) {
+    return ks < 24 && n * ks * 16 <= 30'000'000 && n * ks * 16 <= 5'000'000'000 / k_pad;
 }
 
 static int device_cus() {
@@ -1143,6 +1156,7 @@ struct TileArgs {
     int32_t *labels;
     const int32_t *done;
     int cus;
+    bool coarse;
     hipStream_t s;
 };
 
@@ -1188,7 +1202,7 @@ static void launch_pass(const TileArgs &a, const AssignWs &w, const AsgCoef &ce)
 
 template <int KS>
 static void launch_mfma_ks(const TileArgs &a, const AssignWs &w, const AsgCoef &ce, const AsgCoef &ce16) {
-    if (selected_variant(KS, a.k_pad) < n_variants(KS) / 2) {
+    if (a.coarse) {
         launch_pass<KS, PASS_COARSE>(a, w, ce16);
         launch_pass<KS, PASS_FINE>(a, w, ce);
     } else {
@@ -1199,11 +1213,13 @@ static void launch_mfma_ks(const TileArgs &a, const AssignWs &w, const AsgCoef &
 
 }  // namespace asg
 
-// shared with kmeans.hip (Lloyd)
+// shared with kmeans.hip (Lloyd); n_call: frames of the whole call that these n belong to, so that
+// every chunk of a call takes the same passes
 size_t assign_workspace_bytes(int64_t n, int d, int k, int mode) { return asg::carve_assign(nullptr, n, d, k, mode).bytes; }
 
 int assign_run(const float *X, int64_t n, int d, const float *C, int k, int32_t *labels, int mode,
-               int64_t *n_rechecked, int64_t *n_looped, void *workspace, const int32_t *done, hipStream_t s) {
+               int64_t *n_rechecked, int64_t *n_looped, void *workspace, const int32_t *done, hipStream_t s,
+               int64_t n_call) {
     using namespace asg;
     AssignWs w = carve_assign(workspace, n, d, k, mode);
     if (mode == EMMA_ASSIGN_FP32_PLAIN) {
@@ -1218,12 +1234,14 @@ int assign_run(const float *X, int64_t n, int d, const float *C, int k, int32_t 
     const AsgCoef ce = assign_coeffs(d, d_pad, 3), ce16 = assign_coeffs(d, d_pad, 1);
     k_center_mean<<<(unsigned)cdiv(d_pad, 64), 64 * MU_WAVES, 0, s>>>(C, k, d, d_pad, w.cp.mu, w.rl.count);
     k_center_pack<<<(unsigned)cdiv(k_pad, 4), 256, 0, s>>>(C, k, d, d_pad, k_pad, ce.c1b, w.cp);
-    k_center_pack16<<<(unsigned)cdiv(k_pad, 4), 256, 0, s>>>(C, k, d, d_pad, k_pad, w.cp);
+    const int v = selected_variant(ks, k_pad);
+    const bool coarse = v < 0 ? !few_frames(n_call, ks, k_pad) : v < n_variants(ks) / 2;
+    if (coarse) k_center_pack16<<<(unsigned)cdiv(k_pad, 4), 256, 0, s>>>(C, k, d, d_pad, k_pad, w.cp);
     EMMA_TRY(check_launch("assign center pack"));
     // the first pass over every frame, then the passes over what it leaves: the
     // fine pass, the candidates of the frames that one leaves, the reference
     // loop over them, the full loop over every center for the rest
-    const TileArgs a = {X, n, d, k, k_pad, labels, done, device_cus(), s};
+    const TileArgs a = {X, n, d, k, k_pad, labels, done, device_cus(), coarse, s};
     switch (ks) {
         case 2: launch_mfma_ks<2>(a, w, ce, ce16); break;
         case 4: launch_mfma_ks<4>(a, w, ce, ce16); break;
@@ -1281,7 +1299,7 @@ extern "C" int emma_assign_counted(const float *X, int64_t n, int32_t d, const f
     const size_t need = assign_workspace_bytes(n, d, k, mode);
     EMMA_REQUIRE(workspace && workspace_bytes >= need, "emma_assign: workspace too small (%zu < %zu)",
                  workspace_bytes, need);
-    return assign_run(X, n, d, C, k, labels, mode, n_rechecked, n_looped, workspace, nullptr, (hipStream_t)stream);
+    return assign_run(X, n, d, C, k, labels, mode, n_rechecked, n_looped, workspace, nullptr, (hipStream_t)stream, n);
 }
 
 extern "C" int32_t emma_assign_variants(int32_t d) {
@@ -1298,10 +1316,10 @@ extern "C" int emma_assign_select(int32_t d, int32_t k, int32_t variant) {
     std::lock_guard<std::mutex> lk(g_sel_mu);
     if (!g_sel_init) {
         for (auto &row : g_sel)
-            for (int &v : row) v = 0;
+            for (int &v : row) v = -1;
         g_sel_init = true;
     }
-    g_sel[ks_index(ks)][k_bucket((int)cdiv(k, 32) * 32)] = variant < 0 ? 0 : variant;
+    g_sel[ks_index(ks)][k_bucket((int)cdiv(k, 32) * 32)] = variant < 0 ? -1 : variant;
     return EMMA_OK;
 }
 
@@ -1364,7 +1382,7 @@ extern "C" int emma_assign_noalloc(const float *X, int64_t n, int32_t d, const f
     }
     EMMA_REQUIRE(X && C && labels, "emma_assign_noalloc: NULL pointer");
     if (mode == EMMA_ASSIGN_FP32_PLAIN)  // the plain loop needs no workspace
-        return assign_run(X, n, d, C, k, labels, mode, n_rechecked, nullptr, nullptr, nullptr, s);
+        return assign_run(X, n, d, C, k, labels, mode, n_rechecked, nullptr, nullptr, nullptr, s, n);
     // the center images and constants take a fixed part of the scratch; the
     // recheck arrays (56 bytes per frame) the rest, so the frames run
     // in chunks
@@ -1388,7 +1406,7 @@ extern "C" int emma_assign_noalloc(const float *X, int64_t n, int32_t d, const f
     const AssignWs w = carve_assign(ws, chunk, d, k, mode);
     for (int64_t f0 = 0; f0 < n; f0 += chunk) {
         const int64_t m = n - f0 < chunk ? n - f0 : chunk;
-        EMMA_TRY(assign_run(X + f0 * (int64_t)d, m, d, C, k, labels + f0, mode, nullptr, nullptr, ws, nullptr, s));
+        EMMA_TRY(assign_run(X + f0 * (int64_t)d, m, d, C, k, labels + f0, mode, nullptr, nullptr, ws, nullptr, s, n));
         if (n_rechecked) k_add_i64<<<1, 1, 0, s>>>(n_rechecked, w.rl.count);
     }
     return check_launch("emma_assign_noalloc");

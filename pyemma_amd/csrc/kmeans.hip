@@ -27,7 +27,8 @@ namespace emma {
 
 size_t assign_workspace_bytes(int64_t n, int d, int k, int mode);
 int assign_run(const float *X, int64_t n, int d, const float *C, int k, int32_t *labels, int mode,
-               int64_t *n_rechecked, int64_t *n_looped, void *workspace, const int32_t *done, hipStream_t s);
+               int64_t *n_rechecked, int64_t *n_looped, void *workspace, const int32_t *done, hipStream_t s,
+               int64_t n_call);
 
 namespace km {
 
@@ -881,7 +882,7 @@ extern "C" int emma_lloyd(const float *X, int64_t n, int32_t d, float *C, int32_
     const bool vec = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(C) & 15) == 0;
     for (int it = 0; it < max_iter; ++it) {
-        EMMA_TRY(assign_run(X, n, d, C, k, labels, assign_mode, nullptr, nullptr, w.assign_ws, w.done, s));
+        EMMA_TRY(assign_run(X, n, d, C, k, labels, assign_mode, nullptr, nullptr, w.assign_ws, w.done, s, n));
         const size_t run_shm = sizeof(int32_t) * (size_t)k;
         km::k_lloyd_hist<<<(unsigned)nb, 1024, run_shm, s>>>(n, k, labels, w.blk_cnt, w.done);
         km::k_lloyd_scan<<<1, 1024, 0, s>>>(k, nb, w.cnt, w.off, w.coff, w.blk_cnt, w.done);

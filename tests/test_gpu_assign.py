@@ -351,3 +351,27 @@ def test_list_of_undecided_frames(n, ties):
             assert {"all": n, "some": n // 8}.get(ties, 0) <= int(counts.item()) <= n
     finally:
         _native.check(L.emma_assign_select(5, len(C), -1), "emma_assign_select")
+
+
+@pytest.mark.parametrize("n,d,k", [(200, 30, 40), (33_000, 10, 64), (117_187, 256, 100), (117_188, 256, 100),
+                                   (50_000, 40, 1562), (50_000, 40, 1600), (3_000, 400, 10), (3_000, 512, 600)])
+def test_default_pipeline(n, d, k):
+    """Without a selection the sizes choose the first pass, on either side of the line the
+    labels are the loop's, and the call in chunks re-evaluates the same frames as the whole."""
+    t = _native.torch()
+    g = t.Generator(device="cuda").manual_seed(n + d)
+    X = t.randn((n, d), generator=g, device="cuda")
+    C = X[t.randint(0, n, (k,), generator=g, device="cuda")] + 0.2 * t.randn((k, d), generator=g, device="cuda")
+    L = _native.lib()
+    _native.check(L.emma_assign_select(d, k, -1), "emma_assign_select")
+    ref = _native.assign(X, C, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
+    counts = t.zeros(2, dtype=t.int64, device="cuda")
+    lab = _native.assign(X, C, n_rechecked=counts[:1])
+    assert t.equal(lab, ref)
+    lab.fill_(-1)
+    rc = L.emma_assign_noalloc(_native.ptr(X), n, d, _native.ptr(C), k, _native.ptr(lab),
+                               _native.EMMA_ASSIGN_BF16X3_RECHECK, _native.ptr(counts[1:]), _native.stream_ptr())
+    _native.check(rc, "emma_assign_noalloc")
+    assert t.equal(lab, ref)
+    a, b = counts.tolist()
+    assert a == b
