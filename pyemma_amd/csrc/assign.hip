@@ -493,7 +493,8 @@ constexpr int PASS_COARSE = 0, PASS_FINE = 1, PASS_CAND = 2, PASS_FULL = 3;
 // smallest d that a kernel of KS K-steps sees (pick_ksteps takes the next size above d / 16)
 constexpr int min_dim(int ks) { return (ks == 2 ? 0 : ks == 4 ? 2 : ks == 8 ? 4 : ks == 12 ? 8 : ks == 16 ? 12 : ks == 19 ? 16 : ks == 24 ? 19 : 24) * 16 + 1; }
 
-template <int KS, int FB, int CT, int NW, int PASS>
+// MASK: undecided frames as bits for k_compact, otherwise appended to the list here.
+template <int KS, int FB, int CT, int NW, int PASS, bool MASK>
 __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restrict__ X, int64_t n, int d,
                                                             CenterPack cp, int k, int k_pad, AsgCoef ce,
                                                             int32_t *__restrict__ labels, RecheckLists rl,
@@ -534,7 +535,9 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
             constexpr int NCH = (DP + 31) / 32;                       // 16-byte chunks of a row per lane
             int sub = tid & 7;
             asm volatile("" : "+v"(sub));  // keeps the lane's offsets, masks and mu out of the matrix phase's registers
-            float4_u x[2][NCH], mu4[NCH];
+            // groups in flight: all of them where they are few and short, else the next one
+            constexpr int NB = RG * NCH <= 8 ? RG : 2;
+            float4_u x[NB][NCH], mu4[NCH];
             auto load_group = [&](int g, float4_u *xv) __attribute__((always_inline)) {
                 int64_t pos = f0 + g * RPG + (tid >> 3);
                 pos = pos < nf ? pos : nf - 1;
@@ -627,16 +630,18 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
                     if constexpr (!COARSE) s_e2[r] = e2;
                 }
             };
-            static_assert(F % RPG == 0, "whole groups of rows");
-            load_group(0, x[0]);
+            static_assert(F % RPG == 0 && F <= NT, "whole groups of rows; at the end a thread per frame");
+            static_for<0, NB - 1>([&](auto gc) __attribute__((always_inline)) {
+                load_group(decltype(gc)::value, x[decltype(gc)::value]);
+            });
 #pragma unroll
             for (int i = 0; i < NCH; ++i)
                 mu4[i] = *reinterpret_cast<const float4_u *>(cp.mu + sub * 4 + (i * 32 + 32 <= DP || sub < 4 ? i * 32 : 0));
             static_for<0, RG>([&](auto gc) __attribute__((always_inline)) {
                 constexpr int g = decltype(gc)::value;
-                if constexpr (g + 1 < RG) load_group(g + 1, x[(g + 1) & 1]);
+                if constexpr (g + NB - 1 < RG) load_group(g + NB - 1, x[(g + NB - 1) % NB]);
                 __builtin_amdgcn_sched_barrier(0);
-                convert(g, x[g & 1]);
+                convert(g, x[g % NB]);
                 __builtin_amdgcn_sched_barrier(0);
             });
         }
@@ -889,7 +894,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_assign_tile(const float *__restr
                 labels[fr] = lab;
             }
             const unsigned long long um = __ballot(undecided);
-            if constexpr (FB == 1) {
+            if constexpr (!MASK) {
                 // few frames: appended here, one list reservation per wave
                 if (um) {
                     const int leader = __builtin_ctzll(um);
@@ -1160,14 +1165,14 @@ struct TileArgs {
     hipStream_t s;
 };
 
-template <int KS, int FB, int CT, int NW, int PASS>
+template <int KS, int FB, int CT, int NW, int PASS, bool MASK>
 static void launch_tile(const TileArgs &a, const AssignWs &w, const AsgCoef &ce) {
     int64_t blocks = cdiv(PASS == PASS_CAND ? w.rl.slots : a.n, 32 * FB);
     // a listed pass does not know its list's length here: a resident grid walks it
     const int64_t cap = (int64_t)a.cus * (NW == 4 ? 2 : 1);
     if ((PASS == PASS_FINE || PASS == PASS_CAND) && blocks > cap) blocks = cap;
-    k_assign_tile<KS, FB, CT, NW, PASS><<<(unsigned)blocks, NW * 64, 0, a.s>>>(a.X, a.n, a.d, w.cp, a.k, a.k_pad, ce,
-                                                                               a.labels, w.rl, a.done);
+    k_assign_tile<KS, FB, CT, NW, PASS, MASK><<<(unsigned)blocks, NW * 64, 0, a.s>>>(a.X, a.n, a.d, w.cp, a.k, a.k_pad,
+                                                                                     ce, a.labels, w.rl, a.done);
 }
 
 // Small chunks while there are few of them, so that more workgroups share the work (d = 32,
@@ -1188,16 +1193,30 @@ static void launch_compact(const TileArgs &a, const AssignWs &w) {
 // Tile shape of a pass: 128 (coarse) or 64 frames per workgroup, two center
 // tiles per wave step; two 4-wave workgroups per CU while the fragments of
 // both fit in LDS (d <= 304), one of 8 waves beyond.  Few frames (less than
-// one such workgroup per CU) are cut into workgroups of 32.
+// one such workgroup per CU) are cut into workgroups of 32 (either side of that
+// line, 4096 centers: d = 64 405 and 380 us, d = 512 728 and 754).
+// d <= 64 and up to 1024 centers, passes over every frame: a workgroup is one
+// wave with 64 frames.  Such a workgroup's time is a chain of latencies (rows,
+// LDS, center fragments, the decision), in which the waves of a larger one
+// wait for each other, and with fewer tiles than they take some have no
+// centers.  Whole calls, 2 10^6 frames, us, coarse pass, four waves and one:
+// d = 2, k = 10 205 and 91; d = 32, k = 64 237 and 126; d = 32, k = 1000 460 and 406;
+// k = 2000 744 and 717; k = 4096 1343 and 1361; 200,000 x 10, k = 10, fine pass 49 and 40.
 template <int KS, int PASS>
 static void launch_pass(const TileArgs &a, const AssignWs &w, const AsgCoef &ce) {
     constexpr int FB = PASS == PASS_COARSE ? 4 : 2, NW = KS <= 19 ? 4 : 8;
+    constexpr bool EVERY = PASS == PASS_COARSE || PASS == PASS_FULL, MASK = PASS != PASS_CAND;
     if (cdiv(a.n, 32 * FB) < a.cus) {
-        launch_tile<KS, 1, 1, 4, PASS>(a, w, ce);
+        launch_tile<KS, 1, 1, 4, PASS, false>(a, w, ce);
         return;
     }
-    launch_tile<KS, FB, 2, NW, PASS>(a, w, ce);
-    if (PASS != PASS_CAND) launch_compact<PASS>(a, w);
+    bool waves = false;
+    if constexpr (EVERY && KS <= 4) {
+        waves = a.n >= (int64_t)256 * a.cus && a.k_pad <= 1024;
+        if (waves) launch_tile<KS, 2, 1, 1, PASS, true>(a, w, ce);
+    }
+    if (!waves) launch_tile<KS, FB, 2, NW, PASS, MASK>(a, w, ce);
+    if (MASK) launch_compact<PASS>(a, w);
 }
 
 template <int KS>

@@ -375,3 +375,30 @@ def test_default_pipeline(n, d, k):
     assert t.equal(lab, ref)
     a, b = counts.tolist()
     assert a == b
+
+
+@pytest.mark.parametrize("n", [65_535, 65_536, 65_537, 65_599, 131_073])
+@pytest.mark.parametrize("d,k", [(1, 5), (2, 32), (3, 1), (4, 33), (7, 1024), (31, 1025), (32, 100), (33, 64), (63, 1023),
+                                 (64, 31)])
+def test_one_wave_workgroups(n, d, k):
+    """The shape of few centers at small d on either side of its lines, with frames that tie,
+    overflow or are not finite among the others; both pipelines and the default."""
+    t = _native.torch()
+    g = t.Generator(device="cuda").manual_seed(n + 7 * d + k)
+    X = 2.0 * t.randn((n, d), generator=g, device="cuda")
+    C = (X[t.randint(0, n, (k,), generator=g, device="cuda")] + 0.3 * t.randn((k, d), generator=g, device="cuda")).contiguous()
+    C[k // 2] = C[0]
+    X[n // 5] = 2e19
+    X[n - 1, d - 1] = float("nan")
+    X[n - 2, 0] = float("inf")
+    ref = _native.assign(X, C, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
+    L = _native.lib()
+    looped = t.zeros(1, dtype=t.int64, device="cuda")
+    try:
+        for v in (0, L.emma_assign_variants(d) // 2, -1):
+            _native.check(L.emma_assign_select(d, k, v), "emma_assign_select")
+            lab = _native.assign(X, C, n_looped=looped)
+            assert t.equal(lab, ref), "variant %d: %d labels differ" % (v, int((lab != ref).sum()))
+            assert int(looped.item()) >= 3
+    finally:
+        _native.check(L.emma_assign_select(d, k, -1), "emma_assign_select")
