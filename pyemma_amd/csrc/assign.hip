@@ -1202,6 +1202,10 @@ static void launch_compact(const TileArgs &a, const AssignWs &w) {
 // centers.  Whole calls, 2 10^6 frames, us, coarse pass, four waves and one:
 // d = 2, k = 10 205 and 91; d = 32, k = 64 237 and 126; d = 32, k = 1000 460 and 406;
 // k = 2000 744 and 717; k = 4096 1343 and 1361; 200,000 x 10, k = 10, fine pass 49 and 40.
+// d > 384 and up to 512 centers, coarse pass over every frame: four workgroups
+// of 32 frames per CU instead of one of 128, so that frames are read while
+// others are at their products.  1.9 10^6 x 512, whole call, us: k = 10 1883 and
+// 1051, k = 256 1963 and 1408, k = 500 2246 and 2061, k = 1000 3036 and 3512.
 template <int KS, int PASS>
 static void launch_pass(const TileArgs &a, const AssignWs &w, const AsgCoef &ce) {
     constexpr int FB = PASS == PASS_COARSE ? 4 : 2, NW = KS <= 19 ? 4 : 8;
@@ -1210,12 +1214,16 @@ static void launch_pass(const TileArgs &a, const AssignWs &w, const AsgCoef &ce)
         launch_tile<KS, 1, 1, 4, PASS, false>(a, w, ce);
         return;
     }
-    bool waves = false;
+    bool small = false;
     if constexpr (EVERY && KS <= 4) {
-        waves = a.n >= (int64_t)256 * a.cus && a.k_pad <= 1024;
-        if (waves) launch_tile<KS, 2, 1, 1, PASS, true>(a, w, ce);
+        small = a.n >= (int64_t)256 * a.cus && a.k_pad <= 1024;
+        if (small) launch_tile<KS, 2, 1, 1, PASS, true>(a, w, ce);
     }
-    if (!waves) launch_tile<KS, FB, 2, NW, PASS, MASK>(a, w, ce);
+    if constexpr (PASS == PASS_COARSE && KS == 32) {
+        small = a.k_pad <= 512;
+        if (small) launch_tile<KS, 1, 1, 4, PASS, true>(a, w, ce);
+    }
+    if (!small) launch_tile<KS, FB, 2, NW, PASS, MASK>(a, w, ce);
     if (MASK) launch_compact<PASS>(a, w);
 }
 

@@ -402,3 +402,26 @@ def test_one_wave_workgroups(n, d, k):
             assert int(looped.item()) >= 3
     finally:
         _native.check(L.emma_assign_select(d, k, -1), "emma_assign_select")
+
+
+@pytest.mark.parametrize("n", [32_767, 32_768, 32_769, 40_031])
+@pytest.mark.parametrize("d,k", [(385, 31), (400, 512), (511, 513), (512, 10), (512, 257)])
+def test_few_centers_of_large_dimension(n, d, k):
+    """The coarse pass's shape for few centers beyond 384 dimensions, on either side of its
+    lines, with frames that tie, overflow or are not finite among the others."""
+    t = _native.torch()
+    g = t.Generator(device="cuda").manual_seed(n + d + k)
+    X = t.randn((n, d), generator=g, device="cuda")
+    C = (X[t.randint(0, n, (k,), generator=g, device="cuda")] + 0.3 * t.randn((k, d), generator=g, device="cuda")).contiguous()
+    C[k // 2] = C[0]
+    X[n // 5] = 2e19
+    X[n - 1, d - 1] = float("nan")
+    ref = _native.assign(X, C, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
+    L = _native.lib()
+    try:
+        for v in (0, -1):
+            _native.check(L.emma_assign_select(d, k, v), "emma_assign_select")
+            lab = _native.assign(X, C)
+            assert t.equal(lab, ref), "variant %d: %d labels differ" % (v, int((lab != ref).sum()))
+    finally:
+        _native.check(L.emma_assign_select(d, k, -1), "emma_assign_select")
