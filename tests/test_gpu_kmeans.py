@@ -108,3 +108,20 @@ def test_lloyd_member_order_edges(n, d, k):
     np.testing.assert_array_equal(lab, lab_ref)
     np.testing.assert_array_equal(inert, in_ref)
     np.testing.assert_array_equal(C, C_ref)
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("d", list(range(1, 24)) + [31, 32, 33, 47, 48, 63])
+def test_kmeanspp_row_remainders(d, shift):
+    """Rows of every length around the 16 dims that are read together, aligned and not."""
+    t = _native.torch()
+    rng = np.random.default_rng(d)
+    n = 700
+    X = (rng.standard_normal((n, d)) + 3.0 * rng.standard_normal((6, d))[rng.integers(0, 6, n)]).astype(np.float32)
+    C_ref, idx_ref = on.kmeanspp(X, 25, 4, nthreads=4)
+    buf = t.empty(n * d + shift, dtype=t.float32, device="cuda")
+    Xt = buf[shift:].view(n, d)
+    Xt.copy_(t.from_numpy(X))
+    C, idx = _native.kmeanspp(Xt, 25, 4)
+    np.testing.assert_array_equal(idx.cpu().numpy(), idx_ref)
+    np.testing.assert_array_equal(C.cpu().numpy(), C_ref)
