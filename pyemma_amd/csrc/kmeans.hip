@@ -158,11 +158,11 @@ __device__ __forceinline__ float dist_row(const float *__restrict__ x, const flo
 
 // D^2 update against the new center C[r - 1]: the frames that the triangle
 // inequality leaves are compacted over the workgroup, one thread each.  A thread that
-// reads its row itself touches a cache line of its own with every load; from 64 dims
-// on (ROWS_STAGED) a wave reads its 64 rows together instead, 64 dims at a time with 16
-// lanes to a row, and its threads add from LDS (the next 64 dims in flight meanwhile).
-// Below, half of the lanes or more would have no dims to read.  Rows of any alignment:
-// the loads are 4-byte aligned, those across a row's end element by element.
+// reads its row itself touches a cache line of its own with every load; where that is
+// the time (kmpp_staged) a wave reads its 64 rows together instead, 64 dims at a time
+// with 16 lanes to a row, and its threads add from LDS (the next 64 dims in flight
+// meanwhile).  Rows of any alignment: the loads are 4-byte aligned, those across a
+// row's end element by element.
 // (200,000 distances x 300, k = 1000, per round: 54 us for all rows by their own threads, 30 with
 // the triangle inequality, 26 staged.)
 enum Rows { ROWS_ANY = 0, ROWS_VEC = 1, ROWS_STAGED = 2 };
@@ -469,6 +469,15 @@ __global__ __launch_bounds__(256) void k_kmpp_sum_pick(const float *__restrict__
     const int64_t pick = s_pick;
     if (tid == 0) idx[r] = pick;
     for (int i = tid; i < d; i += 256) C[(int64_t)r * d + i] = X[pick * d + i];
+}
+
+// Below 64 dims half of the lanes or more would have no dims to read.  With at most one
+// workgroup per CU, and frames that the caches hold, the time is one row's chain of
+// loads, which staging makes longer: k = 20, whole call, own rows and staged,
+// 1000 x 300 367 and 482 us, 1000 x 1000 641 and 961, 64,000 x 300 510 and 562,
+// 32,000 x 3001 3751 and 2412, 100,000 x 300 716 and 688.
+static bool kmpp_staged(int64_t n, int d) {
+    return d >= SDIM && (n > 65536 || n * d > 50'000'000 || d > 8192);  // own rows: the center in LDS
 }
 
 struct PpWs {
@@ -864,11 +873,12 @@ extern "C" int emma_kmeanspp(const float *X, int64_t n, int32_t d, int32_t k, ui
     const bool vec = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
     const size_t shm = sizeof(float) * (size_t)d;
     const float factor = km::kmpp_factor(d);
+    const bool staged = km::kmpp_staged(n, d);
     for (int r = 1; r < k; ++r) {
         const float *c = C_out + (int64_t)(r - 1) * d;
         if (r > 1) km::k_kmpp_cc<<<(unsigned)cdiv(r - 1, 4), 256, 0, s>>>(C_out, d, r - 1, w.cc);
         const unsigned g = (unsigned)cdiv(n, 256);
-        if (d >= km::SDIM)
+        if (staged)
             km::k_kmpp_d2<km::ROWS_STAGED><<<g, 256, 0, s>>>(X, n, d, c, r, factor, w.cc, w.d2, w.owner);
         else if (vec)
             km::k_kmpp_d2<km::ROWS_VEC><<<g, 256, shm, s>>>(X, n, d, c, r, factor, w.cc, w.d2, w.owner);

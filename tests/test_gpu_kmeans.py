@@ -125,3 +125,20 @@ def test_kmeanspp_row_remainders(d, shift):
     C, idx = _native.kmeanspp(Xt, 25, 4)
     np.testing.assert_array_equal(idx.cpu().numpy(), idx_ref)
     np.testing.assert_array_equal(C.cpu().numpy(), C_ref)
+
+
+@pytest.mark.parametrize("n,d,k,shift", [(65_536, 64, 6, 0), (65_537, 64, 6, 0), (6_103, 8192, 4, 0), (6_104, 8192, 4, 0),
+                                         (70, 8192, 20, 1), (70, 8193, 20, 0), (900, 301, 30, 1), (300, 1000, 30, 0)])
+def test_kmeanspp_own_or_staged_rows(n, d, k, shift):
+    """Both ways of reading rows of 64 dims and more, on either side of each line."""
+    t = _native.torch()
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d), dtype=np.float32)
+    X += 3.0 * rng.standard_normal((6, d), dtype=np.float32)[rng.integers(0, 6, n)]
+    C_ref, idx_ref = on.kmeanspp(X, k, 4, nthreads=8)
+    buf = t.empty(n * d + shift, dtype=t.float32, device="cuda")
+    Xt = buf[shift:].view(n, d)
+    Xt.copy_(t.from_numpy(X))
+    C, idx = _native.kmeanspp(Xt, k, 4)
+    np.testing.assert_array_equal(idx.cpu().numpy(), idx_ref)
+    np.testing.assert_array_equal(C.cpu().numpy(), C_ref)
