@@ -1938,13 +1938,21 @@ static void make_plan(Plan &pl, const float *X, int64_t n_rows, int d, const int
     p.n_tasks = p.n_sym + (p.has_xy ? p.nb * p.nb : 0);
     const bool weighted = (flags & EMMA_MOM_WEIGHTED) != 0;
     // the column-group kernel where it is built and faster (see k_tri); weighted,
-    // non-reversible and wider moments and the single-level mode stay with k_rev_bf16
+    // non-reversible and wider moments and the single-level mode stay with k_rev_bf16.
+    // So do 4 and 5 groups with few rows per slice, where the time is one
+    // workgroup's chain of stages, which are shorter there.  Whole call, us,
+    // k_rev_bf16 and k_tri: 300 columns, 3000 rows 203 and 244, 4000 259 and 312, 6000 367
+    // and 326, 9000 (two slices) 299 and 313, 12,000 373 and 316; 256 columns, 300 rows 60
+    // and 64, 2000 147 and 145.
+    const int64_t slices8 = cdiv(n_rows > 0 ? n_rows : 1, 8192);
+    static const int min_rows[] = {0, 0, 0, 1500, 5000};
     p.tri = precision == EMMA_PREC_BF16X4 && acc2 && p.rev && !weighted && d <= TRI_MAX_D ? tri_groups(d) : 0;
+    if (p.tri && cdiv(n_rows, slices8) < min_rows[p.tri - 1]) p.tri = 0;
     if (p.tri) {
         // the slices of the 128 x 128 kernel (the same sums, to the last bit); with
         // few of them, a workgroup per span
         static const int nt[] = {1, 1, 2, 3, 4};
-        const int64_t cap = cdiv(n_rows > 0 ? n_rows : 1, 8192);
+        const int64_t cap = slices8;
         p.n_sub = cap < 256 ? 8192 / RFLUSH_TL : 1;
         p.n_slices = (int)(cap < 256 ? cap : 256) * p.n_sub;
         p.n_tasks = 1;
@@ -1952,7 +1960,7 @@ static void make_plan(Plan &pl, const float *X, int64_t n_rows, int d, const int
     } else if (precision == EMMA_PREC_BF16X4) {
         // one 8-wave workgroup per CU: 256 slices make the launch of
         // k_rev_bf16 a whole number of rounds (one per task) over the 256 CUs
-        const int64_t cap = cdiv(n_rows > 0 ? n_rows : 1, 8192);
+        const int64_t cap = slices8;
         p.n_slices = (int)(cap < 256 ? cap : 256);
     } else {
         // about 3 workgroups per CU on 256 CUs, at least ~4k pairs per slice

@@ -218,3 +218,28 @@ def test_reversible_column_groups(d, lengths, lag, stride, skip):
     assert np.array_equal(Mxx, Mxx.T) and np.array_equal(Mxy, Mxy.T)
     np.testing.assert_allclose(sx.cpu().numpy(), s, rtol=1e-6, atol=1e-6 * np.sqrt(wr * np.diag(rxx)).max())
     np.testing.assert_array_equal(sx.cpu().numpy(), sy.cpu().numpy())
+
+
+@pytest.mark.parametrize("d", [193, 256, 257, 300, 320])
+@pytest.mark.parametrize("n,lag", [(1499, 3), (1500, 3), (4999, 3), (5000, 3), (5100, 5003), (5100, 5099), (9999, 3),
+                                   (10_000, 3), (10_000, 9_950)])
+def test_reversible_few_rows(d, n, lag):
+    """Either side of the rows per slice where the kernel for more than 192 columns changes,
+    and fewer pairs than a stage has in each of them (bound as above)."""
+    rng = np.random.default_rng(d + n)
+    X = (rng.standard_normal((n, d)) * 10.0 ** rng.uniform(-2, 2, d) + 3.0).astype(np.float32)
+    w, sx, sy, Mxx, Mxy, _ = _native.moments_lagged(_native.as_device_f32(X), np.array([0, n]), lag, reversible=True,
+                                                    remove_mean=True, c0t=True, precision=_native.EMMA_PREC_BF16X4_ACC)
+    wr = 2.0 * max(n - lag, 0)
+    assert float(w.item()) == wr
+    if wr == 0:
+        return
+    x, y = X[:n - lag].astype(np.float64), X[lag:].astype(np.float64)
+    s = x.sum(axis=0) + y.sum(axis=0)
+    x, y = x - s / wr, y - s / wr
+    rxx, rxy = x.T @ x + y.T @ y, x.T @ y + y.T @ x
+    scale = np.sqrt(np.outer(np.diag(rxx), np.diag(rxx)))
+    tol = 2.0 * (2.0 ** -16 + 6e-6)
+    assert np.all(np.abs(Mxx.cpu().numpy() - rxx) <= tol * scale)
+    assert np.all(np.abs(Mxy.cpu().numpy() - rxy) <= tol * scale)
+    np.testing.assert_allclose(sx.cpu().numpy(), s, rtol=1e-6, atol=1e-6 * np.sqrt(wr * np.diag(rxx)).max())
