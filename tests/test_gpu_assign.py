@@ -425,3 +425,25 @@ def test_few_centers_of_large_dimension(n, d, k):
             assert t.equal(lab, ref), "variant %d: %d labels differ" % (v, int((lab != ref).sum()))
     finally:
         _native.check(L.emma_assign_select(d, k, -1), "emma_assign_select")
+
+
+@pytest.mark.parametrize("d", [20, 60, 130, 190, 256, 300, 350, 512])
+def test_lists_longer_than_the_grid(d):
+    """Every frame undecided, more of them than the resident workgroups of the listed
+    passes hold at once, so that each takes several blocks of the list."""
+    t = _native.torch()
+    g = t.Generator(device="cuda").manual_seed(d)
+    n = 100_003
+    base = 2.0 * t.randn((20, d), generator=g, device="cuda")
+    C = t.cat([base, base]).contiguous()
+    X = base[t.randint(0, 20, (n,), generator=g, device="cuda")] + 0.2 * t.randn((n, d), generator=g, device="cuda")
+    ref = _native.assign(X, C, mode=_native.EMMA_ASSIGN_FP32_PLAIN)
+    L = _native.lib()
+    counts = t.zeros(1, dtype=t.int64, device="cuda")
+    try:
+        for v in (0, L.emma_assign_variants(d) // 2):
+            _native.check(L.emma_assign_select(d, 40, v), "emma_assign_select")
+            lab = _native.assign(X, C, n_rechecked=counts)
+            assert t.equal(lab, ref) and int(counts.item()) == n
+    finally:
+        _native.check(L.emma_assign_select(d, 40, -1), "emma_assign_select")

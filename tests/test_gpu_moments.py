@@ -243,3 +243,35 @@ def test_reversible_few_rows(d, n, lag):
     assert np.all(np.abs(Mxx.cpu().numpy() - rxx) <= tol * scale)
     assert np.all(np.abs(Mxy.cpu().numpy() - rxy) <= tol * scale)
     np.testing.assert_allclose(sx.cpu().numpy(), s, rtol=1e-6, atol=1e-6 * np.sqrt(wr * np.diag(rxx)).max())
+
+
+def test_column_groups_round_like_the_wide_kernel():
+    """The column-group kernel's FP32 sums are those of the kernel for more than 320 columns,
+    bit for bit: the leading columns of a wide matrix give the same moments up to the
+    order of the FP64 additions.  More than 8192 pairs per slice, so that every slot is
+    flushed more than once.  The FP32 values of some 600 spans are added in other orders:
+    600 roundings of 2^-53 in each of the two matrices, of sums that Cauchy-Schwarz bounds
+    by the diagonal of the unshifted sums, and a few more in the corrections; one FP32
+    rounding that differs in every 64 pairs would be 100 times more."""
+    t = _native.torch()
+    n, wide, lag = 2_200_000, 330, 7
+    g = t.Generator(device="cuda").manual_seed(5)
+    X = t.randn((n, wide), generator=g, device="cuda")
+    X[lag:] += 0.7 * X[:-lag].clone()
+    X += 0.5 * t.randn((1, wide), generator=g, device="cuda")
+    off = t.as_tensor(np.concatenate([[0], np.sort(np.random.default_rng(1).integers(1, n, 37)), [n]]), device="cuda")
+
+    def run(A):
+        return _native.moments_lagged(A, off, lag, reversible=True, remove_mean=True, c0t=True,
+                                      precision=_native.EMMA_PREC_BF16X4_ACC)
+
+    w, sx, _, Wxx, Wxy, _ = run(X)
+    for d in (3, 30, 64, 65, 128, 150, 192, 256, 300, 320):
+        wd, sd, _, Mxx, Mxy, _ = run(X[:, :d].contiguous())
+        assert float(wd.item()) == float(w.item())
+        tol = 1500 * 2.0 ** -53
+        diag = Wxx.diagonal()[:d] + sx[:d] ** 2 / w
+        scale = t.sqrt(t.outer(diag, diag))
+        assert bool(((sd - sx[:d]).abs() <= tol * t.sqrt(w * diag)).all()), d
+        for a, b in ((Mxx, Wxx), (Mxy, Wxy)):
+            assert bool(((a - b[:d, :d]).abs() <= tol * scale).all()), (d, float(((a - b[:d, :d]).abs() / scale).max()))
