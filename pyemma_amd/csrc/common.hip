@@ -267,37 +267,39 @@ extern "C" int emma_project(const float *X, int64_t n, int32_t d, const double *
 }
 
 // ------------------------------------------------------------------
-// row affine map: out[i] = X[i,:] . u + u0 in FP64, one wavefront per AFF_ROWS rows:
-// lane l adds columns l, l + 64, ... of each row in that order, then a butterfly.  Bound
+// row affine map: out[i] = X[i,:] . u + u0 in FP64, one wavefront per ROWS rows: lane l
+// adds columns l, l + 64, ... of each row in that order, then a butterfly.  Bound
 // by the read of X; one row per wave has a few loads in flight and a chain of shuffles
-// behind them (2 10^6 x 150: 590 us = 2.0 TB/s; eight rows per wave 286 us).
+// behind them (2 10^6 x 150: 590 us = 2.0 TB/s; eight rows per wave 286 us).  Few rows are
+// spread over one wave each: eight then lengthen a chain that the time consists of (500 x
+// 4000 8.9 and 13.3 us, 50,000 x 64 8.9 and 9.9, 50,000 x 150 13.2 and 11.1).
 // ------------------------------------------------------------------
-constexpr int AFF_ROWS = 8;
+template <int ROWS>
 __global__ __launch_bounds__(256) void k_row_affine(const float *__restrict__ X, int64_t n, int d,
                                                     const double *__restrict__ u, double u0,
                                                     double *__restrict__ out) {
     const int lane = threadIdx.x & 63;
-    const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * AFF_ROWS;
+    const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * ROWS;
     if (row >= n) return;
-    const float *x[AFF_ROWS];
-    double a[AFF_ROWS];
+    const float *x[ROWS];
+    double a[ROWS];
 #pragma unroll
-    for (int r = 0; r < AFF_ROWS; ++r) {
+    for (int r = 0; r < ROWS; ++r) {
         x[r] = X + (row + r < n ? row + r : n - 1) * d;  // rows past the last: not stored
         a[r] = 0.0;
     }
     for (int c = lane; c < d; c += 64) {
-        float v[AFF_ROWS];
+        float v[ROWS];
 #pragma unroll
-        for (int r = 0; r < AFF_ROWS; ++r) v[r] = x[r][c];
+        for (int r = 0; r < ROWS; ++r) v[r] = x[r][c];
         const double uc = u[c];
 #pragma unroll
-        for (int r = 0; r < AFF_ROWS; ++r) a[r] = fma((double)v[r], uc, a[r]);
+        for (int r = 0; r < ROWS; ++r) a[r] = fma((double)v[r], uc, a[r]);
     }
 #pragma unroll
-    for (int r = 0; r < AFF_ROWS; ++r) a[r] = emma::wave_butterfly_sum(a[r]);
+    for (int r = 0; r < ROWS; ++r) a[r] = emma::wave_butterfly_sum(a[r]);
 #pragma unroll
-    for (int r = 0; r < AFF_ROWS; ++r)
+    for (int r = 0; r < ROWS; ++r)
         if (lane == 0 && row + r < n) out[row + r] = a[r] + u0;
 }
 
@@ -306,7 +308,10 @@ extern "C" int emma_row_affine(const float *X, int64_t n, int32_t d, const doubl
     EMMA_REQUIRE(n >= 0 && d > 0, "emma_row_affine: bad sizes n=%lld d=%d", (long long)n, d);
     if (n == 0) return EMMA_OK;
     EMMA_REQUIRE(X && u && out, "emma_row_affine: NULL pointer");
-    k_row_affine<<<(unsigned)cdiv(n, 4 * AFF_ROWS), 256, 0, (hipStream_t)stream>>>(X, n, d, u, u0, out);
+    if (n >= 16384 && n * d > 5'000'000)
+        k_row_affine<8><<<(unsigned)cdiv(n, 4 * 8), 256, 0, (hipStream_t)stream>>>(X, n, d, u, u0, out);
+    else
+        k_row_affine<1><<<(unsigned)cdiv(n, 4), 256, 0, (hipStream_t)stream>>>(X, n, d, u, u0, out);
     return check_launch("row affine");
 }
 

@@ -68,3 +68,16 @@ def test_weighted_moments(pairs, stride, precision):
     assert np.all(np.abs(sx.cpu().numpy() - rs) <= f * 2 * (q @ m))
     assert np.all(np.abs(Mxx.cpu().numpy() - rxx) <= e * big)
     assert np.all(np.abs(Mxy.cpu().numpy() - rxy) <= e * big)
+
+
+@pytest.mark.parametrize("n,d", [(16383, 400), (16384, 400), (16389, 400), (50_000, 100), (50_001, 100), (20_000, 3)])
+def test_row_affine_many_rows(n, d):
+    """Either side of the sizes from which a wave takes eight rows: the same sums."""
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    u = rng.standard_normal(d)
+    out = _native.row_affine(_native.as_device_f32(X), u, 0.5).cpu().numpy()
+    bound = (d + 8) * 2.0 ** -53 * (np.abs(X.astype(np.float64)) @ np.abs(u) + 0.5)
+    assert np.all(np.abs(out - (X.astype(np.float64) @ u + 0.5)) <= bound)
+    parts = [_native.row_affine(_native.as_device_f32(X[a:a + 1000]), u, 0.5).cpu().numpy() for a in range(0, n, 1000)]
+    np.testing.assert_array_equal(out, np.concatenate(parts))
