@@ -124,8 +124,8 @@ def device():
     return t.device("cuda", t.cuda.current_device())
 
 
-def stream_ptr():
-    return ctypes.c_void_p(torch().cuda.current_stream().cuda_stream)
+def stream_ptr(stream=None):
+    return ctypes.c_void_p((torch().cuda.current_stream() if stream is None else stream).cuda_stream)
 
 
 def ptr(t):
@@ -161,24 +161,24 @@ class _SharedWorkspaces(threading.local):
     def __init__(self):
         self.sets = collections.OrderedDict()
 
-    def current(self):
-        t = torch()
-        key = (t.cuda.current_device(), t.cuda.current_stream().cuda_stream)
-        ws = self.sets.pop(key, None)
+    def of(self, stream):
+        key = (stream.device_index, stream.cuda_stream)
+        ws = self.sets.get(key)
         if ws is None:
-            ws = Workspaces()
-        self.sets[key] = ws
-        while len(self.sets) > self.MAX_STREAMS:
-            self.sets.popitem(last=False)
+            ws = self.sets[key] = Workspaces()
+            if len(self.sets) > self.MAX_STREAMS:
+                self.sets.popitem(last=False)
+        self.sets.move_to_end(key)
         return ws
 
 
 _shared = _SharedWorkspaces()
 
 
-def workspace(nbytes, tag="default", own=None):
+def workspace(nbytes, tag="default", own=None, stream=None):
     """Device scratch buffer: of `own` if the caller keeps its Workspaces, else the one of
-    this tag that the calls of this thread on the current stream share.  A call that is
+    this tag that the calls of this thread on the current stream share (stream: that
+    stream, from a caller that has looked it up).  A call that is
     being captured into a graph without its own gets a buffer from the graph's memory pool:
     the graph goes on using the address after a later call has replaced the shared buffer,
     and that pool lives as long as the graph."""
@@ -187,7 +187,7 @@ def workspace(nbytes, tag="default", own=None):
     t = torch()
     if t.cuda.is_current_stream_capturing():
         return t.empty(max(int(nbytes), 256), dtype=t.uint8, device=device())
-    return _shared.current().get(nbytes, tag)
+    return _shared.of(t.cuda.current_stream() if stream is None else stream).get(nbytes, tag)
 
 
 def as_device_f32(X):
@@ -242,7 +242,8 @@ def moments_lagged(Xt, traj_offsets, lag, stride=1, skip=0, reversible=True, rem
         weights = weights.contiguous()
     L = lib()
     ws_bytes = L.emma_moments_workspace_size(n_rows, d, ntraj, flags, precision)
-    ws = workspace(ws_bytes, "moments", workspaces)
+    stream = t.cuda.current_stream()
+    ws = workspace(ws_bytes, "moments", workspaces, stream)
     f64 = dict(dtype=t.float64, device=Xt.device)
     w = t.empty(1, **f64)
     sx = t.empty(d, **f64)
@@ -252,7 +253,7 @@ def moments_lagged(Xt, traj_offsets, lag, stride=1, skip=0, reversible=True, rem
     Myy = t.empty((d, d), **f64) if flags & EMMA_MOM_CTT else None
     check(L.emma_moments_lagged_weighted(ptr(Xt), n_rows, d, ptr(off), ntraj, int(lag), int(stride), int(skip),
                                          flags, int(precision), ptr(weights), ptr(w), ptr(sx), ptr(sy), ptr(Mxx),
-                                         ptr(Mxy), ptr(Myy), ptr(ws), ws.numel(), stream_ptr()),
+                                         ptr(Mxy), ptr(Myy), ptr(ws), ws.numel(), stream_ptr(stream)),
           "emma_moments_lagged")
     return w, sx, sy, Mxx, Mxy, Myy
 
@@ -267,9 +268,10 @@ def assign(Xt, Ct, mode=EMMA_ASSIGN_BF16X3_RECHECK, labels=None, n_rechecked=Non
     if labels is None:
         labels = t.empty(n, dtype=t.int32, device=Xt.device)
     L = lib()
-    ws = workspace(L.emma_assign_workspace_size(n, d, k, mode), "assign", workspaces)
+    stream = t.cuda.current_stream()
+    ws = workspace(L.emma_assign_workspace_size(n, d, k, mode), "assign", workspaces, stream)
     check(L.emma_assign_counted(ptr(Xt), n, d, ptr(Ct), k, ptr(labels), int(mode), ptr(n_rechecked), ptr(n_looped),
-                                ptr(ws), ws.numel(), stream_ptr()), "emma_assign")
+                                ptr(ws), ws.numel(), stream_ptr(stream)), "emma_assign")
     return labels
 
 
@@ -279,9 +281,10 @@ def kmeanspp(Xt, k, seed):
     C = t.empty((k, d), dtype=t.float32, device=Xt.device)
     idx = t.empty(k, dtype=t.int64, device=Xt.device)
     L = lib()
-    ws = workspace(L.emma_kmeanspp_workspace_size(n, d, k), "kmeanspp")
+    stream = t.cuda.current_stream()
+    ws = workspace(L.emma_kmeanspp_workspace_size(n, d, k), "kmeanspp", stream=stream)
     check(L.emma_kmeanspp(ptr(Xt), n, d, int(k), int(seed) & (2 ** 64 - 1), ptr(C), ptr(idx), ptr(ws), ws.numel(),
-                          stream_ptr()), "emma_kmeanspp")
+                          stream_ptr(stream)), "emma_kmeanspp")
     return C, idx
 
 
@@ -295,9 +298,10 @@ def lloyd(Xt, Ct, max_iter, tol, mode=EMMA_ASSIGN_BF16X3_RECHECK):
     n_iter = t.zeros(1, dtype=t.int32, device=Xt.device)
     conv = t.zeros(1, dtype=t.int32, device=Xt.device)
     L = lib()
-    ws = workspace(L.emma_lloyd_workspace_size(n, d, k, mode), "lloyd")
+    stream = t.cuda.current_stream()
+    ws = workspace(L.emma_lloyd_workspace_size(n, d, k, mode), "lloyd", stream=stream)
     check(L.emma_lloyd(ptr(Xt), n, d, ptr(Ct), k, int(max_iter), float(tol), int(mode), ptr(labels), ptr(inertias),
-                       ptr(n_iter), ptr(conv), ptr(ws), ws.numel(), stream_ptr()), "emma_lloyd")
+                       ptr(n_iter), ptr(conv), ptr(ws), ws.numel(), stream_ptr(stream)), "emma_lloyd")
     return labels, inertias, n_iter, conv
 
 

@@ -13,8 +13,8 @@ def on_cpu(monkeypatch):
     state = dict(capturing=False, stream=0, device=0)
     monkeypatch.setattr(_native, "device", lambda: torch.device("cpu"))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: state["device"])
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=state["stream"]))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=state["stream"],
+                                                                                    device_index=state["device"]))
     return state
 
 
