@@ -167,9 +167,12 @@ class LaggedCovariance(object):
         """Whether the column sums of a moments call take in every row of dt: rows
         [0, T - lag) and [lag, T) of each trajectory, without weights, and no row
         in front of the first trajectory or behind the last."""
-        return (self.weights is None and self.stride == 1 and self.skip == 0 and dt.ntraj > 0
-                and dt.offsets[0] == 0 and dt.n_frames == len(dt.X)
-                and (self.lag == 0 or self.c0t) and min(dt.lengths) > self.lag and min(dt.lengths) >= 2 * self.lag)
+        if self.weights is not None or self.stride != 1 or self.skip != 0 or not (self.lag == 0 or self.c0t):
+            return False
+        if dt.ntraj == 0 or dt.offsets[0] != 0 or dt.n_frames != dt.X.shape[0]:
+            return False
+        shortest = dt.lengths.min()
+        return shortest > self.lag and shortest >= 2 * self.lag
 
     def _moments_finish(self, dev, unchecked=None):
         """Host FP64 moments of a launched call, with the constant-mean shift.
