@@ -651,7 +651,7 @@ def batched_leg(args, ntraj=4096, d=128, lag=5, k=512, n_seed=1_000_000, n_plain
     C, _ = _native.kmeanspp(sub, k, 4343)
     del sub
     b = BatchedDiscretizer(X, off, lag, C)
-    w0, mean0, C00_0, C0t_0, lab0 = b.run_eager()  # eager pass (also tunes the tile shapes)
+    w0, mean0, C00_0, C0t_0, lab0 = b.run_eager()  # eager pass (also tunes the first pass)
     b.capture()  # the graph's outputs are filled by its replays
     # per-call times of the eager sequence
     off_dev = torch.as_tensor(np.asarray(off, dtype=np.int64), device=dev)

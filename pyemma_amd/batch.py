@@ -6,12 +6,12 @@ covariance.py:219-244) and the assignment of every frame to a center set
 (AbstractClustering._transform_array, clustering/interface.py:157-167) -- is
 one fixed sequence of kernel launches over device-resident inputs:
 
-  emma_moments_lagged: k_prep -> moment tiles (one launch per task kind over
-                       all trajectories and pair slices) -> FP64 reductions
+  emma_moments_lagged: k_prep -> moments (one launch over all trajectories and
+                       pair slices) -> FP64 reductions
   emma_assign:         center mean / pack -> MFMA distances -> exact recheck
 
 BatchedDiscretizer runs that sequence eagerly once (which also lets the
-autotuner pick the tile shapes for these sizes), then captures it into a HIP
+autotuner pick the first pass for these sizes), then captures it into a HIP
 graph; replay() re-issues the whole sequence with one call.  The graph reads
 the input buffers in place, so new frames of the same shape can be copied
 into `X` between replays.  Nothing inside the sequence allocates memory, uses
@@ -69,7 +69,7 @@ class BatchedDiscretizer(object):
         return out
 
     def run_eager(self):
-        """One uncaptured pass (tunes tile shapes on first use); returns host results."""
+        """One uncaptured pass (tunes the first pass on first use); returns host results."""
         autotune.tune_assign(self.X, self.C, self.assign_mode)
         self.out = self._sequence()
         return self.results()

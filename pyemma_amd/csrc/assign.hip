@@ -484,8 +484,9 @@ __device__ __forceinline__ void track2(float &m1, float &m2, float vp, float nin
 // the other workgroup on the CU covers that phase.  Measured, the first pass
 // alone: 10^7 x 300, k = 1000 9.3 -> 6.6 ms (the whole call at k = 32, where the
 // frames' 12 GB bound it, 7.6 -> 2.8 ms = 4.3 TB/s; 1.2 PFLOP/s per added
-// center, the rate of a large library product here); 10^7 x 32, k = 1000
-// 8.2 -> 2.0 ms; 2 10^6 x 512, k = 4096 12.6 -> 7.8 ms.
+// center, where a large library product reaches 1.13); 10^7 x 32, k = 1000
+// 8.2 -> 2.0 ms (1.6 with one wave per workgroup, see launch_pass); 2 10^6 x 512,
+// k = 4096 12.6 -> 7.8 ms.
 // v_mfma_f32_32x32x16: A = 32 centers x 16 dims, B = 16 dims x 32 frames; lane
 // l holds frame l % 32 and centers 8(e>>2) + 4(l>>5) + (e&3).
 constexpr int PASS_COARSE = 0, PASS_FINE = 1, PASS_CAND = 2, PASS_FULL = 3;
@@ -969,7 +970,7 @@ static AssignWs carve_assign(void *ws, int64_t n, int d, int k, int mode) {
         const int k_pad = (int)cdiv(k, 32) * 32;
         w.cp.img = cv.take<uint8_t>((size_t)(k_pad / 32) * tile_img_bytes(d_pad));
         w.cp.img16 = cv.take<uint8_t>((size_t)(k_pad / 32) * tile_img16_bytes(d_pad));
-        (void)cv.take<float>(k_pad);
+        (void)cv.take<float>(k_pad);  // unused: keeps the sizes, and with them what emma_assign_noalloc accepts
         w.cp.mu = cv.take<float>(d_pad);
         w.cp.sc16 = cv.take<float>(4);
     }
