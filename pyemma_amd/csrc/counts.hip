@@ -135,8 +135,10 @@ extern "C" int emma_count_transitions(const int32_t *dtraj, int64_t n, const int
     // the histogram in LDS where its counters fit and the atomics cost more than one
     // more launch (1000 states, the whole call: 65,536 frames 25 us with atomics, 28 with
     // the launch; 262,144 frames 59 and 30; where a state lasts 50 frames the launch is lost,
-    // 140,000 frames 15 and 18, 10^6 18 and 19)
-    const bool lds_hist = hist && nstates <= HIST_STATES && n >= HIST_MIN_ROWS && n < ((int64_t)1 << 40);
+    // 140,000 frames 15 and 18, 10^6 18 and 19), and a state has frames enough that the
+    // workgroups' sums are fewer than its runs (8192 states, 140,000 frames 137 and 144, 10^6 233 and 198)
+    const bool lds_hist = hist && nstates <= HIST_STATES && n >= HIST_MIN_ROWS && n >= 64 * (int64_t)nstates &&
+                          n < ((int64_t)1 << 40);
     if (lds_hist)
         k_hist<<<(unsigned)std::min<int64_t>(cdiv(n, HIST_ROWS), 512), 1024, sizeof(unsigned int) * (size_t)nstates, s>>>(
             dtraj, n, nstates, (unsigned long long *)hist);

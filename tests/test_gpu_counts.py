@@ -140,3 +140,15 @@ def test_histogram_in_lds(n, k):
     ok = (S >= 0) & (S < k)
     np.testing.assert_array_equal(H.cpu().numpy(), np.bincount(S[ok], minlength=k))
     assert int(bad.item()) == int(((S < -1) | (S >= k)).sum())
+
+
+@pytest.mark.parametrize("n,k", [(524_287, 8192), (524_288, 8192), (600_000, 8192), (262_143, 4096), (262_144, 4096)])
+def test_histogram_of_many_states(n, k):
+    """Either side of 64 frames per state."""
+    from pyemma_amd import _native
+
+    t = _native.torch()
+    S = np.random.default_rng(n).integers(0, k, n).astype(np.int32)
+    C, H, bad = _native.count_transitions(t.from_numpy(S).cuda(), np.array([0, n]), 3, True, k)
+    np.testing.assert_array_equal(H.cpu().numpy(), np.bincount(S, minlength=k))
+    assert int(bad.item()) == 0 and int(C.sum().item()) == n - 3
